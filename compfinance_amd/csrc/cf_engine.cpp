@@ -836,7 +836,8 @@ std::shared_ptr<Prepared> prepare(Engine& E, const cf_model* mdl, const cf_produ
     const int forced = forced_layout();
     auto lds_bytes = [&](int copies) {
         return cfk::smem_layout(md.n_steps, md.n_spots, int(pd.timeline.size()), pd.n_pay, waves, fp64 ? 8 : 4, dup,
-                                pd.kind == CF_PRODUCT_EUROPEANS, adjoint, P->cfg.lean, dup ? P->bt.nb : 0, copies)
+                                pd.kind == CF_PRODUCT_EUROPEANS, adjoint, P->cfg.lean, dup ? P->bt.nb : 0, copies,
+                                cfk::split_layout(fp64 ? 8 : 4, dup, adjoint, P->cfg.lean))
             .total;
     };
     P->ivbar_copies = 1;

@@ -72,16 +72,22 @@ struct BookLayout {
     int as_put;       // [n_asian] int
 };
 
+// Half-width in log-spot up to which a barrier's smoothing zone counts as
+// narrow: the FP64 kernels then take a degree-8 polynomial for the spot
+// (truncation 0.05^9 / 9! = 5.4e-18).  The benchmark's 5% zone is 0.033 wide.
+constexpr double kNarrowZone = 0.05;
+
 // Rows of 64 reals in a wave's checkpoint slot.  The Dupire checkpoint
 // variant also keeps, per step and lane, one byte: the knot count of the
 // state's bracket (grids of up to kMaxStoredKnots knots).
 // The Dupire checkpoint slot starts with kCkptGuardRows rows that the reverse
 // sweep's prefetch may read below step 0 (values never used).
-// FP32 Dupire checkpoints are interleaved by groups of four steps: the state
-// of step i of lane l is element ((i >> 2) * 64 + l) * 4 + (i & 3) (a lane's
-// four states in one 16-byte word), its bracket byte the same element of the
-// byte rows that follow the states; the steps are padded to a multiple of four.
-// FP64 keeps one row of 64 per step.
+// Dupire checkpoints are interleaved by groups of four steps: the state of
+// step i of lane l is element ((i >> 2) * 64 + l) * 4 + (i & 3) (a lane's four
+// states in one 16-byte word, 32 bytes in FP64), its bracket byte the same
+// element of the byte rows that follow the states.  FP32 pads the steps to a
+// multiple of four; FP64 keeps the last n_steps % 4 steps in rows of 64, and
+// its book all of them.
 constexpr int kMaxStoredKnots = 255;
 constexpr int kCkptGuardRows = 4;
 CF_HD inline int ckpt_steps(int n_steps, int real_bytes) { return real_bytes == 4 ? (n_steps + 3) & ~3 : n_steps; }
@@ -215,9 +221,18 @@ struct ReducePack {
 
 // Shared-memory carve of one block.  Offsets in bytes, 16-byte aligned.
 struct SmemLayout {
-    size_t lo, hi, hi_tail, step_sample, invn, knots, bucket, iv, drift, stdv, samples, pay_first, pay_strike, acc,
+    size_t lo, mtab, hi, hi_tail, step_sample, invn, knots, bucket, iv, drift, stdv, samples, pay_first, pay_strike, acc,
         tails, ivbar, total;
 };
+
+// FP64 inverse-normal tail table (moro_tail_f64.inc): quarters of the binades
+// 2^-33 .. 2^-4 of the tail mass, twelve coefficients each; a row is the upper
+// 14 bits of the mass less those of 2^-33.  The SPLIT layout keeps the rows
+// from kMoroLdsRow (a mass of 2^-12) on in LDS; 1 draw in 2,048 lies below.
+constexpr int kMoroTailRows = 120, kMoroTailCoefs = 12;
+constexpr int kMoroTailBias = (1023 - 33) << 2;
+constexpr int kMoroLdsRow = (33 - 12) * 4;
+constexpr size_t kMoroLdsBytes = size_t(kMoroTailRows - kMoroLdsRow) * kMoroTailCoefs * 8;
 
 CF_HD inline size_t cf_align16(size_t x) { return (x + 15) & ~size_t(15); }
 
@@ -244,8 +259,13 @@ CF_HD inline bool merge_tail_blocks(int64_t first, int64_t n)
     return (hi >> 6) > (lo >> 6) && (hi & 63) < (lo & 63);
 }
 
-// Two layouts.  FULL keeps the per-lane low Sobol words (one 32-bit word per
-// dimension and lane) and the local-vol table in LDS.  LEAN, for long
+// The layouts.  FULL keeps the per-lane low Sobol words (one 32-bit word per
+// dimension and lane) and the local-vol table in LDS.  Its SPLIT form, that of
+// the FP64 Dupire adjoint kernels (split_layout), keeps 16 words per dimension
+// instead, from which a lane's word is one XOR, and the upper rows of the
+// inverse normal's tail table: 13 KB against 40 at 156 steps, so that the 30 x
+// 36 grid's block holds two local-vol adjoint grids.  (The pricing kernels
+// store no checkpoints; they measured 4% slower in it.)  LEAN, for long
 // timelines or large grids, keeps only direction numbers 0..5 of each
 // dimension (the low word is formed in registers) and reads the local-vol
 // table from global memory through the caches.
@@ -289,12 +309,31 @@ CF_HD inline R bucket_pos(R x, R invh, R c0, R top)
     return clamp_bucket(fma_r(x, invh, c0), top);
 }
 
+// The bucket of x as an index.  FP64 on the device: the conversion saturates
+// (NaN gives 0), so the clamp is one integer instruction instead of five FP64
+// ones; the index is the same.
+template <typename R>
+CF_HD inline int bucket_index(R x, R invh, R c0, R top, int itop)
+{
+#if defined(__HIP_DEVICE_COMPILE__)
+    if constexpr (sizeof(R) == 8) {
+        int b;
+        asm("v_cvt_i32_f64 %0, %1" : "=v"(b) : "v"(fma_r(x, invh, c0)));
+        asm("v_med3_i32 %0, %1, 0, %2" : "=v"(b) : "v"(b), "s"(itop));
+        return b;
+    }
+#endif
+    (void)itop;
+    return int(bucket_pos(x, invh, c0, top));
+}
+
 template <typename R>
 struct KnotSearch {
     const R* knots;     // knot c at knots[stride c]
     const BucketEntry<R>* table;
     int m, fix, stride;
     R invh, c0, top;    // top = number of buckets - 1
+    int itop;           // the same as an integer
 };
 
 // #{knots <= x}, exactly as upper_bound (interp.h:40): states below the first
@@ -306,7 +345,7 @@ CF_HD inline int count_le(const KnotSearch<R>& s, R x)
 {
     // one read: the bucket's knot count and its first two candidate knots
     // (NaN past the last knot); the knots increase, so each one <= x adds one
-    const BucketEntry<R> e = s.table[int(bucket_pos(x, s.invh, s.c0, s.top))];
+    const BucketEntry<R> e = s.table[bucket_index(x, s.invh, s.c0, s.top, s.itop)];
     const int top = s.m - 1;
     int c = e.lo + int(e.k0 <= x) + int(e.k1 <= x);
     if (WIDE) {
@@ -377,13 +416,18 @@ CF_HD inline int lv_cols(int n_spots) { return n_spots + 2; }
 constexpr int kIvbarCopyPad = 8;
 CF_HD inline int ivbar_copy_stride(int n_steps, int n_spots) { return n_steps * lv_cols(n_spots) + kIvbarCopyPad; }
 
+CF_HD constexpr bool split_layout(int real_bytes, bool dupire, bool adjoint, bool lean)
+{
+    return real_bytes == 8 && dupire && adjoint && !lean;
+}
 CF_HD inline SmemLayout smem_layout(int n_steps, int n_spots, int n_samples, int n_pay, int waves,
                                     int real_bytes, bool dupire, bool europeans, bool adjoint, bool lean,
-                                    int n_buckets, int ivbar_copies)
+                                    int n_buckets, int ivbar_copies, bool split = false)
 {
     SmemLayout L{};
     size_t o = 0;
-    L.lo = o;          o = cf_align16(o + sobol_lo_words(n_steps, lean) * 4);
+    L.lo = o;          o = cf_align16(o + (split ? size_t(sobol_dims4(n_steps)) * 16 : sobol_lo_words(n_steps, lean)) * 4);
+    L.mtab = o;        o = cf_align16(o + (split ? kMoroLdsBytes : 0));
     L.hi = o;          o = cf_align16(o + size_t(waves) * sobol_hi_stride(n_steps) * 4);
     L.hi_tail = o;     o = cf_align16(o + size_t(sobol_hi_stride(n_steps)) * 4);
     L.step_sample = o; o = cf_align16(o + size_t(n_steps + 1) * 4);

@@ -85,9 +85,9 @@ int upload_sobol_dirs(const uint32_t* host, uint32_t** device)
 // Words and normals of paths [first, first + npath) in dim dimensions, formed
 // exactly as the path kernels form them (sobol_stage_lo, sobol_block,
 // sobol_low_word / sobol_words4, inv_normal); written [path][dim].
-// 256-thread blocks; LDS: LO (rows, quads or LEAN), one high row per wave,
-// the tail row, and (FP32 FULL) the inverse-normal table.  The quads layout
-// reads dimensions four at a time up to the last whole group, then one at a
+// 256-thread blocks; LDS: LO (rows, split, quads or LEAN), one high row per wave,
+// the tail row, and (FP32 FULL) the inverse-normal table.  The quads and
+// split layouts read dimensions four at a time up to the last whole group, then one at a
 // time, as the FP32 adjoint kernels' forward sweep does.
 template <typename R, int LO>
 __global__ void __launch_bounds__(256) sobol_points_kernel(const uint32_t* dirs, int dim, int64_t first, int64_t npath,
@@ -111,7 +111,7 @@ __global__ void __launch_bounds__(256) sobol_points_kernel(const uint32_t* dirs,
     const R* tab;
     if constexpr (LEAN && sizeof(R) == 4) tab = reinterpret_cast<const R*>(kInvNormalF32);
     else tab = reinterpret_cast<const R*>(invn);
-    tab -= 4 * kInvNormalRowBias;
+    if constexpr (sizeof(R) == 4) tab -= 4 * kInvNormalRowBias;
     const SobolLaneMasks lm = sobol_lane_masks(lane);
     const int64_t nlo = first + 1, nhi = first + npath;
     const int64_t q0 = nlo >> 6, q1 = nhi >> 6;
@@ -125,10 +125,10 @@ __global__ void __launch_bounds__(256) sobol_points_kernel(const uint32_t* dirs,
                 if (normals) normals[size_t(sl.pidx) * dim + i] = inv_normal(w, tab);
             };
             int i = 0;
-            if constexpr (LO == kLoQuads) {
+            if constexpr (LO == kLoQuads || LO == kLoSplit) {
                 for (; i + 4 <= dim; i += 4) {
                     uint32_t w4[4];
-                    sobol_words4(lo_tab, sl.hl, lane, i, w4);
+                    sobol_words4<LO>(lo_tab, sl.hl, lane, i, w4);
                     for (int k = 0; k < 4; ++k) put(i + k, w4[k]);
                 }
             }
@@ -161,7 +161,8 @@ int launch_sobol_points(int real_bytes, int layout, const uint32_t* dirs, int di
         using T = decltype(real);
         if (layout == kLoLean) return reinterpret_cast<const void*>(&sobol_points_kernel<T, kLoLean>);
         if (layout == kLoQuads) return reinterpret_cast<const void*>(&sobol_points_kernel<T, kLoQuads>);
-        return reinterpret_cast<const void*>(&sobol_points_kernel<T, kLoRows>);
+        // (FULL as the Dupire kernels of the precision hold it)
+        return reinterpret_cast<const void*>(&sobol_points_kernel<T, sizeof(T) == 8 ? kLoSplit : kLoRows>);
     };
     f = real_bytes == 4 ? pick(0.0f) : pick(0.0);
     if (smem > 65536) {

@@ -94,87 +94,96 @@ __device__ __forceinline__ CPtr<T> cptr(const void* p)
     return (CPtr<T>)(p);
 }
 
-// a / b in FP64 from the hardware reciprocal refined by two Newton steps and a
-// residual correction (within an ulp of the IEEE quotient)
+// Maximum and minimum in one instruction (the builtins first quiet their
+// operands, one more instruction each); a NaN gives the other operand.
+__device__ __forceinline__ double max_f64(double a, double b)
+{
+    double r;
+    asm("v_max_f64 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
+    return r;
+}
+__device__ __forceinline__ double min_f64(double a, double b)
+{
+    double r;
+    asm("v_min_f64 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
+    return r;
+}
+// a b + c with c a constant in a scalar register pair, in one instruction (the
+// compiler keeps a polynomial's constants in vector registers where scalar
+// ones run short and copies each before a two-address multiply-add)
+__device__ __forceinline__ double fma_s(double a, double b, double c)
+{
+    double r;
+    asm("v_fma_f64 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(b), "s"(c));
+    return r;
+}
+
+// a / b in FP64 from the hardware reciprocal (relative error e below 2^-22):
+// one third-order step r (1 + e + e^2), whose error e^3 is far under an ulp,
+// and a residual correction of the quotient (within an ulp of the IEEE
+// quotient, which it equals but for rare last-bit cases).  Seven
+// instructions; two Newton steps take eight and the compiler's IEEE division
+// twelve.
 __device__ __forceinline__ double fast_div(double a, double b)
 {
     double r = __builtin_amdgcn_rcp(b);
-    r = fma(fma(-b, r, 1.0), r, r);
-    r = fma(fma(-b, r, 1.0), r, r);
+    const double e = fma(-b, r, 1.0);
+    r = fma(r, fma(e, e, e), r);
     const double q = a * r;
     return fma(fma(-b, q, a), r, q);
 }
 
-// Natural logarithm of a positive normal double: x = 2^e m with m in
-// [1/sqrt(2), sqrt(2)), ln(m) = 2 atanh(s) with s = (m - 1) / (m + 1),
-// |s| <= 0.1716, summed to s^21 (truncation below 1e-17 relative), and
-// e ln(2) added in two parts.  About two ulps; used where the argument is
-// known to be positive and finite (the inverse-normal tail).
-__device__ __forceinline__ double log_pos(double x)
-{
-    double m = __builtin_amdgcn_frexp_mant(x);   // [0.5, 1)
-    int e = __builtin_amdgcn_frexp_exp(x);       // x = m 2^e
-    const bool lo = m < 0.70710678118654752440;
-    m = lo ? m + m : m;
-    e = lo ? e - 1 : e;
-    const double s = fast_div(m - 1.0, m + 1.0);
-    const double s2 = s * s;
-    double p = 1.0 / 21.0;
-    p = fma(p, s2, 1.0 / 19.0);
-    p = fma(p, s2, 1.0 / 17.0);
-    p = fma(p, s2, 1.0 / 15.0);
-    p = fma(p, s2, 1.0 / 13.0);
-    p = fma(p, s2, 1.0 / 11.0);
-    p = fma(p, s2, 1.0 / 9.0);
-    p = fma(p, s2, 1.0 / 7.0);
-    p = fma(p, s2, 1.0 / 5.0);
-    p = fma(p, s2, 1.0 / 3.0);
-    const double ed = double(e);
-    const double ln2_hi = 6.93147180369123816490e-01;   // 0x3FE62E42FEE00000, exact in ed * ln2_hi
-    const double ln2_lo = 1.90821492927058770002e-10;
-    // ed * ln2_hi is exact (32-bit constant times an 11-bit integer)
-    return fma(ed, ln2_hi, fma(2.0 * s * s2, p, fma(ed, ln2_lo, 2.0 * s)));
-}
-
 // Beasley-Springer-Moro inverse normal (gaussians.h:47-87), FP64, same
 // branches and constants as the reference: the central rational form of
-// x = min(p, 1 - p) - 1/2 for |x| < 0.42, else the tail polynomial in
-// log(-log(min(p, 1 - p))); both halves are also evaluated apart
-// (inv_normal4_f64) and give the same values.
+// x = p - 1/2 for |x| < 0.42 (an odd function of x), else the tail polynomial
+// in log(-log(v)) of v = min(p, 1 - p).  The tail is read from a table of
+// polynomials of degree 11 on the quarters of the binades of v
+// (moro_tail_f64.inc, written by gen_moro_tail_f64.py in extended precision):
+// within 2.0 half-ulps of the exact tail (0.48 on average) over the Sobol
+// words, where two logarithms and the polynomial in double round to 4.1
+// (0.75), for 18 instructions and six 16-byte reads instead of 95
+// instructions.
+static __constant__ double kMoroTailF64[kMoroTailRows * kMoroTailCoefs] = {
+#include "moro_tail_f64.inc"
+};
 __device__ __forceinline__ double moro_central(double x)
 {
     const double r = x * x;
-    return x * (((-25.44106049637 * r + 41.39119773534) * r + -18.61500062529) * r + 2.50662823884) /
-           ((((3.13082909833 * r + -21.06224101826) * r + 23.08336743743) * r + -8.47351093090) * r + 1.0);
+    return fast_div(x * (((-25.44106049637 * r + 41.39119773534) * r + -18.61500062529) * r + 2.50662823884),
+                    (((3.13082909833 * r + -21.06224101826) * r + 23.08336743743) * r + -8.47351093090) * r + 1.0);
 }
-__device__ __forceinline__ double moro_tail(double up)
+// the row's polynomial from its coefficients c, and the distance to its midpoint
+__device__ __forceinline__ double moro_tail_row(double v, const double* row)
 {
-    double r = log_pos(-log_pos(up));
-    r = 0.3374754822726147 +
-        r * (0.9761690190917186 +
-        r * (0.1607979714918209 +
-        r * (0.0276438810333863 +
-        r * (0.0038405729373609 +
-        r * (0.0003951896511919 +
-        r * (0.0000321767881768 +
-        r * (0.0000002888167364 + r * 0.0000003960315187)))))));
+    const uint32_t hi = uint32_t(__builtin_bit_cast(uint64_t, v) >> 32);
+    const double mid = __builtin_bit_cast(double, uint64_t((hi & 0xfffc0000u) | 0x20000u) << 32);
+    const double d = v - mid;   // exact
+    const double2* c = reinterpret_cast<const double2*>(row);
+    double r = fma(c[5].y, d, c[5].x);
+#pragma unroll
+    for (int k = 4; k >= 0; --k) r = fma(fma(r, d, c[k].y), d, c[k].x);
     return r;
+}
+// (a mass outside the table, which only an idle lane's word 0 gives, takes an
+// end row)
+__device__ __forceinline__ int moro_row(double v)
+{
+    return min(max(int(uint32_t(__builtin_bit_cast(uint64_t, v) >> 32) >> 18) - kMoroTailBias, 0), kMoroTailRows - 1);
+}
+__device__ __forceinline__ double moro_tail(double v)
+{
+    return moro_tail_row(v, kMoroTailF64 + moro_row(v) * kMoroTailCoefs);
 }
 __device__ __forceinline__ double inv_normal_p(double p)
 {
-    const bool sup = p > 0.5;
-    const double up = sup ? 1.0 - p : p;
-    const double x = up - 0.5;
-    if (fabs(x) < 0.42) {
-        const double z = moro_central(x);
-        return sup ? -z : z;
-    }
-    const double r = moro_tail(up);
-    return sup ? r : -r;
+    const double x = p - 0.5;
+    double z = moro_central(x);
+    if (!(fabs(x) < 0.42)) z = __builtin_copysign(moro_tail(min_f64(p, 1.0 - p)), x);
+    return z;
 }
 
 // of the Sobol uniform u = ONEOVER2POW32 * xi (sobol.h:26, :110-116)
-__device__ __forceinline__ double inv_normal(uint32_t xi, double)
+__device__ __forceinline__ double inv_normal(uint32_t xi, const double*)
 {
     return inv_normal_p(2.3283064365387E-10 * double(xi));
 }
@@ -206,69 +215,68 @@ __device__ __forceinline__ float inv_normal(uint32_t xi, const float* tabm)
     return __uint_as_float(__float_as_uint(p) ^ sgn);   // -p for u >= 1/2
 }
 
-// FP64: the reference's function; the table pointer is unused
-__device__ __forceinline__ double inv_normal(uint32_t xi, const double*) { return inv_normal(xi, 0.0); }
-
-// Four FP64 normals of this lane's Sobol words, with Moro's tail evaluated
-// once per wave.  About 16% of draws need the tail (two logarithms and a
-// polynomial), so a wave of 64 lanes almost always has one that does and,
-// draw by draw, every lane would run it.  Here every lane runs the central
-// form of its four draws; the tail draws of the wave, counted by ballots, go
-// to `row` (this wave's ROW doubles of LDS) by their rank, each lane evaluates
-// at most one, and the owners read their values back (in rounds of ROW when
-// more draws need the tail).  The values equal inv_normal_p's, draw by draw.
-template <int ROW>
-__device__ __forceinline__ void inv_normal4_p(const double p[4], double z[4], double* row, int lane)
+// Four FP64 normals of this lane's uniforms, with Moro's tail evaluated once
+// per wave.  About 16% of draws need the tail, so a wave of 64 lanes almost
+// always has one that does and, draw by draw, every lane would run it.  Here
+// every lane runs the central form of its four draws; the tail masses of the
+// wave, counted by ballots, go to `row` (this wave's ROW doubles of LDS) by
+// their rank, each lane evaluates at most one, and the owners read their
+// values back (in rounds of ROW when more draws need the tail: 41 on
+// average, more than 64 once in 20,000 groups).  The values equal
+// inv_normal_p's, draw by draw.  LTAB: `tab` holds the table's rows from
+// kMoroLdsRow on in LDS (through L1 the reads would wait for the checkpoint
+// stores issued before them: one counter orders loads and stores); a wave with
+// a mass below them, 12% of the groups, reads the whole table through L1.
+template <int ROW, bool LTAB>
+__device__ __forceinline__ void inv_normal4_p(const double p[4], double z[4], double* row, const double* tab, int lane)
 {
-    double up[4];
-    bool sup[4], tail[4];
-    uint64_t m[4];
-    int base[4];
+    static_assert(ROW >= 1 && ROW <= kWave, "a row of at most one double per lane");
+    bool tail[4];
+    int pos[4];    // rank of this lane's draw among the wave's tail draws
     int total = 0;
 #pragma unroll
     for (int k = 0; k < 4; ++k) {
-        sup[k] = p[k] > 0.5;
-        up[k] = sup[k] ? 1.0 - p[k] : p[k];
-        const double x = up[k] - 0.5;
+        const double x = p[k] - 0.5;
         tail[k] = !(fabs(x) < 0.42);
-        const double c = moro_central(x);
-        z[k] = sup[k] ? -c : c;
-        m[k] = __builtin_amdgcn_ballot_w64(tail[k]);
-        base[k] = total;
-        total += __builtin_popcountll(m[k]);
+        z[k] = moro_central(x);
+        const uint64_t m = __builtin_amdgcn_ballot_w64(tail[k]);
+        pos[k] = int(__builtin_amdgcn_mbcnt_hi(uint32_t(m >> 32), __builtin_amdgcn_mbcnt_lo(uint32_t(m), uint32_t(total))));
+        total += __builtin_popcountll(m);
     }
-    static_assert(ROW >= 1 && ROW <= kWave, "a row of at most one double per lane");
     for (int r0 = 0; r0 < total; r0 += ROW) {
 #pragma unroll
-        for (int k = 0; k < 4; ++k) {
-            const int pos = base[k] +
-                            int(__builtin_amdgcn_mbcnt_hi(uint32_t(m[k] >> 32), __builtin_amdgcn_mbcnt_lo(uint32_t(m[k]), 0u))) - r0;
-            if (tail[k] && pos >= 0 && pos < ROW) row[pos] = up[k];
-        }
+        for (int k = 0; k < 4; ++k)
+            if (bool(tail[k] & (uint32_t(pos[k] - r0) < uint32_t(ROW)))) row[pos[k] - r0] = min_f64(p[k], 1.0 - p[k]);
         wave_sync_lds();
-        if (lane < ROW && lane < total - r0) row[lane] = moro_tail(row[lane]);
-        wave_sync_lds();
-#pragma unroll
-        for (int k = 0; k < 4; ++k) {
-            const int pos = base[k] +
-                            int(__builtin_amdgcn_mbcnt_hi(uint32_t(m[k] >> 32), __builtin_amdgcn_mbcnt_lo(uint32_t(m[k]), 0u))) - r0;
-            if (tail[k] && pos >= 0 && pos < ROW) {
-                const double t = row[pos];
-                z[k] = sup[k] ? t : -t;
+        if (lane < ROW && lane < total - r0) {
+            const double v = row[lane];
+            if constexpr (LTAB) {
+                const int r = moro_row(v);
+                if (__builtin_amdgcn_ballot_w64(r < kMoroLdsRow) == 0)
+                    row[lane] = moro_tail_row(v, tab + (r - kMoroLdsRow) * kMoroTailCoefs);
+                else
+                    row[lane] = moro_tail_row(v, kMoroTailF64 + r * kMoroTailCoefs);
+            } else {
+                row[lane] = moro_tail(v);
             }
         }
+        wave_sync_lds();
+#pragma unroll
+        for (int k = 0; k < 4; ++k)
+            if (bool(tail[k] & (uint32_t(pos[k] - r0) < uint32_t(ROW))))
+                z[k] = __builtin_copysign(row[pos[k] - r0], p[k] - 0.5);
         wave_sync_lds();
     }
 }
 
 // Of Sobol words (sobol.h:26, :110-116)
-template <int ROW>
-__device__ __forceinline__ void inv_normal4_f64(const uint32_t w[4], double z[4], double* row, int lane)
+template <int ROW, bool LTAB>
+__device__ __forceinline__ void inv_normal4_f64(const uint32_t w[4], double z[4], double* row, const double* tab, int lane)
 {
     double p[4];
 #pragma unroll
     for (int k = 0; k < 4; ++k) p[k] = 2.3283064365387E-10 * double(w[k]);
-    inv_normal4_p<ROW>(p, z, row, lane);
+    inv_normal4_p<ROW, LTAB>(p, z, row, tab, lane);
 }
 
 // FP32 inverse-normal table: [rows][4 monomial coefficients]
@@ -400,8 +408,11 @@ struct Lane {
     __device__ __forceinline__ double uniform(int i)
     {
         seek(i);
+        // d / (m1 + 1), the division by its reciprocal and one residual step
         const double diff = double(x[0]) - double(y[0]);
-        return x[0] > y[0] ? diff / 4294967088.0 : (diff + 4294967087.0) / 4294967088.0;
+        const double d = x[0] > y[0] ? diff : diff + 4294967087.0;
+        const double q = d * (1.0 / 4294967088.0);
+        return fma(fma(-q, 4294967088.0, d), 1.0 / 4294967088.0, q);
     }
     __device__ __forceinline__ double normal(int i)
     {
@@ -422,12 +433,70 @@ struct Lane {
 };
 }   // namespace mrg
 
+// exp in FP64, in two parts.  exp_reduce: x = n ln(2) / 8 + d with |d| <=
+// 0.0434, and the scale 2^(n / 8) as a sum hi + lo (x beyond +-800 saturates
+// to 0 or infinity).  exp_scaled: (hi + lo) e^d by the Taylor polynomial of
+// degree 8 (truncation below 6e-18 for |d| <= 0.05), the product with hi - 1
+// added last: within 0.51 ulp, in 25 instructions and one 16-byte read
+// against the library function's 35.
+static __constant__ double kExpEighths[16] = {   // 2^(j / 8), hi and lo
+    1.00000000000000000e+00, 0.00000000000000000e+00,
+    1.09050773266525769e+00, -3.04678207981247115e-17,
+    1.18920711500272103e+00, 3.98201523146564611e-17,
+    1.29683955465100964e+00, 2.53825027948883150e-17,
+    1.41421356237309515e+00, -9.66729331345291345e-17,
+    1.54221082540794074e+00, 7.94983480969762086e-17,
+    1.68179283050742900e+00, 8.19901002058149652e-17,
+    1.83400808640934243e+00, 3.28310722424562720e-17,
+};
+struct ExpScale {
+    double hi, lo;
+};
+__device__ __forceinline__ ExpScale exp_reduce(double x, double& d)
+{
+    x = min_f64(max_f64(x, -800.0), 800.0);
+    const double n = __builtin_rint(x * 11.541560327111707);   // 8 / ln(2)
+    // ln(2) / 8 in two parts, the first of 29 bits: n times it is exact
+    d = fma(n, -8.66433973424136638641e-02, x);
+    d = fma(n, -2.27579499813018278006e-10, d);
+    const int k = int(n);
+    const double2 t = reinterpret_cast<const double2*>(kExpEighths)[k & 7];
+    ExpScale s;
+    s.hi = __builtin_amdgcn_ldexp(t.x, k >> 3);
+    s.lo = __builtin_amdgcn_ldexp(t.y, k >> 3);
+    return s;
+}
+// (exp_tail: (hi + lo) e^d - hi; exp_scaled2: the result and its rounding)
+__device__ __forceinline__ double exp_tail(double d, ExpScale s)
+{
+    double q = fma(d, 1.0 / 40320.0, 1.0 / 5040.0);
+    q = fma_s(q, d, 1.0 / 720.0);
+    q = fma_s(q, d, 1.0 / 120.0);
+    q = fma_s(q, d, 1.0 / 24.0);
+    q = fma_s(q, d, 1.0 / 6.0);
+    q = fma(q, d, 0.5);
+    q = fma(q, d, 1.0);
+    return fma(s.hi, q * d, s.lo);
+}
+__device__ __forceinline__ double exp_scaled(double d, ExpScale s) { return s.hi + exp_tail(d, s); }
+__device__ __forceinline__ ExpScale exp_scaled2(double d, ExpScale s)
+{
+    const double t = exp_tail(d, s), hi = s.hi + t;
+    return {hi, (s.hi - hi) + t};
+}
+__device__ __forceinline__ double exp_f64(double x)
+{
+    double d;
+    const ExpScale s = exp_reduce(x, d);
+    return exp_scaled(d, s);
+}
+
 // Spot from the path state: FP64 state is log(S) (reference), FP32 state is
 // log(S / S0), which keeps more significant bits in single precision.
-__device__ __forceinline__ double state_spot(double x, double) { return exp(x); }
+__device__ __forceinline__ double state_spot(double x, double) { return exp_f64(x); }
 __device__ __forceinline__ float state_spot(float x, double s0) { return float(s0) * __expf(x); }
 
-__device__ __forceinline__ double rexp(double x) { return exp(x); }
+__device__ __forceinline__ double rexp(double x) { return exp_f64(x); }
 __device__ __forceinline__ float rexp(float x) { return __expf(x); }
 
 // Local vol at state x on one timeline row (interp.h:26-63): upper_bound on
@@ -490,14 +559,18 @@ __device__ __forceinline__ R euler_step(R x, R vol, R g)
 // in dimension d is LO[d][r] ^ HI_q[d].  The path kernels and the points
 // kernel share these functions.
 
-// LO staged in LDS by a block, in one of three layouts: rows (the 64 lanes'
+// LO staged in LDS by a block, in one of four layouts: rows (the 64 lanes'
 // low words of each dimension, [d][lane]), quads (the same words interleaved
 // by groups of four dimensions, [d / 4][lane][d % 4], for kernels that read a
 // lane's four consecutive dimensions in one 16-byte word; a lane reading one
-// word at a time would stride 16 bytes and conflict on the LDS banks), or
-// LEAN (only direction numbers 0..5: the low word is formed in registers from
-// the lane's masks).
-enum SobolLoLayout { kLoRows = 0, kLoLean = 1, kLoQuads = 2 };
+// word at a time would stride 16 bytes and conflict on the LDS banks), LEAN
+// (only direction numbers 0..5: the low word is formed in registers from the
+// lane's masks), or split: gray6 is linear over the bits of the lane, so its
+// word is the XOR of one of eight words for lane % 8 and one of eight for
+// lane / 8, a quarter of the rows' size; interleaved by four dimensions,
+// [d / 4][16][d % 4], read four at a time (lanes with the same octet read the
+// same address, without conflicts).
+enum SobolLoLayout { kLoRows = 0, kLoLean = 1, kLoQuads = 2, kLoSplit = 3 };
 
 template <int LO>
 __device__ __forceinline__ void sobol_stage_lo(uint32_t* lo_tab, const uint32_t* dirs, int n, int tid, int nthr)
@@ -506,6 +579,19 @@ __device__ __forceinline__ void sobol_stage_lo(uint32_t* lo_tab, const uint32_t*
         for (int e = tid; e < n * 8; e += nthr) {
             const int d = e >> 3, k = e & 7;
             lo_tab[e] = k < 6 ? dirs[k * kSobolDims + d] : 0u;
+        }
+    } else if constexpr (LO == kLoSplit) {
+        // word e: dimension 4 (e >> 6) + (e & 3), entry (e >> 2) & 15 (lane % 8, then 8 + lane / 8)
+        for (int e = tid; e < sobol_dims4(n) * 16; e += nthr) {
+            const int d = ((e >> 6) << 2) + (e & 3), o = (e >> 2) & 15;
+            if (d >= n) continue;
+            const int r = o < 8 ? o : (o - 8) << 3;
+            const uint32_t g = uint32_t(r ^ (r >> 1));
+            uint32_t x = 0;
+#pragma unroll
+            for (int k = 0; k < 6; ++k)
+                if ((g >> k) & 1u) x ^= dirs[k * kSobolDims + d];
+            lo_tab[e] = x;
         }
     } else {
         // word e: rows dimension e >> 6, lane e & 63; quads dimension
@@ -547,18 +633,29 @@ __device__ __forceinline__ uint32_t sobol_low_word(const uint32_t* lo_tab, const
                (lm.m[5] & v[5]);
     } else if constexpr (LO == kLoQuads) {
         return lo_tab[sobol_lo_el(i, lane)];
+    } else if constexpr (LO == kLoSplit) {
+        const uint32_t* v = lo_tab + ((i >> 2) << 6) + (i & 3);
+        return v[(lane & 7) << 2] ^ v[(8 + (lane >> 3)) << 2];
     } else {
         return lo_tab[i * kWave + lane];
     }
 }
 
-// Quads layout: this lane's words of dimensions i .. i + 3 (i a multiple of
-// four, below the padded dimension count), one 16-byte read of LO and one of
-// the lane's high row (16-byte aligned rows)
+// Quads and split layouts: this lane's words of dimensions i .. i + 3 (i a
+// multiple of four, below the padded dimension count), one 16-byte read of LO
+// (two of the split one) and one of the lane's high row (16-byte aligned rows)
+template <int LO = kLoQuads>
 __device__ __forceinline__ void sobol_words4(const uint32_t* lo_tab, const uint32_t* hl, int lane, int i, uint32_t* w)
 {
-    const uint4 lw = *reinterpret_cast<const uint4*>(lo_tab + sobol_lo_el(i, lane));
     const uint4 hw = *reinterpret_cast<const uint4*>(hl + i);
+    uint4 lw;
+    if constexpr (LO == kLoSplit) {
+        const uint4* v = reinterpret_cast<const uint4*>(lo_tab) + ((i >> 2) << 4);
+        const uint4 a = v[lane & 7], b = v[8 + (lane >> 3)];
+        lw = make_uint4(a.x ^ b.x, a.y ^ b.y, a.z ^ b.z, a.w ^ b.w);
+    } else {
+        lw = *reinterpret_cast<const uint4*>(lo_tab + sobol_lo_el(i, lane));
+    }
     w[0] = lw.x ^ hw.x;
     w[1] = lw.y ^ hw.y;
     w[2] = lw.z ^ hw.z;
@@ -652,8 +749,9 @@ __device__ __forceinline__ void path_body(const LaunchParams& P, const int bid, 
     const int mp = lv_cols(m);   // padded local-vol row
     const int stride = out_stride(npay);
     constexpr bool BOOK = PRD == PRD_BOOK;
+    constexpr bool SPLIT = split_layout(int(sizeof(R)), DUP, AD, LEAN);
     const SmemLayout L = smem_layout(n, m, ns, npay, waves, int(sizeof(R)), DUP, EUS, AD, LEAN, P.n_buckets,
-                                     P.ivbar_copies);
+                                     P.ivbar_copies, SPLIT);
 
     uint32_t* lo_tab = reinterpret_cast<uint32_t*>(smem + L.lo);
     uint32_t* hi_all = reinterpret_cast<uint32_t*>(smem + L.hi);
@@ -689,9 +787,12 @@ __device__ __forceinline__ void path_body(const LaunchParams& P, const int bid, 
     // Sobol LO layout: the FP32 Dupire adjoint kernels other than the book
     // read four dimensions at once (quads); the others one at a time (rows)
     constexpr bool QUADS = sizeof(R) == 4 && AD && DUP && !BOOK && !LEAN && !MRG;
-    constexpr int LOL = LEAN ? kLoLean : (QUADS ? kLoQuads : kLoRows);
+    constexpr int LOL = LEAN ? kLoLean : SPLIT ? kLoSplit : (QUADS ? kLoQuads : kLoRows);
     // ---- stage the block's tables in LDS
     sobol_stage_lo<LOL>(lo_tab, P.dirs, n, tid, nthr);
+    double* mtab = reinterpret_cast<double*>(smem + L.mtab);   // SPLIT: tail table rows from kMoroLdsRow on
+    if constexpr (SPLIT)
+        for (int e = tid; e < int(kMoroLdsBytes / 8); e += nthr) mtab[e] = kMoroTailF64[kMoroLdsRow * kMoroTailCoefs + e];
     for (int e = tid; e <= n; e += nthr) step_sample[e] = P.step_sample[e];
     if constexpr (sizeof(R) == 4 && !GINV)
         for (int e = tid; e < kInvNormalRows * 4; e += nthr) invn[e] = kInvNormalF32[e];
@@ -752,13 +853,19 @@ __device__ __forceinline__ void path_body(const LaunchParams& P, const int bid, 
     R* ck = AD ? static_cast<R*>(P.ckpt) + (size_t(slot) * ck_rows + (CKB ? kCkptGuardRows : 0)) * kWave : nullptr;
     // (the FULL layout is only chosen for grids of at most kMaxStoredKnots knots)
     const bool ck_lo = CKB && (!LEAN || m <= kMaxStoredKnots);
-    // FP32: states and bracket bytes interleaved by groups of four steps (a
-    // lane's four in one 16-byte / 4-byte word); FP64: one row per step
-    constexpr bool IL = CKB && sizeof(R) == 4;
+    // States and bracket bytes interleaved by groups of four steps (a lane's
+    // four in one 16-byte, in FP64 32-byte, word and one 4-byte word), except
+    // in the FP64 book, whose steps run one by one: one row per step.  FP32
+    // pads the steps to whole groups; FP64 keeps the steps from n4 on, up to
+    // three, in rows.
+    constexpr bool IL = CKB && (sizeof(R) == 4 || !BOOK);
     const int nck = ckpt_steps(n, int(sizeof(R)));
+    const int n4 = n & ~3;
     uint8_t* ckl = CKB ? reinterpret_cast<uint8_t*>(ck + size_t(nck) * kWave) : nullptr;
     // element of step i of this lane in the states (and bracket bytes)
-    auto ck_el = [&](int i) -> int { return IL ? ((i >> 2) << 8) + (lane << 2) + (i & 3) : i * kWave + lane; };
+    auto ck_el = [&](int i) -> int {
+        return IL && (sizeof(R) == 4 || i < n4) ? ((i >> 2) << 8) + (lane << 2) + (i & 3) : i * kWave + lane;
+    };
     constexpr int kStateRows = BOOK ? 8 + 2 * kMaxBookBarriers + 2 * kMaxBookGroups : 12;
     static_assert(kStateRows == (BOOK ? 8 + 2 * kMaxBookBarriers + 2 * kMaxBookGroups : 8 + 2 + 2),
                   "state rows as state_rows() counts them");
@@ -771,8 +878,32 @@ __device__ __forceinline__ void path_body(const LaunchParams& P, const int bid, 
     ks.invh = R(P.bucket_invh);
     ks.c0 = R(P.bucket_c0);
     ks.top = R(P.n_buckets - 1);
+    ks.itop = P.n_buckets - 1;
     const double s0 = P.spot;
     const int last = ns - 1;
+
+    // The spot of a barrier sample before the last.  FP64: where the smoothing
+    // zone is narrow in log-spot (half-width at most kNarrowZone), it is
+    // e^z_c e^(x - z_c) about the zone's centre z_c, with no reduction: 12
+    // instructions.  States under the zone are taken at its edge, where
+    // nothing changes; above it the polynomial increases, so a spot over the
+    // zone stays over it.  (A zone that reaches down to 0 has no lower edge in
+    // log-spot and is not narrow.)
+    constexpr bool NZONE = DUP && PRD == PRD_BARRIER && sizeof(R) == 8;
+    R z_c = R(0), z_lo = R(0);
+    ExpScale z_e{0.0, 0.0};
+    bool narrow = false;
+    if constexpr (NZONE) {
+        const R xu = log(R(P.bar_smooth)), xl = R(P.bar_xlo);
+        narrow = __builtin_amdgcn_readfirstlane(int(R(0.5) * (xu - xl) <= R(kNarrowZone))) != 0;
+        if (narrow) {
+            z_c = R(0.5) * (xu + xl);
+            double d;
+            const ExpScale s = exp_reduce(z_c, d);
+            z_e = exp_scaled2(d, s);
+            z_lo = xl - z_c;
+        }
+    }
 
     // this lane's local-vol adjoint grid: odd lanes use the second copy, which
     // halves the lanes contending for one address in an atomic
@@ -863,17 +994,27 @@ __device__ __forceinline__ void path_body(const LaunchParams& P, const int bid, 
         mrg::Lane gen;
         if constexpr (MRG) gen.start(P.mrg_jump, P.mrg_seed1, P.mrg_seed2, P.first_path + (active ? pidx : 0));
         // the inverse-normal table (LDS, or for LEAN the constant array
-        // itself) less kInvNormalRowBias rows
+        // itself) less kInvNormalRowBias rows (FP32)
         const R* invn_tab;
         if constexpr (GINV && sizeof(R) == 4) invn_tab = reinterpret_cast<const R*>(kInvNormalF32);
         else invn_tab = invn;
-        invn_tab -= 4 * kInvNormalRowBias;
+        if constexpr (sizeof(R) == 4) invn_tab -= 4 * kInvNormalRowBias;
         auto draw = [&](int i) -> R {
             if constexpr (MRG) {
                 if constexpr (sizeof(R) == 4) return gen.normal_f32(i, invn_tab);
                 else return gen.normal(i);
             }
             else return inv_normal(hl[i] ^ low_word(i), invn_tab);
+        };
+
+        // Sobol words of steps i .. i + 3 (i a multiple of four)
+        auto words4 = [&](int i, uint32_t* w) {
+            if constexpr (SPLIT) {
+                sobol_words4<kLoSplit>(lo_tab, hl, lane, i, w);
+            } else {
+#pragma unroll
+                for (int k = 0; k < 4; ++k) w[k] = hl[i + k] ^ low_word(i + k);
+            }
         };
 
         ProductState<R> ps;
@@ -921,9 +1062,9 @@ __device__ __forceinline__ void path_body(const LaunchParams& P, const int bid, 
                     if (zone) ps.alive = a_prev * f;
                     // exactly-zero factors (F = B + w), rare: from the first one on,
                     // pnz holds the product of the non-zero factors
-                    const bool fz = zone && f == R(0);
-                    nzw = nzw | (__builtin_amdgcn_ballot_w64(fz) != 0);
+                    nzw = nzw | (__builtin_amdgcn_ballot_w64(f == R(0)) != 0);
                     if (nzw) {
+                        const bool fz = zone && f == R(0);
                         if (fz) {
                             if (ps.nzero == 0) ps.pnz = a_prev;
                             ps.nzero++;
@@ -1056,6 +1197,21 @@ __device__ __forceinline__ void path_body(const LaunchParams& P, const int bid, 
         // formed there (forward and reverse)
         constexpr bool UNDER = DUP && PRD == PRD_BARRIER;
         const R x_lo = UNDER ? R(P.bar_xlo) : R(0);
+        auto zone_spot = [&](R x) -> R {
+            if constexpr (NZONE) {
+                double d;
+                ExpScale e;
+                if (narrow) {
+                    d = max_f64(x - z_c, z_lo);
+                    e = z_e;
+                } else {
+                    e = exp_reduce(x, d);
+                }
+                return exp_scaled(d, e);
+            } else {
+                return state_spot(x, s0);
+            }
+        };
         // Dupire barrier: whether timeline points base .. base + 63 are
         // samples, one wave-uniform 64-bit mask from one ballot (bit b: point
         // base + b); the sweeps test a bit per step instead of reading the
@@ -1133,7 +1289,7 @@ __device__ __forceinline__ void path_body(const LaunchParams& P, const int bid, 
                     // (a group of four steps lies in one window of 64)
                     if ((QW ? k == 0 : true) && (i & 63) == 0) fbits = sample_bits(i + 1);
                     if (((fbits >> (i & 63)) & 1u) && __builtin_amdgcn_ballot_w64(x > x_lo) != 0)
-                        observe(0, state_spot(x, s0));
+                        observe(0, zone_spot(x));
                 } else {
                     const int s = __builtin_amdgcn_readfirstlane((step_sample + i0 + 1)[k]);
                     if (s >= 0) observe(s, DUP ? state_spot(x, s0) : x);
@@ -1176,19 +1332,26 @@ __device__ __forceinline__ void path_body(const LaunchParams& P, const int bid, 
                         double pu[4];
 #pragma unroll
                         for (int k = 0; k < 4; ++k) pu[k] = gen.uniform(i + k);
-                        inv_normal4_p<TR>(pu, gz, trow, lane);
+                        inv_normal4_p<TR, SPLIT>(pu, gz, trow, mtab, lane);
                         if (gen.neg) {
 #pragma unroll
                             for (int k = 0; k < 4; ++k) gz[k] = -gz[k];
                         }
                     } else {
                         uint32_t gw[4];
-#pragma unroll
-                        for (int k = 0; k < 4; ++k) gw[k] = hl[i + k] ^ low_word(i + k);
-                        inv_normal4_f64<TR>(gw, gz, trow, lane);
+                        words4(i, gw);
+                        inv_normal4_f64<TR, SPLIT>(gw, gz, trow, mtab, lane);
                     }
 #pragma unroll
-                    for (int k = 0; k < 4; ++k) fwd_step(i, k, std::false_type{}, std::true_type{});
+                    for (int k = 0; k < 4; ++k)
+                        fwd_step(i, k, std::integral_constant<bool, IL>{}, std::true_type{});
+                    if constexpr (IL) {
+                        double2* c = reinterpret_cast<double2*>(ck + ck_el(i));
+                        c[0] = make_double2(gx[0], gx[1]);
+                        c[1] = make_double2(gx[2], gx[3]);
+                        if (ck_lo) *reinterpret_cast<uint32_t*>(ckl + ck_el(i)) = glo;
+                        glo = 0;
+                    }
                 }
             }
             if constexpr (sizeof(R) == 8 && BOOK) {
@@ -1197,7 +1360,6 @@ __device__ __forceinline__ void path_body(const LaunchParams& P, const int bid, 
                 // select, so the book's step is compiled once)
                 double* trow = tails + wave * TR;
                 double gb[4] = {0.0, 0.0, 0.0, 0.0};
-                const int n4 = n & ~3;
                 for (; i < n4; ++i) {
                     const int k = i & 3;
                     if (k == 0) {
@@ -1205,16 +1367,15 @@ __device__ __forceinline__ void path_body(const LaunchParams& P, const int bid, 
                             double pu[4];
 #pragma unroll
                             for (int j = 0; j < 4; ++j) pu[j] = gen.uniform(i + j);
-                            inv_normal4_p<TR>(pu, gb, trow, lane);
+                            inv_normal4_p<TR, SPLIT>(pu, gb, trow, mtab, lane);
                             if (gen.neg) {
 #pragma unroll
                                 for (int j = 0; j < 4; ++j) gb[j] = -gb[j];
                             }
                         } else {
                             uint32_t gw[4];
-#pragma unroll
-                            for (int j = 0; j < 4; ++j) gw[j] = hl[i + j] ^ low_word(i + j);
-                            inv_normal4_f64<TR>(gw, gb, trow, lane);
+                            words4(i, gw);
+                            inv_normal4_f64<TR, SPLIT>(gw, gb, trow, mtab, lane);
                         }
                     }
                     gz[0] = k == 0 ? gb[0] : k == 1 ? gb[1] : k == 2 ? gb[2] : gb[3];
@@ -1310,14 +1471,15 @@ __device__ __forceinline__ void path_body(const LaunchParams& P, const int bid, 
             const R alive_bar = w0 * ps.euro;             // barrier: adjoint of alive
             // at_last: s is the last sample (the last timeline point); the
             // sweeps pass a constant false inside their step loops
-            auto sample_adj = [&](int s, R F, R numv, R discv, R& Fb, R& nb, R& db, bool at_last) {
+            // Fz: the spot the forward took the barrier's smoothing factor at
+            auto sample_adj = [&](int s, R F, R Fz, R numv, R discv, R& Fb, R& nb, R& db, bool at_last) {
                 Fb = R(0); nb = R(0); db = R(0);
                 if constexpr (PRD == PRD_BARRIER) {
                     // d alive / dF = -(product of the other factors) / 2w: alive / f
                     // without a zero factor; with one, pnz for the zero factor
                     // and 0 for the others; 0 with two or more
-                    const bool zone = !ps.dead && F > R(P.minus_smooth);
-                    const R f = (ZT ? R(P.bar_smooth) - F : max(R(P.bar_smooth) - F, tiny_d)) * R(P.inv_two_smooth);
+                    const bool zone = !ps.dead && Fz > R(P.minus_smooth);
+                    const R f = (ZT ? R(P.bar_smooth) - Fz : max(R(P.bar_smooth) - Fz, tiny_d)) * R(P.inv_two_smooth);
                     R others = recip_mul(ps.alive, f);
                     if (ZT && __builtin_expect(nzw, 0))
                         others = ps.nzero == 0 ? others : ((ps.nzero == 1 && f == R(0)) ? ps.pnz : R(0));
@@ -1440,7 +1602,7 @@ __device__ __forceinline__ void path_body(const LaunchParams& P, const int bid, 
                     if (s >= 0) {
                         const R S = state_spot(x, s0);
                         R Fb, nb, db;
-                        sample_adj(s, S, R(1), R(1), Fb, nb, db, true);   // step_sample[n] is the last sample
+                        sample_adj(s, S, zone_spot(x), R(1), R(1), Fb, nb, db, true);   // step_sample[n] is the last sample
                         abar = S * Fb;
                     }
                 }
@@ -1469,7 +1631,7 @@ __device__ __forceinline__ void path_body(const LaunchParams& P, const int bid, 
                         double pu[4];
 #pragma unroll
                         for (int k = 3; k >= 0; --k) pu[k] = i0 + k < n ? gen.uniform(i0 + k) : 0.5;
-                        inv_normal4_p<TR>(pu, mz, tails + wave * TR, lane);
+                        inv_normal4_p<TR, SPLIT>(pu, mz, tails + wave * TR, mtab, lane);
                         if (gen.neg) {
 #pragma unroll
                             for (int k = 0; k < 4; ++k) mz[k] = -mz[k];
@@ -1481,8 +1643,15 @@ __device__ __forceinline__ void path_body(const LaunchParams& P, const int bid, 
                         static_assert(kSeg == 4, "FP64 segments of four draws");
                         uint32_t gw[4];
 #pragma unroll
-                        for (int k = 0; k < 4; ++k) gw[k] = i0 + k < n ? (hl[i0 + k] ^ low_word(i0 + k)) : 0x80000000u;
-                        inv_normal4_f64<TR>(gw, mz, tails + wave * TR, lane);
+                        for (int k = 0; k < 4; ++k) gw[k] = 0x80000000u;
+                        if (i0 + 4 <= n) {
+                            words4(i0, gw);
+                        } else {
+#pragma unroll
+                            for (int k = 0; k < 3; ++k)
+                                if (i0 + k < n) gw[k] = hl[i0 + k] ^ low_word(i0 + k);
+                        }
+                        inv_normal4_f64<TR, SPLIT>(gw, mz, tails + wave * TR, mtab, lane);
                     }
 #pragma unroll
                     for (int k = 0; k < kSeg; ++k) {
@@ -1506,11 +1675,11 @@ __device__ __forceinline__ void path_body(const LaunchParams& P, const int bid, 
                         const int smp = __builtin_amdgcn_readfirstlane(step_sample[i]);
                         if constexpr (UNDER) {
                             if (smp >= 0 && __builtin_amdgcn_ballot_w64(xi > x_lo) != 0)
-                                cb[k] = barrier_sf(state_spot(xi, s0));
+                                cb[k] = barrier_sf(zone_spot(xi));
                         } else if (smp >= 0) {
                             const R S = state_spot(xi, s0);
                             R Fb, nb, db;
-                            sample_adj(smp, S, R(1), R(1), Fb, nb, db, false);
+                            sample_adj(smp, S, S, R(1), R(1), Fb, nb, db, false);
                             cb[k] = S * Fb;
                         }
                         xi = euler_step(xi, b.vol, g);
@@ -1536,7 +1705,7 @@ __device__ __forceinline__ void path_body(const LaunchParams& P, const int bid, 
                     if (s >= 0) {
                         const R S = state_spot(x, s0);
                         R Fb, nb, db;
-                        sample_adj(s, S, R(1), R(1), Fb, nb, db, true);   // step_sample[n] is the last sample
+                        sample_adj(s, S, zone_spot(x), R(1), R(1), Fb, nb, db, true);   // step_sample[n] is the last sample
                         abar = S * Fb;
                     }
                 }
@@ -1547,7 +1716,7 @@ __device__ __forceinline__ void path_body(const LaunchParams& P, const int bid, 
                 const R vmin = R(sizeof(R) == 8 ? kRecoverVolF64 : kRecoverVolF32);
                 // groups of U steps, top down to top - U + 1; the checkpoint
                 // loads of the next group are issued before the current group
-                // is worked (FP64 and the book hold more registers: U = 1).
+                // is worked (the book holds more registers: U = 1; FP64 below).
                 // FP32 groups of four are the aligned groups of the interleaved
                 // checkpoints (steps 4g .. 4g + 3), one 16-byte load of states
                 // and one word of brackets each; the top group may be partial
@@ -1636,12 +1805,12 @@ __device__ __forceinline__ void path_body(const LaunchParams& P, const int bid, 
                         js[k] = b.j;
                         if constexpr (UNDER) {
                             if (smp >= 0 && __builtin_amdgcn_ballot_w64(xi > x_lo) != 0)
-                                sf[k] = barrier_sf(state_spot(xi, s0));
+                                sf[k] = barrier_sf(zone_spot(xi));
                         } else {
                             if (smp >= 0) {
                                 const R S = state_spot(xi, s0);
                                 R Fb, nb, db;
-                                sample_adj(smp, S, R(1), R(1), Fb, nb, db, false);
+                                sample_adj(smp, S, S, R(1), R(1), Fb, nb, db, false);
                                 sf[k] = S * Fb;
                             }
                         }
@@ -1670,7 +1839,82 @@ __device__ __forceinline__ void path_body(const LaunchParams& P, const int bid, 
 #pragma unroll
                     for (int k = 0; k < U; ++k) { buf[k] = nbuf[k]; lbuf[k] = nlbuf[k]; }
                 };
-                if (n > 0) {
+                if constexpr (IL && sizeof(R) == 8) {
+                    // FP64: the steps run one by one, their checkpoints loaded
+                    // in groups of four one group ahead.  (A load one step
+                    // ahead has some 1,000 cycles to come from HBM, less than
+                    // its latency under load.  2^20 paths x 156 steps, 30 x 36
+                    // grid, with the tail table in LDS: 1.04 -> 0.93 ms a call;
+                    // 2^16 paths on the 60 x 36 grid 0.286 -> 0.258.)
+                    if (n > 0) {
+                        const int last = min(n - 1, P.rev_point);
+                        if (last + 1 < n) xnext = ck[ck_el(last + 1)];
+                        auto step = [&](int i, R xi, int lo, auto recover) {
+                            constexpr bool REC = decltype(recover)::value;
+                            int smp;
+                            if constexpr (UNDER) {
+                                if ((i >> 6) != rwin) {
+                                    rwin = i >> 6;
+                                    rbits = sample_bits(rwin << 6);
+                                }
+                                smp = int(((rbits >> (i & 63)) & 1u)) - 1;
+                            } else {
+                                smp = __builtin_amdgcn_readfirstlane(step_sample[i]);
+                            }
+                            if (!ck_lo) lo = count_le<LEAN>(ks, xi);
+                            const Bracket<R> b = local_vol_at(kxi, iv + i * mp, xi, lo);
+                            R ws = recip_mul(xnext - xi, b.vol) - R(0.5) * b.vol;
+                            if constexpr (!REC)
+                                if (__builtin_amdgcn_ballot_w64(b.vol < vmin) != 0)
+                                    if (b.vol < vmin) ws = draw(i) - b.vol;
+                            R sf = R(0);
+                            if constexpr (UNDER) {
+                                if (smp >= 0 && __builtin_amdgcn_ballot_w64(xi > x_lo) != 0)
+                                    sf = barrier_sf(zone_spot(xi));
+                            } else if (smp >= 0) {
+                                const R S = state_spot(xi, s0);
+                                R Fb, nb, db;
+                                sample_adj(smp, S, S, R(1), R(1), Fb, nb, db, false);
+                                sf = S * Fb;
+                            }
+                            const R vb = abar * ws;
+                            abar = abar + vb * b.slope;
+                            abar = abar + sf;
+                            if (active) {
+                                double* row = ivbl + i * mp;
+                                atomicAdd(row + b.j, double(vb * b.wa));
+                                atomicAdd(row + b.j + 1, double(vb * b.wb));
+                            }
+                            xnext = xi;
+                        };
+                        auto sweep = [&](auto recover) {
+                            int top = last;
+                            for (; top >= n4; --top) step(top, ck[ck_el(top)], ck_lo ? int(ckl[ck_el(top)]) : 0, recover);
+                            if (top < 0) return;
+                            double2 c0, c1;
+                            uint32_t cw;
+                            auto load4 = [&](int g) {
+                                const int e = (g << 8) + (lane << 2);
+                                const double2* c = reinterpret_cast<const double2*>(ck + e);
+                                c0 = c[0];
+                                c1 = c[1];
+                                cw = ck_lo ? *reinterpret_cast<const uint32_t*>(ckl + e) : 0u;
+                            };
+                            load4(top >> 2);
+                            for (int g = top >> 2; g >= 0; --g) {
+                                const double2 a0 = c0, a1 = c1;
+                                const uint32_t w = cw;
+                                load4(g - 1);   // (the slot's guard rows below step 0, never used)
+                                const int i = g << 2;
+                                if (i + 3 <= top) step(i + 3, a1.y, int(w >> 24), recover);
+                                if (i + 2 <= top) step(i + 2, a1.x, int((w >> 16) & 0xffu), recover);
+                                if (i + 1 <= top) step(i + 1, a0.y, int((w >> 8) & 0xffu), recover);
+                                step(i, a0.x, int(w & 0xffu), recover);
+                            }
+                        };
+                        if (iv_recover) sweep(std::true_type{}); else sweep(std::false_type{});
+                    }
+                } else if (n > 0) {
                     // the sweep starts at the last point whose sample carries
                     // weight (one payoff's reverse of itemized risk: later
                     // steps have no adjoint), the next state from its checkpoint
@@ -1702,7 +1946,7 @@ __device__ __forceinline__ void path_body(const LaunchParams& P, const int bid, 
                     const R numv = P.spot_measure ? R(s_num[s]) * S : R(s_num[s]);
                     const R discv = R(s_disc[s]);
                     R Fb, nb, db;
-                    sample_adj(s, F, numv, discv, Fb, nb, db, s == last);
+                    sample_adj(s, F, F, numv, discv, Fb, nb, db, s == last);
                     // dF = F (tau + dff/ff), ff = exp(mu (Tf - t))
                     const R tfs = R(tf[s]), tds = R(td[s]), ts = R(tl[s]);
                     R dF[4] = {F * tau[0], F * tau[1], F * (tau[2] + tfs), F * (tau[3] - tfs)};
