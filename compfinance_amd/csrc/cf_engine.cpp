@@ -394,8 +394,21 @@ BookTables build_book(const ProductPlan& d, double width0)
     };
     vector<vector<std::pair<double, int>>> van(ns);
     vector<uint32_t> bar_mask(ns, 0u), bar_last(ns, 0u), grp_mask(ns, 0u), grp_last(ns, 0u);
-    vector<double> bar_par;
-    vector<int> bar_col, bar_put;
+    // the barriers take their places in order of the lower end B - w of their
+    // zone: the kernels stop at the first zone no path has reached
+    vector<double> bar_lo;
+    for (const ProductPlan* q : parts)
+        if (q->kind == CF_PRODUCT_BARRIER) bar_lo.push_back(q->barrier - width0 * q->smooth);
+    vector<int> bar_place(bar_lo.size());
+    for (size_t i = 0; i < bar_lo.size(); ++i)
+        for (size_t j = 0; j < bar_lo.size(); ++j)
+            if (bar_lo[j] < bar_lo[i] || (bar_lo[j] == bar_lo[i] && j < i)) ++bar_place[i];
+    const size_t n_bars = bar_lo.size();
+    if (n_bars > size_t(cfk::kMaxBookBarriers))
+        fail(CF_ERR_CAPACITY, "a book holds at most " + std::to_string(cfk::kMaxBookBarriers) + " barriers");
+    size_t bars_seen = 0;
+    vector<double> bar_par(4 * n_bars);
+    vector<int> bar_col(n_bars), bar_put(n_bars);
     vector<vector<double>> sched;                       // fixing schedules
     vector<vector<std::tuple<double, int, int>>> members;   // per schedule: strike, column, put
     int col = 0;
@@ -406,15 +419,16 @@ BookTables build_book(const ProductPlan& d, double width0)
             for (size_t i = 0; i < q->mats.size(); ++i)
                 for (double k : q->strikes[i]) van[at(q->mats[i])].push_back({k, col++});
         } else if (q->kind == CF_PRODUCT_BARRIER) {
-            const int b = int(bar_col.size());
-            if (b >= cfk::kMaxBookBarriers)
-                fail(CF_ERR_CAPACITY, "a book holds at most " + std::to_string(cfk::kMaxBookBarriers) + " barriers");
+            const size_t b = size_t(bar_place[bars_seen++]);
             for (double t : q->timeline) bar_mask[at(t)] |= 1u << b;
             bar_last[at(q->timeline.back())] |= 1u << b;
             const double w = width0 * q->smooth;
-            bar_par.insert(bar_par.end(), {q->strike, q->barrier + w, q->barrier - w, 1.0 / (2 * w)});
-            bar_col.push_back(col);
-            bar_put.push_back(q->put ? 1 : 0);
+            bar_par[4 * b] = q->strike;
+            bar_par[4 * b + 1] = q->barrier + w;
+            bar_par[4 * b + 2] = q->barrier - w;
+            bar_par[4 * b + 3] = 1.0 / (2 * w);
+            bar_col[b] = col;
+            bar_put[b] = q->put ? 1 : 0;
             col += 2;
         } else if (q->kind == CF_PRODUCT_ASIAN) {
             size_t g = 0;
@@ -472,17 +486,35 @@ BookTables build_book(const ProductPlan& d, double width0)
     // maturing (16-31), schedules fixing (bits 0-3) and ending (4-7), and its
     // vanillas [van_first[s], van_first[s + 1])
     vector<uint32_t> masks(size_t(ns) * 4);
+    const uint32_t all_bars = (1u << n_bars) - 1u;
     for (int k = 0; k < ns; ++k) {
         masks[4 * k] = bar_mask[k] | (bar_last[k] << 16);
         masks[4 * k + 1] = grp_mask[k] | (grp_last[k] << 4);
+        if (n_bars > 0 && bar_mask[k] == all_bars && bar_last[k] == 0) {
+            masks[4 * k + 1] |= cfk::kBookAllBars;
+            if (grp_mask[k] == 0 && van[k].empty()) masks[4 * k + 1] |= cfk::kBookPlain;
+        }
         masks[4 * k + 2] = uint32_t(van_first[k]);
         masks[4 * k + 3] = uint32_t(van_first[k + 1]);
     }
     L.masks = put(masks.data(), masks.size() * 4);
-    L.bar_par = put(bar_par.data(), bar_par.size() * 8);
-    const vector<float> bar_par_f(bar_par.begin(), bar_par.end());
-    L.bar_par_f = put(bar_par_f.data(), bar_par_f.size() * 4);
-    for (size_t b = 0; b < bar_col.size(); ++b) B.lo_min = std::min(B.lo_min, bar_par[4 * b + 2]);
+    // the fours follow (bar_par holds 32 bytes a barrier, 16 in float)
+    vector<double> pars = bar_par;
+    for (size_t b = 0; b < size_t(cfk::kMaxBookBarriers); b += 4) {
+        const double inf = std::numeric_limits<double>::infinity();
+        double p[16] = {inf, inf, inf, inf, inf, inf, inf, inf, 1.0, 1.0, 1.0, 1.0, 0.0, 0.0, 0.0, 0.0};
+        for (size_t j = 0; j < 4 && b + j < n_bars; ++j) {
+            p[j] = bar_par[4 * (b + j) + 2];
+            p[4 + j] = bar_par[4 * (b + j) + 1];
+            p[8 + j] = bar_par[4 * (b + j) + 3];
+        }
+        pars.insert(pars.end(), p, p + 16);
+    }
+    L.bar_par = put(pars.data(), pars.size() * 8);
+    const vector<float> pars_f(pars.begin(), pars.end());
+    L.bar_par_f = put(pars_f.data(), pars_f.size() * 4);
+    B.rows = masks;
+    for (size_t b = 0; b < n_bars; ++b) B.lo_min = std::min(B.lo_min, bar_par[4 * b + 2]);
     L.bar_col = put(bar_col.data(), bar_col.size() * 4);
     L.bar_put = put(bar_put.data(), bar_put.size() * 4);
     L.grp_inv = put(grp_inv.data(), grp_inv.size() * 8);
@@ -926,7 +958,17 @@ std::shared_ptr<Prepared> prepare(Engine& E, const cf_model* mdl, const cf_produ
         P->o_pf = st.add(pd.pay_first);
         P->o_pk = st.add(pd.pay_strike);
     }
-    if (book) P->o_book = st.add(P->book.blob);
+    if (book) {
+        P->o_book = st.add(P->book.blob);
+        if (dup) {
+            // the book's rows by timeline point (empty where it is no sample)
+            vector<uint32_t> rows(size_t(md.n_steps + 1) * 4, 0u);
+            for (int i = 0; i <= md.n_steps; ++i)
+                if (md.step_sample[size_t(i)] >= 0)
+                    std::copy_n(P->book.rows.begin() + 4 * md.step_sample[size_t(i)], 4, rows.begin() + 4 * i);
+            P->o_pf = st.add(rows);
+        }
+    }
     {
         const vector<uint64_t> jump = mrg_jumps(md.n_steps);
         P->o_mrg = st.add(jump);
@@ -1079,7 +1121,10 @@ cfk::LaunchParams launch_params(const Engine& E, const Prepared& PR, const CallS
     P.pay_strike = reinterpret_cast<const double*>(dt + PR.o_pk);
     P.book = dt + PR.o_book;
     P.bk = PR.book.L;
-    P.book_lo = PR.book.lo_min;
+    if (PR.cfg.product == cfk::PRD_BOOK) {
+        P.bar_xlo = PR.book.lo_min > 0 ? std::log(S.fp64 ? PR.book.lo_min : PR.book.lo_min / md.spot) : -HUGE_VAL;
+        if (std::isfinite(P.bar_xlo)) P.bar_xlo -= (S.fp64 ? 1e-10 : 1e-4) * (1 + std::fabs(P.bar_xlo));
+    }
 
     P.block_out = B.block_out;
     P.per_path = B.per_path;

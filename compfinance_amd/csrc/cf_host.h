@@ -101,6 +101,7 @@ struct BookTables {
     vector<unsigned char> blob;
     cfk::BookLayout L{};
     double lo_min = HUGE_VAL;      // the lowest B - w of the barriers
+    vector<uint32_t> rows;         // [n_samples][4], BookLayout::masks
 };
 
 struct ModelPlan {

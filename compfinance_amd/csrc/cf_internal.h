@@ -40,15 +40,19 @@ constexpr double kRecoverVolF64 = 0x1p-10, kRecoverVolF32 = 0x1p-8;
 // Book of products on shared paths (also an Asian on its own): vanilla calls
 // attached to samples, up-and-out barriers and arithmetic-average groups.  Each
 // barrier and each distinct fixing schedule keeps per-lane state in registers,
-// hence the bounds; the book kernels run 512-thread blocks for the registers.
+// hence the bounds on them and on the book kernels' blocks.
 constexpr int kMaxBookBarriers = 16, kMaxBookGroups = 4;
-constexpr int kBookBlock = 512;
+// Bits of a sample's schedule word: every barrier of the book observes at it
+// and none matures; and nothing else happens at it either.
+constexpr uint32_t kBookAllBars = 0x100u, kBookPlain = 0x200u;
 
 // Threads per block of a path kernel: 1024, except the book kernels whose
-// registers need 512 (FP64, and the FP32 recompute variant).
+// registers need 512 (FP64, and the FP32 recompute variant).  (FP64 checkpoint
+// kernels of 768 threads, 168 registers with some spills, ran 2^18 paths in
+// 0.86 ms against 0.77: two passes of the waves either way.)
 constexpr int book_block_limit(int prd, int real_bytes, int adj)
 {
-    return prd == PRD_BOOK && (real_bytes == 8 || adj == ADJ_RECOMPUTE) ? kBookBlock : 1024;
+    return prd == PRD_BOOK && (real_bytes == 8 || adj == ADJ_RECOMPUTE) ? 512 : 1024;
 }
 
 // Byte offsets of the book tables inside one blob (staged whole in LDS).
@@ -59,9 +63,12 @@ struct BookLayout {
     int van_col;      // [n_van] int: payoff column
     int masks;        // [n_samples][4] uint32, 16-byte rows: barriers observing at s (bits 0-15)
                       // and maturing at s (16-31), schedules fixing at s (bits 0-3) and ending
-                      // at s (4-7), first vanilla of s, first vanilla of s + 1
-    int bar_par;      // [n_bar][4] double: strike, B + w, B - w, 1 / 2w
-    int bar_par_f;    // [n_bar][4] the same in float
+                      // at s (4-7) with kBookAllBars and kBookPlain, first vanilla of s, first
+                      // vanilla of s + 1
+    int bar_par;      // [n_bar][4] double: strike, B + w, B - w, 1 / 2w, in order of B - w; then
+                      // [kMaxBookBarriers / 4][16]: the same by fours (four B - w, four B + w,
+                      // four 1 / 2w, four unused), +infinity past the last barrier
+    int bar_par_f;    // the same in float
     int bar_col;      // [n_bar] int: column of the barrier payoff (vanilla next)
     int bar_put;      // [n_bar] int
     int grp_inv;      // [n_grp] double: 1 / number of fixings
@@ -86,8 +93,7 @@ constexpr double kNarrowZone = 0.05;
 // step i of lane l is element ((i >> 2) * 64 + l) * 4 + (i & 3) (a lane's four
 // states in one 16-byte word, 32 bytes in FP64), its bracket byte the same
 // element of the byte rows that follow the states.  FP32 pads the steps to a
-// multiple of four; FP64 keeps the last n_steps % 4 steps in rows of 64, and
-// its book all of them.
+// multiple of four; FP64 keeps the last n_steps % 4 steps in rows of 64.
 constexpr int kMaxStoredKnots = 255;
 constexpr int kCkptGuardRows = 4;
 CF_HD inline int ckpt_steps(int n_steps, int real_bytes) { return real_bytes == 4 ? (n_steps + 3) & ~3 : n_steps; }
@@ -155,13 +161,13 @@ struct LaunchParams {
     int put;
     double strike;
     double bar_smooth, minus_smooth, two_smooth, inv_two_smooth;
-    double bar_xlo;              // Dupire barrier: at or below this state the spot is under the
-                                 // smoothing zone (with a margin over exp's rounding)
-    const int* pay_first;        // Europeans [n_samples + 1]: payoffs of sample s
+    double bar_xlo;              // Dupire barrier and book: at or below this state the spot is under
+                                 // every smoothing zone (with a margin over exp's rounding)
+    const int* pay_first;        // Europeans [n_samples + 1]: payoffs of sample s; a book on Dupire:
+                                 // [n_steps + 1][4], its rows (BookLayout::masks) by timeline point
     const double* pay_strike;    // Europeans [n_pay]
     const void* book;            // book tables, layout bk
     BookLayout bk;
-    double book_lo;              // the lowest B - w of the book's barriers (+inf without one)
 
     // mrg32k3a (null: Sobol): jump matrices [32][2][9], the two component
     // matrices raised to n_steps * 2^j (mod m1, m2), and the seeds as residues

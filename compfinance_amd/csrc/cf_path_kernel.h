@@ -433,12 +433,37 @@ struct Lane {
 };
 }   // namespace mrg
 
-// exp in FP64, in two parts.  exp_reduce: x = n ln(2) / 8 + d with |d| <=
-// 0.0434, and the scale 2^(n / 8) as a sum hi + lo (x beyond +-800 saturates
-// to 0 or infinity).  exp_scaled: (hi + lo) e^d by the Taylor polynomial of
-// degree 8 (truncation below 6e-18 for |d| <= 0.05), the product with hi - 1
-// added last: within 0.51 ulp, in 25 instructions and one 16-byte read
-// against the library function's 35.
+// e^d - 1 over d, without its leading 1: the Taylor series of degree N - 1
+// from d / 2 on, by Horner's rule; N = 8 for |d| <= 0.05 (truncation of e^d below
+// 6e-18), N = 13 for |d| <= 0.3466 (4e-18).
+template <int N>
+__device__ __forceinline__ double exp_series(double d)
+{
+    constexpr double c[14] = {1.0, 1.0, 1.0 / 2.0, 1.0 / 6.0, 1.0 / 24.0, 1.0 / 120.0, 1.0 / 720.0, 1.0 / 5040.0,
+                              1.0 / 40320.0, 1.0 / 362880.0, 1.0 / 3628800.0, 1.0 / 39916800.0, 1.0 / 479001600.0,
+                              1.0 / 6227020800.0};
+    double q = fma(d, c[N], c[N - 1]);
+#pragma unroll
+    for (int k = N - 2; k >= 3; --k) q = fma_s(q, d, c[k]);
+    return fma(q, d, 0.5);
+}
+// exp in FP64: x = n ln(2) + d, 2^n (1 + (d + d^2 series)), within 0.8 ulp; x
+// beyond +-800 saturates to 0 or infinity.  22 instructions, no table (a load
+// would wait for the checkpoint stores issued before it), against the library
+// function's 35.
+__device__ __forceinline__ double exp_f64(double x)
+{
+    x = min_f64(max_f64(x, -800.0), 800.0);
+    const double n = __builtin_rint(x * 1.4426950408889634);
+    // ln(2) in two parts, the first of 33 bits: n times it is exact
+    double d = fma(n, -6.93147180369123816490e-01, x);
+    d = fma(n, -1.90821492927058770002e-10, d);
+    const double r = fma(d * d, exp_series<13>(d), d);
+    return __builtin_amdgcn_ldexp(1.0 + r, int(n));
+}
+
+// e^x as a sum hi + lo good to some 2^-60, for constants formed once per block:
+// x = n ln(2) / 8 + d, 2^(n / 8) from a table as a sum.
 static __constant__ double kExpEighths[16] = {   // 2^(j / 8), hi and lo
     1.00000000000000000e+00, 0.00000000000000000e+00,
     1.09050773266525769e+00, -3.04678207981247115e-17,
@@ -452,43 +477,17 @@ static __constant__ double kExpEighths[16] = {   // 2^(j / 8), hi and lo
 struct ExpScale {
     double hi, lo;
 };
-__device__ __forceinline__ ExpScale exp_reduce(double x, double& d)
+__device__ __forceinline__ ExpScale exp_pair(double x)
 {
-    x = min_f64(max_f64(x, -800.0), 800.0);
     const double n = __builtin_rint(x * 11.541560327111707);   // 8 / ln(2)
     // ln(2) / 8 in two parts, the first of 29 bits: n times it is exact
-    d = fma(n, -8.66433973424136638641e-02, x);
+    double d = fma(n, -8.66433973424136638641e-02, x);
     d = fma(n, -2.27579499813018278006e-10, d);
     const int k = int(n);
     const double2 t = reinterpret_cast<const double2*>(kExpEighths)[k & 7];
-    ExpScale s;
-    s.hi = __builtin_amdgcn_ldexp(t.x, k >> 3);
-    s.lo = __builtin_amdgcn_ldexp(t.y, k >> 3);
-    return s;
-}
-// (exp_tail: (hi + lo) e^d - hi; exp_scaled2: the result and its rounding)
-__device__ __forceinline__ double exp_tail(double d, ExpScale s)
-{
-    double q = fma(d, 1.0 / 40320.0, 1.0 / 5040.0);
-    q = fma_s(q, d, 1.0 / 720.0);
-    q = fma_s(q, d, 1.0 / 120.0);
-    q = fma_s(q, d, 1.0 / 24.0);
-    q = fma_s(q, d, 1.0 / 6.0);
-    q = fma(q, d, 0.5);
-    q = fma(q, d, 1.0);
-    return fma(s.hi, q * d, s.lo);
-}
-__device__ __forceinline__ double exp_scaled(double d, ExpScale s) { return s.hi + exp_tail(d, s); }
-__device__ __forceinline__ ExpScale exp_scaled2(double d, ExpScale s)
-{
-    const double t = exp_tail(d, s), hi = s.hi + t;
-    return {hi, (s.hi - hi) + t};
-}
-__device__ __forceinline__ double exp_f64(double x)
-{
-    double d;
-    const ExpScale s = exp_reduce(x, d);
-    return exp_scaled(d, s);
+    const double r = fma(d * d, exp_series<8>(d), d);
+    const double s = fma(t.x, r, t.y), hi = t.x + s;
+    return {__builtin_amdgcn_ldexp(hi, k >> 3), __builtin_amdgcn_ldexp((t.x - hi) + s, k >> 3)};
 }
 
 // Spot from the path state: FP64 state is log(S) (reference), FP32 state is
@@ -855,10 +854,9 @@ __device__ __forceinline__ void path_body(const LaunchParams& P, const int bid, 
     const bool ck_lo = CKB && (!LEAN || m <= kMaxStoredKnots);
     // States and bracket bytes interleaved by groups of four steps (a lane's
     // four in one 16-byte, in FP64 32-byte, word and one 4-byte word), except
-    // in the FP64 book, whose steps run one by one: one row per step.  FP32
-    // pads the steps to whole groups; FP64 keeps the steps from n4 on, up to
-    // three, in rows.
-    constexpr bool IL = CKB && (sizeof(R) == 4 || !BOOK);
+    // FP32 pads the steps to whole groups; FP64 keeps the steps from n4 on,
+    // up to three, in rows.
+    constexpr bool IL = CKB;
     const int nck = ckpt_steps(n, int(sizeof(R)));
     const int n4 = n & ~3;
     uint8_t* ckl = CKB ? reinterpret_cast<uint8_t*>(ck + size_t(nck) * kWave) : nullptr;
@@ -898,9 +896,7 @@ __device__ __forceinline__ void path_body(const LaunchParams& P, const int bid, 
         narrow = __builtin_amdgcn_readfirstlane(int(R(0.5) * (xu - xl) <= R(kNarrowZone))) != 0;
         if (narrow) {
             z_c = R(0.5) * (xu + xl);
-            double d;
-            const ExpScale s = exp_reduce(z_c, d);
-            z_e = exp_scaled2(d, s);
+            z_e = exp_pair(z_c);
             z_lo = xl - z_c;
         }
     }
@@ -924,7 +920,11 @@ __device__ __forceinline__ void path_body(const LaunchParams& P, const int bid, 
         uint32_t bars, grps;
         int van_lo, van_hi;
     };
-    CPtr<SampleRow> bk_rows_c = cptr<SampleRow>(bkb + P.bk.masks);
+    // (grps also: kBookAllBars, every barrier observes and none matures;
+    // kBookPlain, nothing else happens either).  Dupire: one row per timeline
+    // point (an empty row where it is no sample), so that a step's row is read
+    // by its own index, ahead of the step; Black-Scholes: one per sample.
+    CPtr<SampleRow> bk_rows_c = cptr<SampleRow>(DUP ? static_cast<const void*>(P.pay_first) : bkb + P.bk.masks);
     auto bk_rows = [&](int s) -> SampleRow {
         SampleRow r;
         r.bars = bk_rows_c[s].bars;
@@ -933,6 +933,13 @@ __device__ __forceinline__ void path_body(const LaunchParams& P, const int bid, 
         r.van_hi = bk_rows_c[s].van_hi;
         return r;
     };
+    // barriers by fours, in the kernel's precision, past the last one at
+    // +infinity: the lower ends of their zones, B + w, 1 / 2w
+    struct alignas(16) BarFour {
+        R lo[4], up[4], i2s[4], pad[4];
+    };
+    CPtr<BarFour> bk_four_c =
+        cptr<BarFour>(bkb + (sizeof(R) == 4 ? P.bk.bar_par_f + P.bk.n_bar * 16 : P.bk.bar_par + P.bk.n_bar * 32));
     CPtr<int> bk_grp_first = cptr<int>(bkb + P.bk.grp_first);
     CPtr<double> bk_as_strike = cptr<double>(bkb + P.bk.as_strike);
     CPtr<int> bk_as_col = cptr<int>(bkb + P.bk.as_col);
@@ -955,7 +962,6 @@ __device__ __forceinline__ void path_body(const LaunchParams& P, const int bid, 
         return r;
     };
     CPtr<double> wts = cptr<double>(P.weights);
-    const R bk_lo = R(P.book_lo);   // the lowest B - w (rounding keeps it the lowest)
     // Barrier smoothing factors (B + w - F) / 2w: FP64 tracks exactly-zero
     // factors (F = B + w) as the tape does.  FP32 keeps B + w - F at least
     // tiny_d instead, so a factor is never 0 and the product of the others,
@@ -965,14 +971,31 @@ __device__ __forceinline__ void path_body(const LaunchParams& P, const int bid, 
     const R tiny_d = ZT ? R(0) : max(R(P.two_smooth) * R(1e-30), R(1e-37));
     constexpr int NBAR = BOOK ? kMaxBookBarriers : 1, NGRP = BOOK ? kMaxBookGroups : 1;
     // Book barrier state in one real per barrier:
+    //   sign bit set  breached (survival 0, no derivative)
     //   v in [0, 1]   no exactly-zero smoothing factor yet, v = product of the
     //                 factors (the survival factor)
-    //   v in [-1, 0)  one zero factor, -v = product of the others (FP64)
-    //   v = -2        two or more zero factors (FP64)
-    //   v = -4        breached (survival 0, no derivative)
-    // FP32 keeps every factor at least 1e-30 (as the single barrier keeps
-    // B + w - F above a floor), so its states are only [0, 1] or -4.
-    constexpr float kTwoZeros = -2.0f, kBreached = -4.0f;
+    //   v > 1         one zero factor, v = 2^1000 x the product of the others
+    //                 (FP64; a second one makes it 0, as two have no derivative)
+    // A smoothing factor is (B + w - F) / 2w clamped to [0, 1], so an update is
+    // a product for every lane, in the zone, under it or breached.  FP32 keeps
+    // every factor at least 1e-30 (as the single barrier keeps B + w - F above
+    // a floor), so its states are only [0, 1] or breached.
+    constexpr double kZeroScale = 0x1p1000, kZeroMark = 0x1p600;   // (weighted: above the mark)
+    // v after an observation at distance t = B + w - F, 1 / 2w = i2s
+    auto bar_update = [&](R v, R t, R i2s) -> R {
+        if constexpr (sizeof(R) == 4) {
+            const R f = __builtin_amdgcn_fmed3f(t * i2s, 1e-30f, 1.0f);
+            return __uint_as_float(__float_as_uint(v * f) | (__float_as_uint(t) & 0x80000000u));
+        } else {
+            double f;
+            asm("v_mul_f64 %0, %1, %2 clamp" : "=v"(f) : "v"(t), "s"(i2s));
+            const uint64_t sign = __builtin_bit_cast(uint64_t, t) & (uint64_t(1) << 63);
+            return __builtin_bit_cast(double, __builtin_bit_cast(uint64_t, v * f) | sign);
+        }
+    };
+    // the survival factor of a state
+    auto bar_alive = [&](R v) -> R { return v > R(0) && (!ZT || v <= R(1)) ? v : R(0); };
+    const R bk_xlo = BOOK && DUP ? R(P.bar_xlo) : R(0);   // every zone is above this state
 
     for (int64_t q = q0 + int64_t(bid) * waves + wave; q <= qe; q += int64_t(nblk) * waves) {
         // ---- high Sobol words of this block of 64 indices (and of the
@@ -1025,9 +1048,16 @@ __device__ __forceinline__ void path_body(const LaunchParams& P, const int bid, 
         // vanilla, the adjoint of its survival factor; per fixing schedule
         // the running sum, replaced at its last fixing by the adjoint of each
         // fixing, and the weighted intrinsic value (numeraire adjoint)
-        R bst[NBAR], babar[NBAR], gsum[NGRP], gq[NGRP];
+        // (FP64 keeps one value per barrier: at its maturity the state is
+        // replaced by its product with weight x vanilla, 0 after a breach,
+        // which is all that the reverse needs; its registers bound the waves
+        // on a compute unit)
+        constexpr int NBB = ZT ? 1 : NBAR;
+        R bst[NBAR], babar[NBB], gsum[NGRP], gq[NGRP];
 #pragma unroll
-        for (int b = 0; b < NBAR; ++b) { bst[b] = R(1); babar[b] = R(0); }
+        for (int b = 0; b < NBAR; ++b) bst[b] = R(1);
+#pragma unroll
+        for (int b = 0; b < NBB; ++b) babar[b] = R(0);
 #pragma unroll
         for (int g = 0; g < NGRP; ++g) { gsum[g] = R(0); gq[g] = R(0); }
 
@@ -1042,7 +1072,8 @@ __device__ __forceinline__ void path_body(const LaunchParams& P, const int bid, 
 
         // observation of product sample s with spot S (and for Black-Scholes
         // the sample's forward factor / numeraire / discount)
-        auto observe = [&](int s, R S) {
+        // (book: with the sample's row sm)
+        auto observe = [&](int s, R S, SampleRow sm) {
             R F = S, numv = R(1), discv = R(1);
             if constexpr (!DUP) {
                 F = S * R(s_ff[s]);
@@ -1088,57 +1119,73 @@ __device__ __forceinline__ void path_body(const LaunchParams& P, const int bid, 
                 if (P.per_path && active) P.per_path[pidx * npay] = v;
                 if constexpr (AD) ps.aggp = ps.aggp + R(wts[0]) * pay;
             } else if constexpr (PRD == PRD_BOOK) {
-                const SampleRow sm = bk_rows(s);
                 // vanilla calls at this sample (European / Europeans parts)
                 for (int k = sm.van_lo; k < sm.van_hi; ++k) {
                     const R kk = R(bk_van_strike[k]);
                     emit(bk_van_col[k], (F - kk > R(0) ? F - kk : R(0)) / numv);
                 }
-                // up-and-out barriers (mcPrd.h:256-287, one state per barrier),
-                // branch free: breach, smoothing zone, exactly-zero factor;
-                // no state changes while no lane is at or above the lowest zone
-                const uint32_t bm0 = sm.bars & 0xffffu, bl = sm.bars >> 16;
-                const uint32_t bm = bm0 && __any(F > bk_lo) ? bm0 : 0u;
-                if (bm | bl) {
+                // up-and-out barriers (mcPrd.h:256-287, one state per barrier,
+                // ordered by the lower end of their zone): a product per
+                // barrier for all lanes (bar_update), no state changes while no
+                // lane is above the zone.  A wave vote per barrier instead, to
+                // skip those with no live lane in the zone, visits half as many
+                // but costs more scalar work and branches than it saves.
+                const uint32_t bl = sm.bars >> 16;
+                const bool all_bars = (sm.grps & kBookAllBars) != 0;
+                if (all_bars) {
+#pragma unroll
+                    for (int b = 0; b + 3 < NBAR; b += 4) {
+                        if (__builtin_amdgcn_ballot_w64(F > bk_four_c[b >> 2].lo[0]) == 0) continue;
+                        R up[4], i2s[4];
+#pragma unroll
+                        for (int j = 0; j < 4; ++j) {
+                            up[j] = bk_four_c[b >> 2].up[j];
+                            i2s[j] = bk_four_c[b >> 2].i2s[j];
+                        }
+                        R t[4], v[4];
+                        uint64_t zero = 0;
+#pragma unroll
+                        for (int j = 0; j < 4; ++j) {
+                            t[j] = up[j] - F;
+                            v[j] = bst[b + j];
+                            if constexpr (ZT) zero |= __builtin_amdgcn_ballot_w64(t[j] == R(0));
+                            bst[b + j] = bar_update(v[j], t[j], i2s[j]);
+                        }
+                        if (ZT && zero != 0) {
+                            asm volatile("");   // an exactly-zero factor: rare, a branch of its own
+#pragma unroll
+                            for (int j = 0; j < 4; ++j)
+                                if (t[j] == R(0) && !(v[j] > R(1))) bst[b + j] = v[j] * R(kZeroScale);
+                        }
+                    }
+                }
+                if (!all_bars && sm.bars) {
 #pragma unroll
                     for (int b = 0; b < NBAR; ++b) {
-                        if (!(((bm | bl) >> b) & 1u)) continue;
+                        if (!(((sm.bars | bl) >> b) & 1u)) continue;
                         const BarPar bp = bar_par(b);
-                        // the state changes only at or above the zone and only
-                        // before a breach: skipped when no live lane of the wave
-                        // is there
-                        if (((bm >> b) & 1u) && __any(F > bp.lo && bst[b] > R(kBreached))) {
-                            const R bs = bp.up, ms = bp.lo;
-                            const R v = bst[b];
-                            const bool live = v > R(kBreached);
-                            const bool zone = live && F > ms && !(F > bs);
-                            R nv = v;
-                            if constexpr (ZT) {
-                                const R f = (bs - F) * bp.i2s;
-                                nv = zone && f != R(0) && v >= R(-1) ? v * f : nv;          // one more factor
-                                nv = zone && f == R(0) ? (v >= R(0) ? -v : R(kTwoZeros)) : nv;   // a zero factor
-                            } else {
-                                // FP32: a factor at least 1e-30, never exactly 0
-                                // (the state stays in [0, 1] until a breach)
-                                const R f = max((bs - F) * bp.i2s, R(1e-30));
-                                nv = v * (zone ? f : R(1));
-                            }
-                            nv = live && F > bs ? R(kBreached) : nv;                    // breach
-                            bst[b] = nv;
+                        if ((sm.bars >> b) & 1u) {
+                            const R t = bp.up - F, v = bst[b];
+                            bst[b] = bar_update(v, t, bp.i2s);
+                            if (ZT && t == R(0) && !(v > R(1))) bst[b] = v * R(kZeroScale);
                         }
                         if ((bl >> b) & 1u) {
                             const R k = bp.k;
                             const R intrinsic = bk_bar_put[b] ? (k - F > R(0) ? k - F : R(0))
                                                                          : (F - k > R(0) ? F - k : R(0));
                             const R euro = intrinsic / numv;
-                            const R alive = bst[b] > R(0) ? bst[b] : R(0);
+                            const R alive = bar_alive(bst[b]);
                             const int col = bk_bar_col[b];
                             emit(col, alive * euro);
                             emit(col + 1, euro);
                             // weight x vanilla: the adjoint of the survival
                             // factor (the ITEM kernels keep the vanilla and
                             // weigh it before the reverse sweep)
-                            if constexpr (AD) babar[b] = ITEM ? euro : R(wts[col]) * euro;
+                            if constexpr (AD) {
+                                const R we = ITEM ? euro : R(wts[col]) * euro;
+                                if constexpr (ZT) bst[b] = bst[b] > R(0) ? we * bst[b] : R(0);
+                                else babar[b] = we;
+                            }
                         }
                     }
                 }
@@ -1192,6 +1239,11 @@ __device__ __forceinline__ void path_body(const LaunchParams& P, const int bid, 
             }
         };
 
+        // book: the row of sample s, at timeline point i
+        auto row_of = [&](int s, int i) -> SampleRow {
+            if constexpr (BOOK) return bk_rows(DUP ? i : s);
+            else return SampleRow{};
+        };
         // Dupire barrier: a sample other than the last one changes nothing
         // while the spot is under the smoothing zone, so the spot is not
         // formed there (forward and reverse)
@@ -1199,15 +1251,10 @@ __device__ __forceinline__ void path_body(const LaunchParams& P, const int bid, 
         const R x_lo = UNDER ? R(P.bar_xlo) : R(0);
         auto zone_spot = [&](R x) -> R {
             if constexpr (NZONE) {
-                double d;
-                ExpScale e;
-                if (narrow) {
-                    d = max_f64(x - z_c, z_lo);
-                    e = z_e;
-                } else {
-                    e = exp_reduce(x, d);
-                }
-                return exp_scaled(d, e);
+                if (!narrow) return exp_f64(x);
+                const double d = max_f64(x - z_c, z_lo);
+                const double r = fma(d * d, exp_series<8>(d), d);
+                return z_e.hi + fma(z_e.hi, r, z_e.lo);
             } else {
                 return state_spot(x, s0);
             }
@@ -1234,7 +1281,7 @@ __device__ __forceinline__ void path_body(const LaunchParams& P, const int bid, 
 #pragma unroll
             for (int b = 0; b < NBAR; ++b) {
                 bst[b] = stq[(8 + b) * kWave];
-                babar[b] = stq[(8 + NBAR + b) * kWave];
+                if constexpr (!ZT) babar[b] = stq[(8 + NBAR + b) * kWave];
             }
 #pragma unroll
             for (int g = 0; g < NGRP; ++g) {
@@ -1250,7 +1297,7 @@ __device__ __forceinline__ void path_body(const LaunchParams& P, const int bid, 
             if constexpr (DUP) x = R(P.x0); else x = R(s0);   // Dupire: log-spot state; BS: spot
             {
                 const int s = step_sample[0];
-                if (s >= 0) observe(s, DUP ? state_spot(x, s0) : x);
+                if (s >= 0) observe(s, UNDER ? zone_spot(x) : DUP ? state_spot(x, s0) : x, row_of(s, 0));
             }
             // step i0 + k, with every per-step address a fixed offset (k) from a
             // base formed once per group of steps at i0.  GRP: a step of an
@@ -1263,6 +1310,8 @@ __device__ __forceinline__ void path_body(const LaunchParams& P, const int bid, 
             auto fwd_step = [&](int i0, int k, auto grp, auto qw) {
                 constexpr bool GRP = decltype(grp)::value, QW = decltype(qw)::value;
                 const int i = i0 + k;
+                SampleRow row{};
+                if constexpr (BOOK && DUP) row = bk_rows(i + 1);
                 R g;
                 if constexpr (QW) g = gz[k];
                 else if constexpr (MRG || LEAN) g = draw(i);
@@ -1289,10 +1338,16 @@ __device__ __forceinline__ void path_body(const LaunchParams& P, const int bid, 
                     // (a group of four steps lies in one window of 64)
                     if ((QW ? k == 0 : true) && (i & 63) == 0) fbits = sample_bits(i + 1);
                     if (((fbits >> (i & 63)) & 1u) && __builtin_amdgcn_ballot_w64(x > x_lo) != 0)
-                        observe(0, zone_spot(x));
+                        observe(0, zone_spot(x), SampleRow{});
+                } else if constexpr (BOOK && DUP) {
+                    // (a plain barrier sample changes nothing while every state
+                    // is under the zones)
+                    if ((row.bars | row.grps) != 0 || row.van_hi > row.van_lo)
+                        if (!(row.grps & kBookPlain) || __builtin_amdgcn_ballot_w64(x > bk_xlo) != 0)
+                            observe(0, state_spot(x, s0), row);
                 } else {
                     const int s = __builtin_amdgcn_readfirstlane((step_sample + i0 + 1)[k]);
-                    if (s >= 0) observe(s, DUP ? state_spot(x, s0) : x);
+                    if (s >= 0) observe(s, DUP ? state_spot(x, s0) : x, row_of(s, 0));
                 }
             };
             // FP32 Dupire adjoint kernels other than the book: groups of four steps
@@ -1360,9 +1415,11 @@ __device__ __forceinline__ void path_body(const LaunchParams& P, const int bid, 
                 // select, so the book's step is compiled once)
                 double* trow = tails + wave * TR;
                 double gb[4] = {0.0, 0.0, 0.0, 0.0};
-                for (; i < n4; ++i) {
+                double gs0 = 0.0, gs1 = 0.0, gs2 = 0.0;
+                uint32_t gl4 = 0;
+                for (; i < n; ++i) {
                     const int k = i & 3;
-                    if (k == 0) {
+                    if (k == 0 && i < n4) {
                         if constexpr (MRG) {
                             double pu[4];
 #pragma unroll
@@ -1378,11 +1435,33 @@ __device__ __forceinline__ void path_body(const LaunchParams& P, const int bid, 
                             inv_normal4_f64<TR, SPLIT>(gw, gb, trow, mtab, lane);
                         }
                     }
-                    gz[0] = k == 0 ? gb[0] : k == 1 ? gb[1] : k == 2 ? gb[2] : gb[3];
-                    fwd_step(i, 0, std::false_type{}, std::true_type{});
+                    if (i < n4) gz[0] = k == 0 ? gb[0] : k == 1 ? gb[1] : k == 2 ? gb[2] : gb[3];
+                    else gz[0] = draw(i);
+                    // (checkpoints: the four steps' states and brackets
+                    // gathered, stored with the last)
+                    glo = 0;
+                    fwd_step(i, 0, std::integral_constant<bool, IL>{}, std::true_type{});
+                    if constexpr (IL) {
+                        if (i < n4) {
+                            if (k == 0) gs0 = gx[0];
+                            if (k == 1) gs1 = gx[0];
+                            if (k == 2) gs2 = gx[0];
+                            gl4 = (gl4 >> 8) | (glo << 24);
+                            if (k == 3) {
+                                double2* c = reinterpret_cast<double2*>(ck + ck_el(i - 3));
+                                c[0] = make_double2(gs0, gs1);
+                                c[1] = make_double2(gs2, gx[0]);
+                                if (ck_lo) *reinterpret_cast<uint32_t*>(ckl + ck_el(i - 3)) = gl4;
+                            }
+                        } else {
+                            ck[i * kWave + lane] = gx[0];
+                            if (ck_lo) ckl[i * kWave + lane] = uint8_t(glo);
+                        }
+                    }
                 }
+            } else {
+                for (; i < n; ++i) fwd_step(i, 0, std::false_type{}, std::false_type{});
             }
-            for (; i < n; ++i) fwd_step(i, 0, std::false_type{}, std::false_type{});
 
             // ---- payoffs of the barrier (known at the end of the path)
             if constexpr (PRD == PRD_BARRIER) {
@@ -1426,7 +1505,7 @@ __device__ __forceinline__ void path_body(const LaunchParams& P, const int bid, 
 #pragma unroll
                 for (int b = 0; b < NBAR; ++b) {
                     stq[(8 + b) * kWave] = bst[b];
-                    stq[(8 + NBAR + b) * kWave] = babar[b];
+                    if constexpr (!ZT) stq[(8 + NBAR + b) * kWave] = babar[b];
                 }
 #pragma unroll
                 for (int g = 0; g < NGRP; ++g) {
@@ -1443,7 +1522,10 @@ __device__ __forceinline__ void path_body(const LaunchParams& P, const int bid, 
                 // intrinsic values (the numeraire adjoint)
 #pragma unroll
                 for (int b = 0; b < NBAR; ++b)
-                    if (b < P.bk.n_bar) babar[b] = R(wts[bk_bar_col[b]]) * babar[b];
+                    if (b < P.bk.n_bar) {
+                        if constexpr (ZT) bst[b] = R(wts[bk_bar_col[b]]) * bst[b];
+                        else babar[b] = R(wts[bk_bar_col[b]]) * babar[b];
+                    }
 #pragma unroll
                 for (int g = 0; g < NGRP; ++g) {
                     if (g >= P.bk.n_grp) continue;
@@ -1463,6 +1545,33 @@ __device__ __forceinline__ void path_body(const LaunchParams& P, const int bid, 
                 }
             }
 
+            // book: the spot above which barrier b has an adjoint on this
+            // lane, the lower end of its zone, or +infinity (breached, the
+            // vanilla out of the money or without weight).  Kept per barrier in
+            // a register (FP64 in float, under the zone by more than its
+            // rounding), so that a sample's test is one comparison: as masks
+            // they would spill from scalar registers.  rv_lo, rv_x: the lowest
+            // of them, as a spot and as a state.
+            float rth[NBAR];
+            R rv_lo = R(INFINITY), rv_x = R(INFINITY);
+            if constexpr (BOOK) {
+                float lo_min = INFINITY;
+#pragma unroll
+                for (int b = 0; b < NBAR; ++b) {
+                    const float lo = float(bk_four_c[b >> 2].lo[b & 3]);
+                    const float th = sizeof(R) == 4 ? lo : lo - 1e-6f * fabsf(lo);
+                    if constexpr (ZT) rth[b] = bst[b] != R(0) ? th : INFINITY;
+                    else rth[b] = bst[b] > R(0) && babar[b] != R(0) ? th : INFINITY;
+                    lo_min = fminf(lo_min, rth[b]);
+                }
+                rv_lo = R(lo_min);
+                if constexpr (DUP) {
+                    const R xl = sizeof(R) == 4 ? R(__logf(lo_min / float(s0))) : R(log(double(lo_min)));
+                    rv_x = lo_min > 0.0f ? xl - R(sizeof(R) == 4 ? 1e-4 : 1e-10) * (R(1) + fabs(xl)) : R(-INFINITY);
+                    if (!(lo_min < INFINITY)) rv_x = R(INFINITY);
+                }
+            }
+
             // adjoints of the forward, numeraire and discount at sample s
             const R w0 = R(wts[0]);
             const R w1 = npay > 1 ? R(wts[1]) : R(0);
@@ -1472,7 +1581,8 @@ __device__ __forceinline__ void path_body(const LaunchParams& P, const int bid, 
             // at_last: s is the last sample (the last timeline point); the
             // sweeps pass a constant false inside their step loops
             // Fz: the spot the forward took the barrier's smoothing factor at
-            auto sample_adj = [&](int s, R F, R Fz, R numv, R discv, R& Fb, R& nb, R& db, bool at_last) {
+            // sm: the book's row of the sample
+            auto sample_adj = [&](int s, SampleRow sm, R F, R Fz, R numv, R discv, R& Fb, R& nb, R& db, bool at_last) {
                 Fb = R(0); nb = R(0); db = R(0);
                 if constexpr (PRD == PRD_BARRIER) {
                     // d alive / dF = -(product of the other factors) / 2w: alive / f
@@ -1498,7 +1608,6 @@ __device__ __forceinline__ void path_body(const LaunchParams& P, const int bid, 
                     db = w0 * intrinsic / numv;
                     nb = -w0 * intrinsic * discv / (numv * numv);
                 } else if constexpr (PRD == PRD_BOOK) {
-                    const SampleRow sm = bk_rows(s);
                     for (int k = sm.van_lo; k < sm.van_hi; ++k) {
                         const R kk = R(bk_van_strike[k]);
                         const R wk = R(wts[bk_van_col[k]]);
@@ -1507,10 +1616,34 @@ __device__ __forceinline__ void path_body(const LaunchParams& P, const int bid, 
                             nb += -wk * (F - kk) / (numv * numv);
                         }
                     }
-                    // no lane at or above the lowest zone: no survival adjoint
-                    const uint32_t bm0 = sm.bars & 0xffffu, bl = sm.bars >> 16;
-                    const uint32_t bm = bm0 && __any(F > bk_lo) ? bm0 : 0u;
-                    if (bm | bl) {
+                    // d alive / dF = -(product of the other factors) / 2w: the
+                    // state over the factor without a zero factor; with one,
+                    // its product for the zero factor and 0 for the others
+                    auto zone_adj = [&](int b, R up, R i2s) {
+                        const R v = bst[b];
+                        if constexpr (ZT) {
+                            // v: the weighted vanilla times the state
+                            const R d = up - F;
+                            R a = recip_mul(v, d);
+                            const bool one = fabs(v) > R(kZeroMark);
+                            if (__builtin_amdgcn_ballot_w64(one) != 0) {
+                                asm volatile("");   // (rare: a branch of its own)
+                                if (one) a = d == R(0) ? v * R(1.0 / kZeroScale) * i2s : R(0);
+                            }
+                            Fb -= a;
+                        } else {
+                            // FP32 (factors at least 1e-30)
+                            const R f = max((up - F) * i2s, R(1e-30));
+                            Fb -= babar[b] * i2s * recip_mul(v, f);
+                        }
+                    };
+                    const uint32_t bm = sm.bars & 0xffffu;
+                    uint32_t bl = sm.bars >> 16;
+                    const float Ff = float(F);
+                    if (bl) {
+                        // (opaque: the tests of the mask's bits stay here,
+                        // where some barrier matures)
+                        asm volatile("" : "+s"(bl));
 #pragma unroll
                         for (int b = 0; b < NBAR; ++b) {
                             if (!(((bm | bl) >> b) & 1u)) continue;
@@ -1522,31 +1655,33 @@ __device__ __forceinline__ void path_body(const LaunchParams& P, const int bid, 
                                 const R intrinsic = put ? (k - F > R(0) ? k - F : R(0))
                                                         : (F - k > R(0) ? F - k : R(0));
                                 const R dmax = put ? (k > F ? R(-1) : R(0)) : (F > k ? R(1) : R(0));
-                                const R alive = bst[b] > R(0) ? bst[b] : R(0);
-                                const R euro_bar = R(wts[col]) * alive + R(wts[col + 1]);
+                                // weight x survival factor (FP64: from the
+                                // weighted vanilla times the state, where the
+                                // vanilla is 0 it does not matter)
+                                R wa;
+                                if constexpr (ZT) {
+                                    const R euro = intrinsic / numv;
+                                    wa = euro != R(0) && !(fabs(bst[b]) > R(kZeroMark)) ? bst[b] / euro : R(0);
+                                } else {
+                                    wa = R(wts[col]) * bar_alive(bst[b]);
+                                }
+                                const R euro_bar = wa + R(wts[col + 1]);
                                 Fb += euro_bar * dmax / numv;
                                 nb += -euro_bar * (intrinsic / numv) / numv;
                             }
-                            if ((bm >> b) & 1u) {
-                                // d alive / dF = -(product of the other factors) / 2w
-                                const R v = bst[b];
-                                if constexpr (ZT) {
-                                    if (v > R(kBreached) && F > bp.lo) {   // smoothing zone
-                                        const R i2s = bp.i2s;
-                                        const R f = (bp.up - F) * i2s;
-                                        // product of the other factors: v / f without a zero
-                                        // factor, the non-zero ones for the only zero factor
-                                        // (v >= 0 with f == 0 only after the product underflowed
-                                        // to zero: the other factors' product is 0)
-                                        const R others = v >= R(0) ? (f != R(0) ? recip_mul(v, f) : R(0))
-                                                                   : ((v >= R(-1) && f == R(0)) ? -v : R(0));
-                                        Fb -= babar[b] * others * i2s;
-                                    }
-                                } else if (v > R(kBreached) && F > bp.lo) {
-                                    // FP32 (factors at least 1e-30): the others' product
-                                    // is v / f (a wave with no lane in the zone skips it)
-                                    const R f = max((bp.up - F) * bp.i2s, R(1e-30));
-                                    Fb -= babar[b] * bp.i2s * recip_mul(v, f);
+                            if (Ff > rth[b] && F > bp.lo && ((bm >> b) & 1u)) zone_adj(b, bp.up, bp.i2s);
+                        }
+                    } else if (bm && __builtin_amdgcn_ballot_w64(F > rv_lo) != 0) {
+                        // some lane is above the lowest zone that its path
+                        // has an adjoint in (one sample in three of the
+                        // 55-payoff book); then few barriers have one
+#pragma unroll
+                        for (int b = 0; b < NBAR; ++b) {
+                            if (Ff > rth[b]) {
+                                if ((bm >> b) & 1u) {
+                                    const R lo = bk_four_c[b >> 2].lo[b & 3];
+                                    if (sizeof(R) == 4 || F > lo)
+                                        zone_adj(b, bk_four_c[b >> 2].up[b & 3], bk_four_c[b >> 2].i2s[b & 3]);
                                 }
                             }
                         }
@@ -1602,7 +1737,7 @@ __device__ __forceinline__ void path_body(const LaunchParams& P, const int bid, 
                     if (s >= 0) {
                         const R S = state_spot(x, s0);
                         R Fb, nb, db;
-                        sample_adj(s, S, zone_spot(x), R(1), R(1), Fb, nb, db, true);   // step_sample[n] is the last sample
+                        sample_adj(s, row_of(s, n), S, zone_spot(x), R(1), R(1), Fb, nb, db, true);   // step_sample[n] is the last sample
                         abar = S * Fb;
                     }
                 }
@@ -1677,10 +1812,13 @@ __device__ __forceinline__ void path_body(const LaunchParams& P, const int bid, 
                             if (smp >= 0 && __builtin_amdgcn_ballot_w64(xi > x_lo) != 0)
                                 cb[k] = barrier_sf(zone_spot(xi));
                         } else if (smp >= 0) {
-                            const R S = state_spot(xi, s0);
-                            R Fb, nb, db;
-                            sample_adj(smp, S, S, R(1), R(1), Fb, nb, db, false);
-                            cb[k] = S * Fb;
+                            const SampleRow row = row_of(smp, i);
+                            if (!(row.grps & kBookPlain) || __builtin_amdgcn_ballot_w64(xi > rv_x) != 0) {
+                                const R S = state_spot(xi, s0);
+                                R Fb, nb, db;
+                                sample_adj(smp, row, S, S, R(1), R(1), Fb, nb, db, false);
+                                cb[k] = S * Fb;
+                            }
                         }
                         xi = euler_step(xi, b.vol, g);
                     }
@@ -1705,7 +1843,7 @@ __device__ __forceinline__ void path_body(const LaunchParams& P, const int bid, 
                     if (s >= 0) {
                         const R S = state_spot(x, s0);
                         R Fb, nb, db;
-                        sample_adj(s, S, zone_spot(x), R(1), R(1), Fb, nb, db, true);   // step_sample[n] is the last sample
+                        sample_adj(s, row_of(s, n), S, zone_spot(x), R(1), R(1), Fb, nb, db, true);   // step_sample[n] is the last sample
                         abar = S * Fb;
                     }
                 }
@@ -1716,7 +1854,7 @@ __device__ __forceinline__ void path_body(const LaunchParams& P, const int bid, 
                 const R vmin = R(sizeof(R) == 8 ? kRecoverVolF64 : kRecoverVolF32);
                 // groups of U steps, top down to top - U + 1; the checkpoint
                 // loads of the next group are issued before the current group
-                // is worked (the book holds more registers: U = 1; FP64 below).
+                // is worked (the book, with more registers: U = 1; FP64 below).
                 // FP32 groups of four are the aligned groups of the interleaved
                 // checkpoints (steps 4g .. 4g + 3), one 16-byte load of states
                 // and one word of brackets each; the top group may be partial
@@ -1728,6 +1866,7 @@ __device__ __forceinline__ void path_body(const LaunchParams& P, const int bid, 
                 static_assert(U <= kCkptGuardRows, "the prefetch reads at most kCkptGuardRows rows below 0");
                 R buf[U];
                 int lbuf[U];
+                SampleRow prow{};       // book: the row of the group's step, read a step ahead
                 int rwin = -1;          // UNDER: window of 64 points held in rbits
                 uint64_t rbits = 0;
                 // states and brackets of steps top, top - 1, ..., top - U + 1
@@ -1753,6 +1892,8 @@ __device__ __forceinline__ void path_body(const LaunchParams& P, const int bid, 
                     R nbuf[U];
                     int nlbuf[U];
                     load_group(top - U, nbuf, nlbuf);
+                    SampleRow nrow{};
+                    if constexpr (BOOK) nrow = bk_rows(max(top - 1, 0));
                     // phase 1, independent of the adjoint chain: brackets, the
                     // derivative of each step to its vol, the sample adjoints
                     R ws[U], sl[U], wa[U], wb[U], sf[U];
@@ -1775,7 +1916,7 @@ __device__ __forceinline__ void path_body(const LaunchParams& P, const int bid, 
                         smps[2] = v.y;
                         smps[3] = v.x;
                     } else {
-                        smps[0] = step_sample[top];
+                        smps[0] = BOOK ? 0 : step_sample[top];
                     }
 #pragma unroll
                     for (int k = 0; k < U; ++k) {
@@ -1807,10 +1948,12 @@ __device__ __forceinline__ void path_body(const LaunchParams& P, const int bid, 
                             if (smp >= 0 && __builtin_amdgcn_ballot_w64(xi > x_lo) != 0)
                                 sf[k] = barrier_sf(zone_spot(xi));
                         } else {
-                            if (smp >= 0) {
+                            const SampleRow row = BOOK ? prow : SampleRow{};
+                            const bool on = BOOK ? (row.bars | row.grps) != 0 || row.van_hi > row.van_lo : smp >= 0;
+                            if (on && (!(row.grps & kBookPlain) || __builtin_amdgcn_ballot_w64(xi > rv_x) != 0)) {
                                 const R S = state_spot(xi, s0);
                                 R Fb, nb, db;
-                                sample_adj(smp, S, S, R(1), R(1), Fb, nb, db, false);
+                                sample_adj(smp, row, S, S, R(1), R(1), Fb, nb, db, false);
                                 sf[k] = S * Fb;
                             }
                         }
@@ -1838,6 +1981,7 @@ __device__ __forceinline__ void path_body(const LaunchParams& P, const int bid, 
                     }
 #pragma unroll
                     for (int k = 0; k < U; ++k) { buf[k] = nbuf[k]; lbuf[k] = nlbuf[k]; }
+                    prow = nrow;
                 };
                 if constexpr (IL && sizeof(R) == 8) {
                     // FP64: the steps run one by one, their checkpoints loaded
@@ -1859,22 +2003,26 @@ __device__ __forceinline__ void path_body(const LaunchParams& P, const int bid, 
                                 }
                                 smp = int(((rbits >> (i & 63)) & 1u)) - 1;
                             } else {
-                                smp = __builtin_amdgcn_readfirstlane(step_sample[i]);
+                                smp = BOOK ? 0 : __builtin_amdgcn_readfirstlane(step_sample[i]);
                             }
+                            // (book: the row read a step ahead)
+                            const SampleRow row = prow;
+                            if constexpr (BOOK) prow = bk_rows(max(i - 1, 0));
+                            const bool on = BOOK ? (row.bars | row.grps) != 0 || row.van_hi > row.van_lo : smp >= 0;
                             if (!ck_lo) lo = count_le<LEAN>(ks, xi);
                             const Bracket<R> b = local_vol_at(kxi, iv + i * mp, xi, lo);
                             R ws = recip_mul(xnext - xi, b.vol) - R(0.5) * b.vol;
                             if constexpr (!REC)
-                                if (__builtin_amdgcn_ballot_w64(b.vol < vmin) != 0)
+                                if (!iv_recover && __builtin_amdgcn_ballot_w64(b.vol < vmin) != 0)
                                     if (b.vol < vmin) ws = draw(i) - b.vol;
                             R sf = R(0);
                             if constexpr (UNDER) {
                                 if (smp >= 0 && __builtin_amdgcn_ballot_w64(xi > x_lo) != 0)
                                     sf = barrier_sf(zone_spot(xi));
-                            } else if (smp >= 0) {
+                            } else if (on && (!(row.grps & kBookPlain) || __builtin_amdgcn_ballot_w64(xi > rv_x) != 0)) {
                                 const R S = state_spot(xi, s0);
                                 R Fb, nb, db;
-                                sample_adj(smp, S, S, R(1), R(1), Fb, nb, db, false);
+                                sample_adj(smp, row, S, S, R(1), R(1), Fb, nb, db, false);
                                 sf = S * Fb;
                             }
                             const R vb = abar * ws;
@@ -1887,24 +2035,24 @@ __device__ __forceinline__ void path_body(const LaunchParams& P, const int bid, 
                             }
                             xnext = xi;
                         };
+                        double2 c0, c1;
+                        uint32_t cw;
+                        auto load4 = [&](int g) {   // (below step 0: the slot's guard rows, never used)
+                            const int e = (g << 8) + (lane << 2);
+                            const double2* c = reinterpret_cast<const double2*>(ck + e);
+                            c0 = c[0];
+                            c1 = c[1];
+                            cw = ck_lo ? *reinterpret_cast<const uint32_t*>(ckl + e) : 0u;
+                        };
                         auto sweep = [&](auto recover) {
                             int top = last;
                             for (; top >= n4; --top) step(top, ck[ck_el(top)], ck_lo ? int(ckl[ck_el(top)]) : 0, recover);
                             if (top < 0) return;
-                            double2 c0, c1;
-                            uint32_t cw;
-                            auto load4 = [&](int g) {
-                                const int e = (g << 8) + (lane << 2);
-                                const double2* c = reinterpret_cast<const double2*>(ck + e);
-                                c0 = c[0];
-                                c1 = c[1];
-                                cw = ck_lo ? *reinterpret_cast<const uint32_t*>(ckl + e) : 0u;
-                            };
                             load4(top >> 2);
                             for (int g = top >> 2; g >= 0; --g) {
                                 const double2 a0 = c0, a1 = c1;
                                 const uint32_t w = cw;
-                                load4(g - 1);   // (the slot's guard rows below step 0, never used)
+                                load4(g - 1);
                                 const int i = g << 2;
                                 if (i + 3 <= top) step(i + 3, a1.y, int(w >> 24), recover);
                                 if (i + 2 <= top) step(i + 2, a1.x, int((w >> 16) & 0xffu), recover);
@@ -1912,6 +2060,34 @@ __device__ __forceinline__ void path_body(const LaunchParams& P, const int bid, 
                                 step(i, a0.x, int(w & 0xffu), recover);
                             }
                         };
+                        if constexpr (BOOK) {
+                            // the book's step is compiled once: steps from
+                            // n4 on read their row, the others a group of
+                            // four loaded a group ahead
+                            prow = bk_rows(last);
+                            load4(min(last, n4 - 1) >> 2);
+                            double2 a0 = c0, a1 = c1;
+                            uint32_t w = cw;
+                            for (int i = last; i >= 0; --i) {
+                                const int k = i & 3;
+                                R xi;
+                                int lo;
+                                if (i >= n4) {
+                                    xi = ck[i * kWave + lane];
+                                    lo = ck_lo ? int(ckl[i * kWave + lane]) : 0;
+                                } else {
+                                    if (k == 3 || i == last) {
+                                        a0 = c0;
+                                        a1 = c1;
+                                        w = cw;
+                                        load4((i >> 2) - 1);
+                                    }
+                                    xi = k == 3 ? a1.y : k == 2 ? a1.x : k == 1 ? a0.y : a0.x;
+                                    lo = int((w >> (8 * k)) & 0xffu);
+                                }
+                                step(i, xi, lo, std::false_type{});
+                            }
+                        } else
                         if (iv_recover) sweep(std::true_type{}); else sweep(std::false_type{});
                     }
                 } else if (n > 0) {
@@ -1922,6 +2098,7 @@ __device__ __forceinline__ void path_body(const LaunchParams& P, const int bid, 
                     int top = VG ? ((last >> 2) << 2) + 3 : last;
                     if (top + 1 < n) xnext = ck[ck_el(top + 1)];
                     load_group(top, buf, lbuf);
+                    if constexpr (BOOK) prow = bk_rows(top);
                     if (VG && top >= n) {
                         group(top, std::true_type{});
                         top -= U;
@@ -1946,7 +2123,7 @@ __device__ __forceinline__ void path_body(const LaunchParams& P, const int bid, 
                     const R numv = P.spot_measure ? R(s_num[s]) * S : R(s_num[s]);
                     const R discv = R(s_disc[s]);
                     R Fb, nb, db;
-                    sample_adj(s, F, F, numv, discv, Fb, nb, db, s == last);
+                    sample_adj(s, row_of(s, 0), F, F, numv, discv, Fb, nb, db, s == last);
                     // dF = F (tau + dff/ff), ff = exp(mu (Tf - t))
                     const R tfs = R(tf[s]), tds = R(td[s]), ts = R(tl[s]);
                     R dF[4] = {F * tau[0], F * tau[1], F * (tau[2] + tfs), F * (tau[3] - tfs)};
