@@ -26,7 +26,8 @@ SOURCES = ([("cf_kern_inst.hip", "cf_kern_r%d_a%d_b%d" % (r, a, b),
             for r in (0, 1) for a in (0, 1, 2)] +
 
            [(s, os.path.splitext(s)[0], []) for s in ("cf_kernels.hip", "cf_engine.cpp", "cf_store.cpp",
-                                                      "cf_server.cpp", "cf_calib.cpp", "cf_noalloc.hip")])
+                                                      "cf_server.cpp", "cf_calib.cpp", "cf_noalloc.hip",
+                                                      "cf_itemized.hip")])
 
 # Packed FP32 instructions are disabled for all device code.  Multiply-adds
 # are fused only within one source expression (-ffp-contract=on), so every

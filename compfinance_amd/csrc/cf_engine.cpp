@@ -1520,6 +1520,207 @@ static vector<int> payoff_last_points(const Prepared& PR)
     return pts;
 }
 
+// The maturities' calls in order of strike, and the time interpolation of the
+// steps, as the itemized kernels read them.
+struct ItemTables {
+    Staging st;
+    size_t first, points, strikes, out_col, col_point, order, t_lo, t_hi, tj0, tj1, tw0, tw1, sqrtdt;
+    int most = 0;   // calls of one maturity at most
+    explicit ItemTables(const Prepared& PR)
+    {
+        const ProductPlan& pd = PR.pd;
+        const ModelPlan& md = PR.md;
+        const int ns = int(pd.timeline.size()), nc = pd.n_pay;
+        vector<int> pts(static_cast<size_t>(ns), 0), oc(static_cast<size_t>(nc)), cp(static_cast<size_t>(nc)), ord(static_cast<size_t>(nc));
+        for (int i = 0; i <= md.n_steps; ++i)
+            if (md.step_sample[size_t(i)] >= 0) pts[size_t(md.step_sample[size_t(i)])] = i;
+        vector<double> k(static_cast<size_t>(nc));
+        for (int s = 0; s < ns; ++s) {
+            const int lo = pd.pay_first[size_t(s)], hi = pd.pay_first[size_t(s) + 1];
+            most = std::max(most, hi - lo);
+            for (int c = lo; c < hi; ++c) oc[size_t(c)] = c;
+            std::stable_sort(oc.begin() + lo, oc.begin() + hi,
+                             [&](int x, int y) { return pd.pay_strike[size_t(x)] < pd.pay_strike[size_t(y)]; });
+            for (int c = lo; c < hi; ++c) {
+                k[size_t(c)] = pd.pay_strike[size_t(oc[size_t(c)])];
+                cp[size_t(c)] = pts[size_t(s)];
+            }
+        }
+        for (int c = 0; c < nc; ++c) ord[size_t(c)] = c;
+        std::stable_sort(ord.begin(), ord.end(), [&](int x, int y) { return cp[size_t(x)] > cp[size_t(y)]; });
+        const size_t n = size_t(md.n_steps), nT = size_t(md.n_times);
+        vector<int> j0(n), j1(n), tl(nT, 0), th(nT, 0);
+        vector<double> w0(n), w1(n);
+        for (size_t i = 0; i < n; ++i) {
+            j0[i] = PR.tw[i].j0;
+            j1[i] = PR.tw[i].j1;
+            w0[i] = PR.tw[i].w0;
+            w1[i] = PR.tw[i].w1;
+            for (int j : {j0[i], j1[i]}) {
+                if (th[size_t(j)] == 0) tl[size_t(j)] = int(i);
+                th[size_t(j)] = int(i) + 1;
+            }
+        }
+        first = st.add(pd.pay_first);
+        points = st.add(pts);
+        strikes = st.add(k);
+        out_col = st.add(oc);
+        col_point = st.add(cp);
+        order = st.add(ord);
+        t_lo = st.add(tl);
+        t_hi = st.add(th);
+        tj0 = st.add(j0);
+        tj1 = st.add(j1);
+        tw0 = st.add(w0);
+        tw1 = st.add(w1);
+        sqrtdt = st.add(PR.sqrtdt);
+    }
+};
+
+// Itemized risk of a Europeans product on Dupire: the calls of a maturity
+// share their sweeps (cf_itemized.hip).  The caller holds the engine's lock.
+// Returns false, doing nothing, where its kernels do not apply: grids of more
+// knots than a bracket byte counts, local vols below the recovery threshold
+// (the sweep would draw normals again), more calls of one maturity than the
+// listing kernel counts, a grid over the LDS, or too little device memory; the
+// caller then sweeps once per payoff.
+static bool run_multi_europeans(Engine& E, const Prepared& PR, const CallShape& S, const cf_num* num,
+                                double* payoff_means, double* risks)
+{
+    const ModelPlan& md = PR.md;
+    if (md.kind != CF_MODEL_DUPIRE || PR.pd.kind != CF_PRODUCT_EUROPEANS || S.npay < 2) return false;
+    if (!PR.iv_recover || md.n_spots > cfk::kMaxStoredKnots) return false;
+    const ItemTables T(PR);
+    if (T.most > cfk::kMaxItemStrikes) return false;
+    const int rb = S.fp64 ? 8 : 4;
+    // the local-vol table in LDS beside a grid, else through L1; a block takes
+    // the whole LDS of its compute unit for copies of its grid
+    bool giv = false;
+    auto lds = [&] { return cfk::item_smem(md.n_steps, md.n_spots, 16, rb, giv).total; };
+    if (lds() > size_t(E.max_lds)) giv = true;
+    if (lds() > size_t(E.max_lds)) return false;
+    cfk::ItemParams I;
+    std::memset(&I, 0, sizeof I);
+    // up to 64 blocks a list, of at least one pass of 1024 paths
+    const int64_t passes = (S.n_path + 1023) / 1024, per = (passes + 63) / 64;
+    if (S.n_path > int64_t(1) << 30) return false;
+    I.per_block = int(per * 1024);
+    I.chunks = int((S.n_path + I.per_block - 1) / I.per_block);
+    I.n_cols = S.npay;
+    const int64_t q0 = (S.first + 1) >> 6, q1 = (S.first + S.n_path) >> 6;
+    const size_t blocks64 = size_t(q1 - q0 + 1 - (S.merge ? 1 : 0));
+    const int state_rows = cfk::state_rows(false);
+    const size_t npar = 1 + size_t(md.n_spots) * size_t(md.n_times);
+    size_t total = 0;
+    auto part = [&total](size_t bytes) {
+        const size_t o = total;
+        total += al256(bytes);
+        return o;
+    };
+    const size_t o_ck = part(blocks64 * size_t(S.ck_rows) * cfk::kWave * size_t(rb));
+    const size_t o_st = part(blocks64 * size_t(state_rows) * cfk::kWave * size_t(rb));
+    const size_t o_ids = part(size_t(I.n_cols) * size_t(S.n_path) * 4);
+    const size_t o_cnt = part(size_t(I.n_cols) * 4);
+    const size_t o_grid = part(size_t(I.n_cols) * S.ivn * 8);
+    const size_t o_del = part(size_t(I.n_cols) * 8);
+    const size_t o_risk = part(npar * size_t(I.n_cols) * 8);
+
+    struct Owned : DevBuf {
+        ~Owned() { if (p) (void)hipFree(p); }
+    } once;
+    DevBuf& buf = total <= Engine::kItemKeep ? E.item : static_cast<DevBuf&>(once);
+    if (total > buf.cap) {
+        E.item.give_back();
+        size_t free_b = 0, total_b = 0;
+        hip_check(hipMemGetInfo(&free_b, &total_b), "hipMemGetInfo");
+        if (total + (size_t(256) << 20) > free_b) return false;
+    }
+    unsigned char* d = static_cast<unsigned char*>(buf.ensure(total));
+    DevBuf& tab = const_cast<Prepared&>(PR).item;   // (under the engine's lock)
+    if (!tab.p) {
+        tab.ensure(T.st.bytes.size());
+        hip_check(hipMemcpy(tab.p, T.st.bytes.data(), T.st.bytes.size(), hipMemcpyHostToDevice), "table upload");
+    }
+    const unsigned char* dt = static_cast<const unsigned char*>(tab.p);
+
+    // the forward: payoff means, checkpoints and end states
+    const CallBytes nb = call_bytes(S);
+    double* h_out = static_cast<double*>(E.pin_out.ensure((size_t(S.stride) + S.ivn) * 8));
+    double* h_in = static_cast<double*>(E.pin_in.ensure(size_t(S.npay) * 8));
+    CallBuffers B;
+    B.tables = static_cast<const unsigned char*>(PR.tables.p);
+    B.block_out = static_cast<double*>(E.block_out.ensure(nb.block_out));
+    B.reduced = static_cast<double*>(E.pin_out.dev);
+    B.weights = static_cast<double*>(E.weights.ensure(nb.weights));
+    B.ckpt = d + o_ck;
+    E.weights_on_device = nullptr;   // this call rewrites the weights buffer
+    std::fill(h_in, h_in + S.npay, 0.0);
+    hip_check(hipMemcpyAsync(B.weights, h_in, size_t(S.npay) * 8, hipMemcpyHostToDevice, E.stream), "upload");
+    cfk::LaunchParams P = launch_params(E, PR, S, B);
+    P.state = d + o_st;
+    P.ck_mode = 1;
+    Sequence q;
+    CallShape S_fwd = S;
+    S_fwd.ivn = 0;   // (no adjoint grids to sum)
+    E.ivbar_blocks.ensure(nb.ivbar_blocks);
+    P.ivbar_blocks = static_cast<double*>(E.ivbar_blocks.p);
+    make_sequence(PR, S_fwd, B, P, &q);
+    q.cfg.item = true;
+    ready_sequence(q);
+    enqueue_sequence(q, E.stream, nullptr, nullptr);
+
+    I.first_path = S.first;
+    I.n_path = S.n_path;
+    I.merge_tail = S.merge ? 1 : 0;
+    I.n_steps = md.n_steps;
+    I.n_spots = md.n_spots;
+    I.n_times = md.n_times;
+    I.spot = md.spot;
+    I.ckpt = d + o_ck;
+    I.state = d + o_st;
+    I.ck_rows = S.ck_rows;
+    I.state_rows = state_rows;
+    I.knots = P.knots;
+    I.inv_dx = P.inv_dx;
+    I.iv = P.iv;
+    auto ti = [dt](size_t o) { return reinterpret_cast<const int*>(dt + o); };
+    auto td = [dt](size_t o) { return reinterpret_cast<const double*>(dt + o); };
+    I.first = ti(T.first);
+    I.points = ti(T.points);
+    I.strikes = td(T.strikes);
+    I.out_col = ti(T.out_col);
+    I.col_point = ti(T.col_point);
+    I.order = ti(T.order);
+    I.t_lo = ti(T.t_lo);
+    I.t_hi = ti(T.t_hi);
+    I.tj0 = ti(T.tj0);
+    I.tj1 = ti(T.tj1);
+    I.tw0 = td(T.tw0);
+    I.tw1 = td(T.tw1);
+    I.sqrtdt = td(T.sqrtdt);
+    I.counts = reinterpret_cast<uint32_t*>(d + o_cnt);
+    I.ids = reinterpret_cast<uint32_t*>(d + o_ids);
+    I.lds = E.max_lds;
+    I.grids = reinterpret_cast<double*>(d + o_grid);
+    I.deltas = reinterpret_cast<double*>(d + o_del);
+    I.risks = reinterpret_cast<double*>(d + o_risk);
+    const int rc = cfk::launch_item_reverse(I, int(PR.pd.timeline.size()), rb, giv, E.stream);
+    if (rc != 0) hip_check(hipError_t(rc), "itemized reverse launch");
+    // (large ladders go straight to the caller's memory)
+    const size_t rbytes = npar * size_t(I.n_cols) * 8;
+    const bool pinned = rbytes <= (size_t(16) << 20);
+    double* h_risk = pinned ? static_cast<double*>(E.pin_item.ensure(rbytes)) : risks;
+    hip_check(hipMemcpyAsync(h_risk, I.risks, rbytes, hipMemcpyDeviceToHost, E.stream), "download");
+    hip_check(hipStreamSynchronize(E.stream), "kernel execution");
+    if (pinned) std::memcpy(risks, h_risk, rbytes);
+    S_fwd.adjoint = false;
+    Call c;
+    c.num = num;
+    c.means = payoff_means;
+    collect_results(PR, S_fwd, h_out, h_out + S.stride, c);
+    return true;
+}
+
 // Itemized risk over shared paths (the reference's single sweep with vector
 // adjoints, mcBase.h:858-989): one forward-only launch keeps every block of 64
 // paths' checkpoints and end states, then one reverse-only launch per payoff
@@ -1535,6 +1736,8 @@ bool run_multi(const cf_model* mdl, const cf_product* prd, const cf_num* num, do
         lookup(E, mdl, prd, fp64, cfk::ADJ_CHECKPOINT, true, call_block(E, num, fp64));
     const Prepared& PR = *PP;
     const CallShape S = shape_call(E, PR, num, true);
+    if (run_multi_europeans(E, PR, S, num, payoff_means, risks)) return true;
+    E.item.give_back();
     const CallBytes nb = call_bytes(S);
     const int64_t q0 = (S.first + 1) >> 6, q1 = (S.first + S.n_path) >> 6;
     const size_t blocks64 = size_t(q1 - q0 + 1 - (S.merge ? 1 : 0));

@@ -148,6 +148,12 @@ struct DevBuf {
         cap = want;
         return p;
     }
+    void give_back()
+    {
+        if (p) (void)hipFree(p);
+        p = nullptr;
+        cap = 0;
+    }
 };
 
 // Grow-only pinned host buffer (uploads and downloads without staging copies).
@@ -211,9 +217,11 @@ struct Prepared {
     // interpolation weights of each step
     vector<double> sqrtdt;
     vector<Interp1> tw;
+    DevBuf item;   // tables of the itemized risk of Europeans, uploaded by the first such call
     ~Prepared()
     {
         if (tables.p) (void)hipFree(tables.p);
+        if (item.p) (void)hipFree(item.p);
     }
 };
 
@@ -228,6 +236,12 @@ struct Engine {
     uint32_t* d_dirs = nullptr;
     DevBuf block_out, ivbar_blocks, reduced, per_path, per_path_agg, ckpt, weights;
     PinnedBuf pin_in, pin_out;
+    // itemized risk: checkpoints, lists and grids of one call, kept between
+    // calls up to kItemKeep bytes and given back by an itemized call that
+    // takes buffers of its own, and the risks' download
+    static constexpr size_t kItemKeep = size_t(256) << 20;
+    DevBuf item;
+    PinnedBuf pin_item;
     // the aggregation weights last uploaded to `weights` (skipped when a call repeats them)
     vector<double> weights_last;
     const void* weights_on_device = nullptr;

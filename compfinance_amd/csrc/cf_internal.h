@@ -461,6 +461,71 @@ CF_HD inline SmemLayout smem_layout(int n_steps, int n_spots, int n_samples, int
     return L;
 }
 
+// ---- itemized risk of a Europeans product on Dupire (cf_itemized.hip)
+
+// Calls of one maturity at most (LDS counters of the listing kernel).
+constexpr int kMaxItemStrikes = 64;
+// Copies of a reverse block's grid at most.
+constexpr int kMaxItemCopies = 8;
+
+// The calls are numbered by maturity, then by strike ("columns" c; out_col maps
+// them to the payoff columns).  Column c's list holds the paths whose spot at
+// the maturity passes exactly the strikes up to its own.
+struct ItemParams {
+    int64_t first_path, n_path;
+    int merge_tail;
+    int n_steps, n_spots, n_times, n_cols;
+    double spot;
+    const void* ckpt;            // the forward-only launch's checkpoints, one slot per block of 64 paths
+    const void* state;           // and end states
+    int ck_rows, state_rows;
+    const void* knots;           // as in LaunchParams
+    const void* inv_dx;
+    const void* iv;
+    const int* first;            // [n_samples + 1] columns of each maturity
+    const int* points;           // [n_samples] its timeline point
+    const double* strikes;       // [n_cols]
+    const int* out_col;          // [n_cols]
+    const int* col_point;        // [n_cols] timeline point of the column's maturity
+    const int* order;            // [n_cols] columns by falling timeline point
+    // steps [t_lo, t_hi) interpolate local-vol time t; per step the two times and weights
+    const int* t_lo;
+    const int* t_hi;
+    const int* tj0;
+    const int* tj1;
+    const double* tw0;
+    const double* tw1;
+    const double* sqrtdt;
+    uint32_t* counts;            // [n_cols] lengths of the lists
+    uint32_t* ids;               // [n_cols][n_path] the lists
+    int chunks, per_block;       // a list is swept by up to `chunks` blocks of per_block paths
+    int lds;                     // LDS bytes of a reverse block
+    double* grids;               // [n_cols][n_steps][n_spots] sums of the lists
+    double* deltas;              // [n_cols]
+    double* risks;               // [1 + n_spots n_times][n_cols]
+};
+
+// LDS of a reverse block that sweeps n_steps steps; `total` with one grid, more
+// copies follow the first.
+struct ItemSmem {
+    size_t knots, iv, acc, grid, total;
+};
+CF_HD inline ItemSmem item_smem(int n_steps, int n_spots, int waves, int real_bytes, bool giv)
+{
+    ItemSmem L{};
+    size_t o = 0;
+    L.knots = o; o = cf_align16(o + size_t(2 * (n_spots + 1)) * real_bytes);
+    L.iv = o;    o = cf_align16(o + (giv ? 0 : size_t(n_steps) * lv_cols(n_spots) * real_bytes));
+    L.acc = o;   o = cf_align16(o + size_t(waves) * 8);
+    L.grid = o;  o = cf_align16(o + size_t(ivbar_copy_stride(n_steps, n_spots)) * 8);
+    L.total = o;
+    return L;
+}
+
+// The listing, the sweeps and the mapping, after the forward-only launch;
+// giv: the local-vol table through L1 (it and the grids exceed LDS).
+int launch_item_reverse(const ItemParams& P, int n_samples, int real_bytes, bool giv, void* stream);
+
 // Host-side launch entry points, defined in cf_kernels.hip.
 struct KernelConfig {
     int precision;   // 0 = FP64, 1 = FP32
