@@ -1244,9 +1244,9 @@ __device__ __forceinline__ void path_body(const LaunchParams& P, const int bid, 
             if constexpr (BOOK) return bk_rows(DUP ? i : s);
             else return SampleRow{};
         };
-        // Dupire barrier: a sample other than the last one changes nothing
-        // while the spot is under the smoothing zone, so the spot is not
-        // formed there (forward and reverse)
+        // Dupire barrier: a sample other than the last one changes nothing on
+        // a path that is under the smoothing zone or breached, so the spot is
+        // not formed where all the wave's paths are (forward and reverse)
         constexpr bool UNDER = DUP && PRD == PRD_BARRIER;
         const R x_lo = UNDER ? R(P.bar_xlo) : R(0);
         auto zone_spot = [&](R x) -> R {
@@ -1337,7 +1337,7 @@ __device__ __forceinline__ void path_body(const LaunchParams& P, const int bid, 
                 if constexpr (UNDER) {
                     // (a group of four steps lies in one window of 64)
                     if ((QW ? k == 0 : true) && (i & 63) == 0) fbits = sample_bits(i + 1);
-                    if (((fbits >> (i & 63)) & 1u) && __builtin_amdgcn_ballot_w64(x > x_lo) != 0)
+                    if (((fbits >> (i & 63)) & 1u) && __builtin_amdgcn_ballot_w64(x > x_lo && !ps.dead) != 0)
                         observe(0, zone_spot(x), SampleRow{});
                 } else if constexpr (BOOK && DUP) {
                     // (a plain barrier sample changes nothing while every state
@@ -1724,6 +1724,24 @@ __device__ __forceinline__ void path_body(const LaunchParams& P, const int bid, 
                 return zone ? sf : R(0);
             };
 
+            // A path whose adjoint is zero at the last point and stays zero
+            // adds nothing: the barrier's vanilla out of the money, or breached
+            // and no weight on the vanilla; the European out of the money.
+            // Its lane issues no atomics, the load of the LDS pipe in these
+            // kernels (2^20 paths x 156 steps, strike 120 on a spot of 100: FP32
+            // 0.53 -> 0.38 ms, FP64 0.92 -> 0.80, FP32 recompute 0.63 -> 0.56).
+            // (A state out of range is not left out.)  x_adj: the state above
+            // which the lane's samples have an adjoint.
+            auto swept = [&](R abar_end) -> bool {
+                if constexpr (PRD == PRD_BARRIER || PRD == PRD_EUROPEAN) {
+                    const bool zero = PRD == PRD_EUROPEAN ? ns == 1 : ps.euro == R(0) || (ps.dead && w1 == R(0));
+                    return active && !(zero && abar_end == R(0) && x - x == R(0));
+                } else {
+                    return active;
+                }
+            };
+            const R x_adj = UNDER ? (ps.dead || ps.euro == R(0) ? R(INFINITY) : x_lo) : R(0);
+
             if constexpr (DUP && RECOMP) {
                 // ---- reverse sweep, recompute variant: segments of kSeg steps
                 // from the last one back; each segment is first re-simulated
@@ -1741,6 +1759,7 @@ __device__ __forceinline__ void path_body(const LaunchParams& P, const int bid, 
                         abar = S * Fb;
                     }
                 }
+                const bool live = swept(abar);
                 const int nseg = (n + kSeg - 1) / kSeg;
                 for (int sg = nseg - 1; sg >= 0; --sg) {
                     const int i0 = sg * kSeg;
@@ -1809,7 +1828,7 @@ __device__ __forceinline__ void path_body(const LaunchParams& P, const int bid, 
                         cj[k] = b.j;
                         const int smp = __builtin_amdgcn_readfirstlane(step_sample[i]);
                         if constexpr (UNDER) {
-                            if (smp >= 0 && __builtin_amdgcn_ballot_w64(xi > x_lo) != 0)
+                            if (smp >= 0 && __builtin_amdgcn_ballot_w64(xi > x_adj) != 0)
                                 cb[k] = barrier_sf(zone_spot(xi));
                         } else if (smp >= 0) {
                             const SampleRow row = row_of(smp, i);
@@ -1826,7 +1845,7 @@ __device__ __forceinline__ void path_body(const LaunchParams& P, const int bid, 
                     for (int k = kSeg - 1; k >= 0; --k) {
                         const int i = i0 + k;
                         if (i >= n) continue;
-                        if (active) {
+                        if (live) {
                             double* row = ivbl + i * mp;
                             atomicAdd(row + cj[k], double(abar * cw[k]));
                             atomicAdd(row + cj[k] + 1, double(abar * cv[k]));
@@ -1834,7 +1853,7 @@ __device__ __forceinline__ void path_body(const LaunchParams& P, const int bid, 
                         abar = abar * ca[k] + cb[k];
                     }
                 }
-                if (active) padj[0] += double(abar) / s0;      // d log(S0) / d S0
+                if (live) padj[0] += double(abar) / s0;      // d log(S0) / d S0
             } else if constexpr (DUP) {
                 // ---- reverse sweep over the Euler steps (mcMdlDupire.h:259-279)
                 R abar = R(0);   // adjoint of the log-spot state at the current point
@@ -1847,6 +1866,7 @@ __device__ __forceinline__ void path_body(const LaunchParams& P, const int bid, 
                         abar = S * Fb;
                     }
                 }
+                const bool live = swept(abar);
                 R xnext = x;     // state at point i + 1
                 // every local-vol node at least the recovery threshold: no
                 // normal is drawn again
@@ -1945,7 +1965,7 @@ __device__ __forceinline__ void path_body(const LaunchParams& P, const int bid, 
                         wb[k] = b.wb;
                         js[k] = b.j;
                         if constexpr (UNDER) {
-                            if (smp >= 0 && __builtin_amdgcn_ballot_w64(xi > x_lo) != 0)
+                            if (smp >= 0 && __builtin_amdgcn_ballot_w64(xi > x_adj) != 0)
                                 sf[k] = barrier_sf(zone_spot(xi));
                         } else {
                             const SampleRow row = BOOK ? prow : SampleRow{};
@@ -1969,7 +1989,7 @@ __device__ __forceinline__ void path_body(const LaunchParams& P, const int bid, 
                     }
                     // phase 3: scatter onto the two bracketing local-vol nodes
                     // (rows top - U + 1 .. top at fixed offsets from one base)
-                    if (active) {
+                    if (live) {
                         double* rows = ivbl + (top - (U - 1)) * mp;
 #pragma unroll
                         for (int k = 0; k < U; ++k) {
@@ -2017,7 +2037,7 @@ __device__ __forceinline__ void path_body(const LaunchParams& P, const int bid, 
                                     if (b.vol < vmin) ws = draw(i) - b.vol;
                             R sf = R(0);
                             if constexpr (UNDER) {
-                                if (smp >= 0 && __builtin_amdgcn_ballot_w64(xi > x_lo) != 0)
+                                if (smp >= 0 && __builtin_amdgcn_ballot_w64(xi > x_adj) != 0)
                                     sf = barrier_sf(zone_spot(xi));
                             } else if (on && (!(row.grps & kBookPlain) || __builtin_amdgcn_ballot_w64(xi > rv_x) != 0)) {
                                 const R S = state_spot(xi, s0);
@@ -2028,7 +2048,7 @@ __device__ __forceinline__ void path_body(const LaunchParams& P, const int bid, 
                             const R vb = abar * ws;
                             abar = abar + vb * b.slope;
                             abar = abar + sf;
-                            if (active) {
+                            if (live) {
                                 double* row = ivbl + i * mp;
                                 atomicAdd(row + b.j, double(vb * b.wa));
                                 atomicAdd(row + b.j + 1, double(vb * b.wb));
@@ -2105,7 +2125,7 @@ __device__ __forceinline__ void path_body(const LaunchParams& P, const int bid, 
                     }
                     for (; top >= U - 1; top -= U) group(top, std::false_type{});
                 }
-                if (active) padj[0] += double(abar) / s0;      // d log(S0) / d S0
+                if (live) padj[0] += double(abar) / s0;      // d log(S0) / d S0
             } else {
                 // ---- Black-Scholes: forward tangents of the spot with respect
                 // to (spot, vol, rate, div), replaying the checkpointed normals

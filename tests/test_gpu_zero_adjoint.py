@@ -1,0 +1,41 @@
+"""Paths whose adjoint is zero (the vanilla out of the money, a breach without
+weight on the vanilla) are left out of the reverse sweep: risks against the
+CPU oracle's tape where all paths are such, none, and some, with and without
+weight on the vanilla, calls and puts, both layouts, both adjoint variants and
+both sources of normals.  FP64 to 1e-10 of the risks' scale (the bound of the
+parity tests); zero risks are exactly zero."""
+import numpy as np
+import pytest
+
+import compfinance_amd as cf
+import pyoracle as po
+from compfinance_amd import workloads as W
+
+pytestmark = pytest.mark.gpu
+
+
+def check(mk, product, oracle, weights, mode, sobol):
+    n = 700
+    num = cf.NumericalParam(numPath=n, useSobol=sobol, aadMode=mode)
+    res = cf.mcParallelSimulAAD(product, cf.Dupire(**mk), num=num, weights=weights)
+    kw = {} if sobol else dict(mrg=(num.seed1, num.seed2))
+    _, _, risks = po.aad(po.Model(**mk), oracle, n, weights=weights, **kw)
+    assert np.abs(res.risks - risks).max() <= 1e-10 * np.abs(risks).max()
+
+
+@pytest.mark.parametrize("mode", [cf.AAD_CHECKPOINT, cf.AAD_RECOMPUTE])
+@pytest.mark.parametrize("sobol,put", [(True, False), (False, True)])
+@pytest.mark.parametrize("weights", [[1.0, 0.0], [1.0, 0.4], [0.0, 1.0]])
+@pytest.mark.parametrize("strike", [1.0, 105.0, 1.0e4])
+@pytest.mark.parametrize("weeks,n_spots", [(7, 30), (66, 30), (66, 260)])
+def test_barrier(engine, weeks, n_spots, strike, weights, sobol, put, mode):
+    mk = W.dupire_args(n_spots)
+    pk = W.barrier_args(strike=strike, barrier=112.0, maturity=weeks / 52.0, put=put)
+    check(mk, cf.UOC(**pk), po.Product(**pk), weights, mode, sobol)
+
+
+@pytest.mark.parametrize("mode", [cf.AAD_CHECKPOINT, cf.AAD_RECOMPUTE])
+@pytest.mark.parametrize("strike", [1.0, 100.0, 1.0e4])
+def test_european(engine, strike, mode):
+    mk, pk = W.dupire_args(30), dict(strike=strike, exerciseDate=1.0)
+    check(mk, cf.European(**pk), po.Product(**pk), [1.0], mode, True)
