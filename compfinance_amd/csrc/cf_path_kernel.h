@@ -775,13 +775,15 @@ __device__ __forceinline__ void path_body(const LaunchParams& P, const int bid, 
     // the inverse-normal table (FP32) and the knot search table are read from
     // global memory through the L1 cache, not LDS, by the LEAN kernels and by
     // the FP32 recompute kernels, whose re-simulation otherwise loads the LDS
-    // most (measured: C3 FP32 recompute 0.719 -> 0.643 ms; the pricing kernels
-    // are faster with both in LDS).  The FP32 Dupire checkpoint kernels other
-    // than the book, bound by the LDS pipe, read the inverse-normal table
-    // through L1 (C3 0.587 -> 0.576 ms; with the knot search table as well
-    // they lose: the vector memory path saturates instead)
+    // most (measured: C3 FP32 recompute 0.719 -> 0.643 ms).  The other FP32
+    // Dupire kernels but the book's, bound by the LDS pipe, read the
+    // inverse-normal table through L1: a step's six LDS reads take 28 cycles
+    // of the pipe and 15 more of bank conflicts, as many as its vector
+    // instructions.  (Pricing 2^19 paths x 156 steps 0.131 -> 0.116 ms, C3 risk
+    // 0.587 -> 0.576 ms; with the knot search table as well they lose: the
+    // vector memory path saturates instead)
     constexpr bool GTAB = LEAN || (RECOMP && sizeof(R) == 4);
-    constexpr bool GINV = GTAB || (sizeof(R) == 4 && ADJ == ADJ_CHECKPOINT && DUP && !BOOK);
+    constexpr bool GINV = GTAB || (sizeof(R) == 4 && DUP && !BOOK && ADJ != ADJ_RECOMPUTE);
 
     // Sobol LO layout: the FP32 Dupire adjoint kernels other than the book
     // read four dimensions at once (quads); the others one at a time (rows)
