@@ -1046,6 +1046,21 @@ CallShape shape_call(const Engine& E, const Prepared& PR, const cf_num* num, boo
     return S;
 }
 
+void add_ck_slots(const Prepared& PR, size_t limit, CallShape* S)
+{
+    // (a redrawn normal would need the words of each path's own block)
+    const bool product = PR.cfg.product == cfk::PRD_BARRIER ||
+                         (PR.cfg.product == cfk::PRD_EUROPEAN && PR.pd.timeline.size() == 1);
+    if (!S->adjoint || !S->fp64 || PR.md.kind != CF_MODEL_DUPIRE || PR.cfg.recompute || !product || !PR.iv_recover ||
+        S->slots == 0)
+        return;
+    const int64_t q0 = (S->first + 1) >> 6, q1 = (S->first + S->n_path) >> 6;
+    const int64_t blocks = q1 - q0 + 1 - (S->merge ? 1 : 0);
+    const size_t one = call_bytes(*S).ckpt / size_t(S->ck_slots);
+    S->ck_slots = int(std::max<int64_t>(1, std::min({int64_t(cfk::kMaxCkSlots), (blocks + S->slots - 1) / S->slots,
+                                                     one ? int64_t(limit / one) : int64_t(1)})));
+}
+
 static size_t al256(size_t x) { return (x + 255) & ~size_t(255); }
 
 size_t CallBytes::total() const
@@ -1061,7 +1076,7 @@ CallBytes call_bytes(const CallShape& S)
     b.ivbar_blocks = size_t(S.grid) * S.ivn * 8;
     b.ivbar = S.ivn * 8;
     b.weights = S.adjoint ? size_t(S.npay) * 8 : 0;
-    b.ckpt = size_t(S.slots) * S.ck_rows * cfk::kWave * (S.fp64 ? 8 : 4);
+    b.ckpt = size_t(S.slots) * S.ck_slots * S.ck_rows * cfk::kWave * (S.fp64 ? 8 : 4);
     return b;
 }
 
@@ -1140,6 +1155,7 @@ cfk::LaunchParams launch_params(const Engine& E, const Prepared& PR, const CallS
     P.ivbar_copies = PR.ivbar_copies;
     P.iv_recover = PR.iv_recover ? 1 : 0;
     P.rev_point = md.n_steps;
+    P.ck_slots = S.ck_slots;
     return P;
 }
 
@@ -1250,7 +1266,14 @@ int run(const cf_model* mdl, const cf_product* prd, Call& c)
     hip_check(hipSetDevice(E.device), "hipSetDevice");
     const std::shared_ptr<Prepared> PP = lookup(E, mdl, prd, fp64, adjoint_kind(c), true, call_block(E, c.num, fp64));
     const Prepared& PR = *PP;
-    const CallShape S = shape_call(E, PR, c.num, c.adjoint);
+    CallShape S = shape_call(E, PR, c.num, c.adjoint);
+    add_ck_slots(PR, kCkSlotsBytes, &S);
+    if (S.ck_slots > 1 && call_bytes(S).ckpt > E.ckpt.cap) {
+        // (as many as the device's memory holds)
+        size_t free_b = 0, total_b = 0;
+        hip_check(hipMemGetInfo(&free_b, &total_b), "hipMemGetInfo");
+        if (call_bytes(S).ckpt + (size_t(256) << 20) > free_b + E.ckpt.cap) S.ck_slots = 1;
+    }
     const CallBytes nb = call_bytes(S);
 
     double* h_in = static_cast<double*>(E.pin_in.ensure(size_t(S.npay) * 8));

@@ -306,9 +306,15 @@ struct CallShape {
     int grid = 0, waves = 0, slots = 0, stride = 0, npay = 0, ck_rows = 0, n_steps = 0;
     size_t ivn = 0;                 // Dupire adjoint: steps x spots
     bool adjoint = false, fp64 = false;
+    int ck_slots = 1;               // checkpoint slots per wave
     bool merge = false;             // the last block of 64 Sobol indices runs in the first block's lanes
 };
 CallShape shape_call(const Engine& E, const Prepared& PR, const cf_num* num, bool adjoint);
+// Checkpoints of the synchronous calls with more than one slot per wave.
+constexpr size_t kCkSlotsBytes = size_t(2) << 30;
+// More checkpoint slots per wave for the kernels that sweep the paths of
+// several blocks together, within `limit` bytes of checkpoints.
+void add_ck_slots(const Prepared& PR, size_t limit, CallShape* S);
 
 // Device buffers of one call.
 struct CallBuffers {
@@ -318,7 +324,7 @@ struct CallBuffers {
     double* ivbar_blocks = nullptr; // [grid][ivn]
     double* ivbar = nullptr;        // [ivn]
     double* weights = nullptr;      // [npay]
-    void* ckpt = nullptr;           // [slots][ck_rows][64] reals
+    void* ckpt = nullptr;           // [slots][ck_slots][ck_rows][64] reals
     double* per_path = nullptr;     // [n_path][npay] or null
     double* per_path_agg = nullptr; // [n_path] or null
 };

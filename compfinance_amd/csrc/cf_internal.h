@@ -96,6 +96,10 @@ constexpr double kNarrowZone = 0.05;
 // multiple of four; FP64 keeps the last n_steps % 4 steps in rows of 64.
 constexpr int kMaxStoredKnots = 255;
 constexpr int kCkptGuardRows = 4;
+// Slots that a wave of the Dupire checkpoint kernels of a barrier or a European
+// keeps at most: the paths with an adjoint of up to so many blocks of 64 are
+// swept together.
+constexpr int kMaxCkSlots = 4;
 CF_HD inline int ckpt_steps(int n_steps, int real_bytes) { return real_bytes == 4 ? (n_steps + 3) & ~3 : n_steps; }
 CF_HD inline int ckpt_rows(int n_steps, bool dupire, bool recompute, int real_bytes)
 {
@@ -195,6 +199,7 @@ struct LaunchParams {
     int rev_point;               // the reverse starts at this timeline point's step (n_steps: all;
                                  // itemized risk: the one payoff's last observation)
     void* state;                 // [blocks of 64 paths][state_rows(product)][64] reals
+    int ck_slots;                // checkpoint slots of a wave, at least 1 (kMaxCkSlots)
 };
 
 // Calls packed into one launch of a path kernel: call r runs on blocks

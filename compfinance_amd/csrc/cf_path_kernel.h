@@ -851,7 +851,16 @@ __device__ __forceinline__ void path_body(const LaunchParams& P, const int bid, 
     // Sobol indices (set per block below)
     // (only the ITEM checkpoint kernels read ck_mode)
     const int ck_mode = ITEM && ADJ == ADJ_CHECKPOINT ? P.ck_mode : 0;
-    R* ck = AD ? static_cast<R*>(P.ckpt) + (size_t(slot) * ck_rows + (CKB ? kCkptGuardRows : 0)) * kWave : nullptr;
+    // PK: the swept paths of up to ck_slots blocks share a reverse sweep (see
+    // there); ck is the slot of the block in work.  FP64 (2^20 paths x 156
+    // steps, one path in ten swept: 0.80 -> 0.67 ms).  FP32 sweeps each block by
+    // itself: its sweeps take less than the checkpoints of four slots, which
+    // leave the last-level cache, cost (0.38 against 0.41 ms).
+    constexpr bool PK = CKB && !ITEM && sizeof(R) == 8 && (PRD == PRD_BARRIER || PRD == PRD_EUROPEAN);
+    const int ck_slots = PK ? P.ck_slots : 1;
+    R* const ck0 = AD ? static_cast<R*>(P.ckpt) +
+                            (size_t(slot) * ck_slots * ck_rows + (CKB ? kCkptGuardRows : 0)) * kWave : nullptr;
+    R* ck = ck0;
     // (the FULL layout is only chosen for grids of at most kMaxStoredKnots knots)
     const bool ck_lo = CKB && (!LEAN || m <= kMaxStoredKnots);
     // States and bracket bytes interleaved by groups of four steps (a lane's
@@ -861,7 +870,8 @@ __device__ __forceinline__ void path_body(const LaunchParams& P, const int bid, 
     constexpr bool IL = CKB;
     const int nck = ckpt_steps(n, int(sizeof(R)));
     const int n4 = n & ~3;
-    uint8_t* ckl = CKB ? reinterpret_cast<uint8_t*>(ck + size_t(nck) * kWave) : nullptr;
+    uint8_t* const ckl0 = CKB ? reinterpret_cast<uint8_t*>(ck + size_t(nck) * kWave) : nullptr;
+    uint8_t* ckl = ckl0;
     // element of step i of this lane in the states (and bracket bytes)
     auto ck_el = [&](int i) -> int {
         return IL && (sizeof(R) == 4 || i < n4) ? ((i >> 2) << 8) + (lane << 2) + (i & 3) : i * kWave + lane;
@@ -998,6 +1008,12 @@ __device__ __forceinline__ void path_body(const LaunchParams& P, const int bid, 
     // the survival factor of a state
     auto bar_alive = [&](R v) -> R { return v > R(0) && (!ZT || v <= R(1)) ? v : R(0); };
     const R bk_xlo = BOOK && DUP ? R(P.bar_xlo) : R(0);   // every zone is above this state
+
+    // PK: swept paths waiting for a full wave, in lanes 0 .. pk_n - 1 of pk_src
+    // (lane of the block, slot << 6, count of zero factors << 28, breached
+    // << 30), from pk_used slots up to the one before pk_slot
+    uint32_t pk_src = 0;
+    int pk_n = 0, pk_used = 0, pk_slot = 0;
 
     for (int64_t q = q0 + int64_t(bid) * waves + wave; q <= qe; q += int64_t(nblk) * waves) {
         // ---- high Sobol words of this block of 64 indices (and of the
@@ -1547,6 +1563,106 @@ __device__ __forceinline__ void path_body(const LaunchParams& P, const int bid, 
                 }
             }
 
+            const R w0 = R(wts[0]);
+            const R w1 = npay > 1 ? R(wts[1]) : R(0);
+            // A path whose adjoint is zero at the last point and stays zero
+            // adds nothing: the barrier's vanilla out of the money, or breached
+            // and no weight on the vanilla; the European out of the money.
+            // Its lane issues no atomics, the load of the LDS pipe in these
+            // kernels (2^20 paths x 156 steps, strike 120 on a spot of 100: FP32
+            // 0.53 -> 0.38 ms, FP64 0.92 -> 0.80, FP32 recompute 0.63 -> 0.56).
+            // (A state or weight out of range is not left out.)
+            bool live = active;
+            if constexpr (DUP && (PRD == PRD_BARRIER || PRD == PRD_EUROPEAN)) {
+                const R F = state_spot(x, s0), k = R(P.strike);
+                const bool in = PRD == PRD_BARRIER && P.put ? k > F : F > k;
+                const bool zero = PRD == PRD_EUROPEAN ? ns == 1 && !in : !in || (ps.dead && w1 == R(0));
+                live = active && !(zero && x - x == R(0) && F - F == R(0) && w0 - w0 == R(0));
+            }
+            // PK: the swept paths of up to ck_slots blocks are gathered, each
+            // lane of a sweep reading the checkpoints and the end state of its
+            // own block's slot (the end state in the slot's guard rows), until
+            // they fill a wave, their slots are all taken or the wave's last
+            // block is done; pk_cnt: the paths of the sweep.
+            int pk_cnt = kWave;
+            uint32_t src = uint32_t(lane);
+            bool pk_last = false;
+            if (PK && ck_slots > 1) {
+                ck[lane - kWave] = x;
+                if constexpr (PRD == PRD_BARRIER) {
+                    // (the product of the factors, with zero ones that of the others)
+                    ck[lane - 2 * kWave] = ps.nzero == 0 ? ps.alive : ps.pnz;
+                    ck[lane - 3 * kWave] = ps.euro;
+                }
+                // (other lanes read the slot: after its stores)
+                __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+                const uint64_t lm = __builtin_amdgcn_ballot_w64(live);
+                const int nl = __builtin_popcountll(lm), total = pk_n + nl;
+                // the live lanes from lane pk_n on, the others behind them
+                auto rank = [&](uint64_t mk) {
+                    return int(__builtin_amdgcn_mbcnt_hi(uint32_t(mk >> 32), __builtin_amdgcn_mbcnt_lo(uint32_t(mk), 0u)));
+                };
+                const int dst = pk_n + (live ? rank(lm) : nl + rank(~lm));
+                const uint32_t mine = uint32_t(lane) | uint32_t(pk_slot) << 6 | uint32_t(min(ps.nzero, 2)) << 28 |
+                                      (ps.dead ? 1u << 30 : 0u);
+                const uint32_t got = uint32_t(__builtin_amdgcn_ds_permute((dst & (kWave - 1)) << 2, int(mine)));
+                src = lane < pk_n ? pk_src : got;
+                pk_last = q + int64_t(nblk) * waves > qe;
+                bool kept;
+                if (total >= kWave) {
+                    pk_src = got;
+                    pk_n = total - kWave;
+                    kept = pk_n > 0;
+                    pk_used = kept ? 1 : 0;
+                } else {
+                    pk_src = src;
+                    pk_used += nl > 0 ? 1 : 0;
+                    pk_cnt = pk_last || pk_used == ck_slots ? total : 0;
+                    kept = nl > 0 && pk_cnt == 0;
+                    pk_n = total;
+                    if (pk_cnt > 0) { pk_n = 0; pk_used = 0; }
+                }
+                if (kept) {
+                    pk_slot = pk_slot + 1 == ck_slots ? 0 : pk_slot + 1;
+                    ck = ck0 + size_t(pk_slot) * ck_rows * kWave;
+                    ckl = ckl0 + size_t(pk_slot) * ck_rows * kWave * sizeof(R);
+                }
+            } else if constexpr (PK) {
+                if (__builtin_amdgcn_ballot_w64(live) == 0) pk_cnt = 0;
+            }
+
+            for (bool more = pk_cnt > 0; more;) {
+            more = false;
+            // the lane's path of the sweep: its lane in the block and its slot
+            int rl = lane;
+            uint32_t so = 0;
+            if (PK && ck_slots > 1) {
+                live = lane < pk_cnt;
+                if (!live) src = __builtin_amdgcn_readfirstlane(src);
+                rl = int(src & 63u);
+                so = ((src >> 6) & 63u) * uint32_t(ck_rows * kWave);
+                const R* e = ck0 + (so + uint32_t(rl));
+                x = e[-kWave];
+                if constexpr (PRD == PRD_BARRIER) {
+                    ps.nzero = int((src >> 28) & 3u);
+                    ps.dead = (src >> 30) != 0;
+                    ps.pnz = e[-2 * kWave];
+                    ps.alive = ps.nzero == 0 ? ps.pnz : R(0);
+                    ps.euro = e[-3 * kWave];
+                    nzw = __builtin_amdgcn_ballot_w64(ps.nzero != 0) != 0;
+                }
+                if (pk_last && pk_n > 0) { more = true; src = pk_src; pk_cnt = pk_n; pk_n = 0; }
+            }
+            // checkpoints of the lane's path: byte offsets of the states and
+            // brackets of an aligned group of four, and of a state row
+            const uint32_t vx = (so + uint32_t(rl << 2)) * uint32_t(sizeof(R));
+            const uint32_t vb4 = so * uint32_t(sizeof(R)) + uint32_t(rl << 2);
+            auto at = [](const void* base, uint32_t off) -> const char* {
+                return static_cast<const char*>(base) + off;
+            };
+            const R* const ckr = PK ? ck0 : ck;
+            const uint8_t* const cklr = PK ? ckl0 : ckl;
+
             // book: the spot above which barrier b has an adjoint on this
             // lane, the lower end of its zone, or +infinity (breached, the
             // vanilla out of the money or without weight).  Kept per barrier in
@@ -1575,8 +1691,6 @@ __device__ __forceinline__ void path_body(const LaunchParams& P, const int bid, 
             }
 
             // adjoints of the forward, numeraire and discount at sample s
-            const R w0 = R(wts[0]);
-            const R w1 = npay > 1 ? R(wts[1]) : R(0);
             const R alive_eff = ps.dead ? R(0) : ps.alive;
             const R euro_bar = w0 * alive_eff + w1;       // barrier: adjoint of the vanilla
             const R alive_bar = w0 * ps.euro;             // barrier: adjoint of alive
@@ -1726,22 +1840,6 @@ __device__ __forceinline__ void path_body(const LaunchParams& P, const int bid, 
                 return zone ? sf : R(0);
             };
 
-            // A path whose adjoint is zero at the last point and stays zero
-            // adds nothing: the barrier's vanilla out of the money, or breached
-            // and no weight on the vanilla; the European out of the money.
-            // Its lane issues no atomics, the load of the LDS pipe in these
-            // kernels (2^20 paths x 156 steps, strike 120 on a spot of 100: FP32
-            // 0.53 -> 0.38 ms, FP64 0.92 -> 0.80, FP32 recompute 0.63 -> 0.56).
-            // (A state out of range is not left out.)  x_adj: the state above
-            // which the lane's samples have an adjoint.
-            auto swept = [&](R abar_end) -> bool {
-                if constexpr (PRD == PRD_BARRIER || PRD == PRD_EUROPEAN) {
-                    const bool zero = PRD == PRD_EUROPEAN ? ns == 1 : ps.euro == R(0) || (ps.dead && w1 == R(0));
-                    return active && !(zero && abar_end == R(0) && x - x == R(0));
-                } else {
-                    return active;
-                }
-            };
             const R x_adj = UNDER ? (ps.dead || ps.euro == R(0) ? R(INFINITY) : x_lo) : R(0);
 
             if constexpr (DUP && RECOMP) {
@@ -1761,7 +1859,6 @@ __device__ __forceinline__ void path_body(const LaunchParams& P, const int bid, 
                         abar = S * Fb;
                     }
                 }
-                const bool live = swept(abar);
                 const int nseg = (n + kSeg - 1) / kSeg;
                 for (int sg = nseg - 1; sg >= 0; --sg) {
                     const int i0 = sg * kSeg;
@@ -1868,7 +1965,6 @@ __device__ __forceinline__ void path_body(const LaunchParams& P, const int bid, 
                         abar = S * Fb;
                     }
                 }
-                const bool live = swept(abar);
                 R xnext = x;     // state at point i + 1
                 // every local-vol node at least the recovery threshold: no
                 // normal is drawn again
@@ -1894,13 +1990,13 @@ __device__ __forceinline__ void path_body(const LaunchParams& P, const int bid, 
                 // states and brackets of steps top, top - 1, ..., top - U + 1
                 auto load_group = [&](int top, R* xb, int* lb) {
                     if constexpr (VG) {
-                        const int e = ck_el(top - 3);   // a 16-byte aligned group
-                        const float4 v = *reinterpret_cast<const float4*>(ck + e);
+                        const int e = (top - 3) * kWave;   // an aligned group
+                        const float4 v = *reinterpret_cast<const float4*>(at(ckr + e, vx));
                         xb[0] = v.w;
                         xb[1] = v.z;
                         xb[2] = v.y;
                         xb[3] = v.x;
-                        const uint32_t w = ck_lo ? *reinterpret_cast<const uint32_t*>(ckl + e) : 0u;
+                        const uint32_t w = ck_lo ? *reinterpret_cast<const uint32_t*>(at(cklr + e, vb4)) : 0u;
 #pragma unroll
                         for (int k = 0; k < 4; ++k) lb[k] = int((w >> (8 * (3 - k))) & 0xffu);
                     } else {
@@ -2060,15 +2156,18 @@ __device__ __forceinline__ void path_body(const LaunchParams& P, const int bid, 
                         double2 c0, c1;
                         uint32_t cw;
                         auto load4 = [&](int g) {   // (below step 0: the slot's guard rows, never used)
-                            const int e = (g << 8) + (lane << 2);
-                            const double2* c = reinterpret_cast<const double2*>(ck + e);
+                            const double2* c = reinterpret_cast<const double2*>(at(ckr + (g << 8), vx));
                             c0 = c[0];
                             c1 = c[1];
-                            cw = ck_lo ? *reinterpret_cast<const uint32_t*>(ckl + e) : 0u;
+                            cw = ck_lo ? *reinterpret_cast<const uint32_t*>(at(cklr + (g << 8), vb4)) : 0u;
                         };
                         auto sweep = [&](auto recover) {
                             int top = last;
-                            for (; top >= n4; --top) step(top, ck[ck_el(top)], ck_lo ? int(ckl[ck_el(top)]) : 0, recover);
+                            for (; top >= n4; --top) {
+                                const uint32_t e = so + uint32_t(rl);
+                                step(top, (ckr + top * kWave)[e],
+                                     ck_lo ? int((cklr + top * kWave)[e + so * uint32_t(sizeof(R) - 1)]) : 0, recover);
+                            }
                             if (top < 0) return;
                             load4(top >> 2);
                             for (int g = top >> 2; g >= 0; --g) {
@@ -2181,6 +2280,7 @@ __device__ __forceinline__ void path_body(const LaunchParams& P, const int bid, 
                     const int s = step_sample[i + 1];
                     if (s >= 0) accumulate(s, spot);
                 }
+            }
             }
         }
     }

@@ -39,3 +39,22 @@ def test_barrier(engine, weeks, n_spots, strike, weights, sobol, put, mode):
 def test_european(engine, strike, mode):
     mk, pk = W.dupire_args(30), dict(strike=strike, exerciseDate=1.0)
     check(mk, cf.European(**pk), po.Product(**pk), [1.0], mode, True)
+
+
+@pytest.mark.parametrize("strike,weights", [(120.0, [1.0, 0.0]), (100.0, [1.0, 0.3]), (1.0, [0.0, 1.0]),
+                                            (1.0e4, [1.0, 0.0]), (118.0, None)])
+@pytest.mark.parametrize("n,first", [((1 << 19) + 77, 0), (1 << 20, 1000)])
+def test_paths_of_several_blocks_are_swept_together(engine, n, first, strike, weights):
+    """A wave with several blocks of 64 paths gathers the swept ones: the call
+    equals the path-weighted mean of calls small enough for one block a wave.
+    The same terms in another order, to 1e-11 of their scale."""
+    mdl = cf.Dupire(**W.dupire_args(30))
+    prd = cf.European(strike, 0.75) if weights is None else cf.UOC(**W.barrier_args(strike=strike, maturity=0.75))
+    weights = weights or [1.0]
+    res = cf.mcParallelSimulAAD(prd, mdl, num=cf.NumericalParam(numPath=n, firstPath=first), weights=weights)
+    part, total = 1 << 17, 0.0
+    for lo in range(0, n, part):
+        m = min(part, n - lo)
+        total = total + m * cf.mcParallelSimulAAD(
+            prd, mdl, num=cf.NumericalParam(numPath=m, firstPath=first + lo), weights=weights).risks
+    assert np.abs(res.risks - total / n).max() <= 1e-11 * np.abs(total / n).max()
