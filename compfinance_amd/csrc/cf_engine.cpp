@@ -874,8 +874,8 @@ std::shared_ptr<Prepared> prepare(Engine& E, const cf_model* mdl, const cf_produ
     };
     P->ivbar_copies = 1;
     // the FULL checkpoint kernels keep each state's bracket in a byte, and the
-    // FULL kernels' knot search reads at most two knots of a bucket
-    const int lean_from = forced == 1 || (dup && (md.n_spots > cfk::kMaxStoredKnots || P->bt.fix > 2)) ? 1 : 0;
+    // FULL kernels' knot search reads one knot of a bucket
+    const int lean_from = forced == 1 || (dup && (md.n_spots > cfk::kMaxStoredKnots || P->bt.fix > 1)) ? 1 : 0;
     for (int lean = lean_from; lean < 2; ++lean) {
         P->cfg.lean = lean != 0;
         P->smem = lds_bytes(1);

@@ -290,34 +290,46 @@ struct alignas(16) BucketEntry {
     int lo, pad;
 };
 
+// The FULL layout's copy in LDS, for tables of at most one knot a bucket (any
+// grid whose buckets are not capped): one 8-byte read in FP32, half the
+// entry's, which the LDS pipe bounds.
+template <typename R>
+struct alignas(2 * sizeof(R)) BucketOne {
+    R k0;
+    int lo;
+};
+
 // ---- knot search (upper_bound on the knots, interp.h:40), one definition for
 // the kernels and for the host that builds the table.  The bucket of state x
-// is floor(clamp(fma(x, invh, c0), 0, nb - 1)): monotone in x, so the knots
+// is, in FP64, floor(clamp(fma(x, invh, c0), 0, nb - 1)) and in FP32 the same
+// of the nearest integer, read off the low bits of the sum with 1.5 2^23
+// (part of c0), without a conversion: monotone in x, so the knots
 // of earlier buckets are all <= x and those of later buckets all > x.
 // Bucket b holds lo, the number of knots in earlier buckets, and its first two
 // knots (NaN past the last knot); at most `fix` knots share a bucket.
+constexpr float kBucketMagic = 12582912.0f;         // 1.5 2^23
+constexpr uint32_t kBucketMagicBits = 0x4b400000u;
 #if defined(__HIP_DEVICE_COMPILE__)
-__device__ inline float clamp_bucket(float b, float top) { return __builtin_amdgcn_fmed3f(b, 0.0f, top); }
+__device__ inline float clamp_bucket(float b, float lo, float top) { return __builtin_amdgcn_fmed3f(b, lo, top); }
 #else
-inline float clamp_bucket(float b, float top)
+inline float clamp_bucket(float b, float lo, float top)
 {
-    b = b > 0.0f ? b : 0.0f;
+    b = b > lo ? b : lo;
     return b < top ? b : top;
 }
 #endif
-CF_HD inline double clamp_bucket(double b, double top)
+CF_HD inline double clamp_bucket(double b, double lo, double top)
 {
-    b = b > 0.0 ? b : 0.0;
+    b = b > lo ? b : lo;
     return b < top ? b : top;
 }
 CF_HD inline float fma_r(float a, float b, float c) { return __builtin_fmaf(a, b, c); }
 CF_HD inline double fma_r(double a, double b, double c) { return __builtin_fma(a, b, c); }
 
-// Bucket of x, as a real in [0, top] (NaN: converts to bucket 0 on the device).
-template <typename R>
-CF_HD inline R bucket_pos(R x, R invh, R c0, R top)
+// FP32: the bucket of x as the bits of 1.5 2^23 + bucket (NaN: bucket 0).
+CF_HD inline uint32_t bucket_bits(float x, float invh, float c0, float top)
 {
-    return clamp_bucket(fma_r(x, invh, c0), top);
+    return __builtin_bit_cast(uint32_t, clamp_bucket(fma_r(x, invh, c0), kBucketMagic, kBucketMagic + top));
 }
 
 // The bucket of x as an index.  FP64 on the device: the conversion saturates
@@ -326,16 +338,20 @@ CF_HD inline R bucket_pos(R x, R invh, R c0, R top)
 template <typename R>
 CF_HD inline int bucket_index(R x, R invh, R c0, R top, int itop)
 {
+    if constexpr (sizeof(R) == 4) {
+        (void)itop;
+        return int(bucket_bits(x, invh, c0, top) - kBucketMagicBits);
+    } else {
 #if defined(__HIP_DEVICE_COMPILE__)
-    if constexpr (sizeof(R) == 8) {
         int b;
         asm("v_cvt_i32_f64 %0, %1" : "=v"(b) : "v"(fma_r(x, invh, c0)));
         asm("v_med3_i32 %0, %1, 0, %2" : "=v"(b) : "v"(b), "s"(itop));
         return b;
-    }
+#else
+        (void)itop;
+        return int(clamp_bucket(fma_r(x, invh, c0), 0.0, top));
 #endif
-    (void)itop;
-    return int(bucket_pos(x, invh, c0, top));
+    }
 }
 
 template <typename R>
@@ -368,6 +384,13 @@ CF_HD inline int count_le(const KnotSearch<R>& s, R x)
     return c;
 }
 
+// The FULL layout's search (at most one knot a bucket).
+template <typename R>
+CF_HD inline int count_le_one(const BucketOne<R>& e, R x)
+{
+    return e.lo + int(e.k0 <= x);
+}
+
 // Host: the knot search table of increasing knots (at least one), in the
 // kernel's real type.  Buckets of width at most half the smallest knot gap
 // (at most 16384 of them), so that normally no more than two knots share one.
@@ -393,10 +416,18 @@ inline KnotTable<R> build_knot_table(const R* knots, int m)
         nb = int(want < 16384.0 ? want : 16384.0);
     }
     t.invh = nb > 1 ? R(double(nb) / range) : R(0);
-    t.c0 = R(-double(x0) * double(t.invh));
+    if (sizeof(R) == 4) {
+        // whole buckets around the grid, the first at an integer
+        double first = std::floor(double(x0) * double(t.invh));
+        if (!(std::fabs(first) < 2097152.0)) { nb = 1; t.invh = R(0); first = 0.0; }
+        t.c0 = R(double(kBucketMagic) - first);
+        if (nb > 1) nb += 2;
+    } else {
+        t.c0 = R(-double(x0) * double(t.invh));
+    }
     const R top = R(nb - 1);
     std::vector<int> cnt(size_t(nb), 0);
-    for (int k = 0; k < m; ++k) cnt[size_t(int(bucket_pos(knots[k], t.invh, t.c0, top)))]++;
+    for (int k = 0; k < m; ++k) cnt[size_t(bucket_index(knots[k], t.invh, t.c0, top, nb - 1))]++;
     t.entries.resize(size_t(nb));
     const R none = R(NAN);
     int acc = 0;
@@ -447,9 +478,7 @@ CF_HD inline SmemLayout smem_layout(int n_steps, int n_spots, int n_samples, int
     L.invn = o;        o = cf_align16(o + (real_bytes == 4 && !lean ? size_t(kInvNormalRows) * 4 * 4 : 0));
     // interval (start, inverse width) pairs, interleaved
     L.knots = o;       o = cf_align16(o + (dupire ? size_t(2 * (n_spots + 1)) * real_bytes : 0));
-    L.bucket = o;      o = cf_align16(o + (dupire && !lean ? size_t(n_buckets) * (real_bytes == 4 ? sizeof(BucketEntry<float>)
-                                                                                            : sizeof(BucketEntry<double>))
-                                                           : 0));
+    L.bucket = o;      o = cf_align16(o + (dupire && !lean ? size_t(n_buckets) * size_t(2 * real_bytes) : 0));
     L.iv = o;          o = cf_align16(o + (dupire && !lean ? size_t(n_steps) * lv_cols(n_spots) * real_bytes : 0));
     L.drift = o;       o = cf_align16(o + (dupire ? 0 : size_t(n_steps) * real_bytes));
     L.stdv = o;        o = cf_align16(o + (dupire ? 0 : size_t(n_steps) * real_bytes));

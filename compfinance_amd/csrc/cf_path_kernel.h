@@ -202,17 +202,19 @@ __device__ __forceinline__ double inv_normal(uint32_t xi, const double*)
 constexpr int kInvNormalRowBias = 127 << 3;
 __device__ __forceinline__ float inv_normal(uint32_t xi, const float* tabm)
 {
-    const uint32_t sgn = xi & 0x80000000u;            // u >= 1/2 for the reference scaling
-    // 2^32 - xi, exact.  xi = 0 would give row -1016: the kernel never passes
-    // it (only Sobol index 0 has a zero word, and its lane reads 2^31 instead)
-    // (as signed integers xi < 0 exactly when u >= 1/2, and xi = 2^31 maps to itself)
-    const uint32_t xs = uint32_t(max(int(xi), int(0u - xi)));
-    const uint32_t bits = __float_as_uint(float(xs));
+    // 2^32 min(u, 1 - u) is |xi| as signed integers (xi < 0 exactly when
+    // u >= 1/2, and 2^31 maps to itself): one conversion gives its float, with
+    // the sign of 1/2 - u in the sign bit.  xi = 0 would give row -1016: the
+    // kernel never passes it (only Sobol index 0 has a zero word, and its lane
+    // reads 2^31 instead)
+    const uint32_t bits = __float_as_uint(float(int(xi)));
     // row (bits >> 20) - 1016 in [0, kInvNormalRows - 1], 16 bytes a row
-    const float4 c = *reinterpret_cast<const float4*>(tabm + ((bits >> 18) & 0x3ffcu));
-    const float t = fmaf(float(bits & 0xfffffu), 1.0f / 524288.0f, -1.0f);
+    const float4 c = *reinterpret_cast<const float4*>(tabm + ((bits >> 18) & 0x1ffcu));
+    // the row's argument m / 2^19 - 1 of the float's last 20 bits m, exactly:
+    // as the mantissa of a float in [4, 4.5)
+    const float t = fmaf(__uint_as_float((bits & 0xfffffu) | 0x40800000u), 4.0f, -17.0f);
     const float p = fmaf(fmaf(fmaf(c.w, t, c.z), t, c.y), t, c.x);
-    return __uint_as_float(__float_as_uint(p) ^ sgn);   // -p for u >= 1/2
+    return __uint_as_float(__float_as_uint(p) ^ (bits & 0x80000000u));   // -p for u >= 1/2
 }
 
 // Four FP64 normals of this lane's uniforms, with Moro's tail evaluated once
@@ -509,7 +511,7 @@ struct Bracket {
     R wa, wb;     // adjoint weights of nodes j and j + 1
 };
 
-// Interval c = count_le(ks, x), the number of knots <= x, found by the
+// Interval c = knot_count(x), the number of knots <= x, found by the
 // caller (the reverse sweep reloads it from the forward's).  The interval
 // tables make the flat extrapolation an ordinary interval: for c = 0 and
 // c = m the padded row repeats the end value and the inverse width is 0, so
@@ -531,12 +533,6 @@ __device__ __forceinline__ Bracket<R> local_vol_at(const R* kxi, const R* row, R
     b.wa = R(1) - t;
     b.wb = t;
     return b;
-}
-
-template <bool LEAN, typename R>
-__device__ __forceinline__ Bracket<R> local_vol(const KnotSearch<R>& ks, const R* kxi, const R* row, R x)
-{
-    return local_vol_at(kxi, row, x, count_le<LEAN>(ks, x));
 }
 
 __device__ __forceinline__ double recip_mul(double a, double b) { return fast_div(a, b); }
@@ -756,7 +752,7 @@ __device__ __forceinline__ void path_body(const LaunchParams& P, const int bid, 
     uint32_t* hi_all = reinterpret_cast<uint32_t*>(smem + L.hi);
     int* step_sample = reinterpret_cast<int*>(smem + L.step_sample);
     R* kxi = reinterpret_cast<R*>(smem + L.knots);   // interval (start, inverse width) pairs
-    BucketEntry<R>* bucket = reinterpret_cast<BucketEntry<R>*>(smem + L.bucket);
+    BucketOne<R>* bucket = reinterpret_cast<BucketOne<R>*>(smem + L.bucket);
     R* iv_lds = reinterpret_cast<R*>(smem + L.iv);
     R* drift = reinterpret_cast<R*>(smem + L.drift);
     R* stdv = reinterpret_cast<R*>(smem + L.stdv);
@@ -772,22 +768,19 @@ __device__ __forceinline__ void path_body(const LaunchParams& P, const int bid, 
     R* invn = reinterpret_cast<R*>(smem + L.invn);   // FP32 inverse-normal table
 
     const int tid = threadIdx.x, nthr = blockDim.x;
-    // the inverse-normal table (FP32) and the knot search table are read from
-    // global memory through the L1 cache, not LDS, by the LEAN kernels and by
-    // the FP32 recompute kernels, whose re-simulation otherwise loads the LDS
-    // most (measured: C3 FP32 recompute 0.719 -> 0.643 ms).  The other FP32
-    // Dupire kernels but the book's, bound by the LDS pipe, read the
-    // inverse-normal table through L1: a step's six LDS reads take 28 cycles
-    // of the pipe and 15 more of bank conflicts, as many as its vector
-    // instructions.  (Pricing 2^19 paths x 156 steps 0.131 -> 0.116 ms, C3 risk
-    // 0.587 -> 0.576 ms; with the knot search table as well they lose: the
-    // vector memory path saturates instead)
-    constexpr bool GTAB = LEAN || (RECOMP && sizeof(R) == 4);
-    constexpr bool GINV = GTAB || (sizeof(R) == 4 && DUP && !BOOK && ADJ != ADJ_RECOMPUTE);
+    // The inverse-normal table (FP32) and the knot search table are read from
+    // global memory through the L1 cache, not LDS, by the LEAN kernels.  The
+    // FP32 recompute kernels and the FP32 Dupire kernels but the book's, bound
+    // by the LDS pipe, read the inverse-normal table through L1, the widest of
+    // a step's LDS reads and the one with the most bank conflicts.  (Pricing
+    // 2^19 paths x 156 steps 0.131 -> 0.116 ms, C3 risk 0.587 -> 0.576 ms; with
+    // the knot search table as well the vector memory path saturates instead.)
+    constexpr bool GINV = LEAN || (sizeof(R) == 4 && (RECOMP || (DUP && !BOOK)));
 
-    // Sobol LO layout: the FP32 Dupire adjoint kernels other than the book
-    // read four dimensions at once (quads); the others one at a time (rows)
-    constexpr bool QUADS = sizeof(R) == 4 && AD && DUP && !BOOK && !LEAN && !MRG;
+    // Sobol LO layout: the FP32 Dupire kernels other than the book read four
+    // dimensions at once (quads), FP64 ones too (split); the others one at a
+    // time (rows)
+    constexpr bool QUADS = sizeof(R) == 4 && DUP && !BOOK && !LEAN && !MRG;
     constexpr int LOL = LEAN ? kLoLean : SPLIT ? kLoSplit : (QUADS ? kLoQuads : kLoRows);
     // ---- stage the block's tables in LDS
     sobol_stage_lo<LOL>(lo_tab, P.dirs, n, tid, nthr);
@@ -802,8 +795,12 @@ __device__ __forceinline__ void path_body(const LaunchParams& P, const int bid, 
         const R* gi = static_cast<const R*>(P.inv_dx);
         const R* gv = static_cast<const R*>(P.iv);
         for (int e = tid; e <= m; e += nthr) { kxi[2 * e] = gk[e]; kxi[2 * e + 1] = gi[e]; }
-        if constexpr (!GTAB)
-            for (int e = tid; e < P.n_buckets; e += nthr) bucket[e] = static_cast<const BucketEntry<R>*>(P.bucket)[e];
+        if constexpr (!LEAN)
+            for (int e = tid; e < P.n_buckets; e += nthr) {
+                const BucketEntry<R>& b = static_cast<const BucketEntry<R>*>(P.bucket)[e];
+                bucket[e].k0 = b.k0;
+                bucket[e].lo = b.lo;
+            }
         if constexpr (!LEAN)
             for (int e = tid; e < n * mp; e += nthr) iv_lds[e] = gv[e];
     } else {
@@ -882,13 +879,26 @@ __device__ __forceinline__ void path_body(const LaunchParams& P, const int bid, 
     KnotSearch<R> ks;
     ks.knots = kxi + 2;     // the knots themselves: interval starts from interval 1
     ks.stride = 2;
-    if constexpr (GTAB) ks.table = static_cast<const BucketEntry<R>*>(P.bucket); else ks.table = bucket;
+    ks.table = static_cast<const BucketEntry<R>*>(P.bucket);
     ks.m = m;
     ks.fix = P.bucket_fix;
     ks.invh = R(P.bucket_invh);
     ks.c0 = R(P.bucket_c0);
     ks.top = R(P.n_buckets - 1);
     ks.itop = P.n_buckets - 1;
+    // number of knots <= x.  FP32: the entry's address straight from the
+    // bucket's bits
+    const uint32_t bucket_at = uint32_t(L.bucket) - (kBucketMagicBits << 3);
+    auto knot_count = [&](R x) -> int {
+        if constexpr (LEAN) {
+            return count_le<true>(ks, x);
+        } else if constexpr (sizeof(R) == 4) {
+            const uint32_t off = (bucket_bits(x, ks.invh, ks.c0, ks.top) << 3) + bucket_at;
+            return count_le_one(*reinterpret_cast<const BucketOne<R>*>(smem + off), x);
+        } else {
+            return count_le_one(bucket[bucket_index(x, ks.invh, ks.c0, ks.top, ks.itop)], x);
+        }
+    };
     const double s0 = P.spot;
     const int last = ns - 1;
 
@@ -1325,6 +1335,7 @@ __device__ __forceinline__ void path_body(const LaunchParams& P, const int bid, 
             uint32_t glo = 0;
             R gz[4];          // QW: the group's four normals, drawn before its steps
             uint64_t fbits = 0;   // UNDER: bit b, point 64 (i >> 6) + 1 + b is a sample
+            uint64_t open = UNDER ? ~__builtin_amdgcn_ballot_w64(ps.dead) : 0;   // the lanes not breached
             auto fwd_step = [&](int i0, int k, auto grp, auto qw) {
                 constexpr bool GRP = decltype(grp)::value, QW = decltype(qw)::value;
                 const int i = i0 + k;
@@ -1340,7 +1351,7 @@ __device__ __forceinline__ void path_body(const LaunchParams& P, const int bid, 
                     else if constexpr (ADJ == ADJ_CHECKPOINT) (ck + i0 * kWave + lane)[k * kWave] = x;
                     if constexpr (RECOMP)
                         if ((i & (kSeg - 1)) == 0) ck[(i / kSeg) * kWave + lane] = x;
-                    const int lo = count_le<LEAN>(ks, x);
+                    const int lo = knot_count(x);
                     if constexpr (GRP) glo |= uint32_t(lo) << (8 * k);
                     else if constexpr (IL) { if (ck_lo) ckl[ck_el(i)] = uint8_t(lo); }
                     else if constexpr (CKB) { if (ck_lo) (ckl + i0 * kWave + lane)[k * kWave] = uint8_t(lo); }
@@ -1355,8 +1366,10 @@ __device__ __forceinline__ void path_body(const LaunchParams& P, const int bid, 
                 if constexpr (UNDER) {
                     // (a group of four steps lies in one window of 64)
                     if ((QW ? k == 0 : true) && (i & 63) == 0) fbits = sample_bits(i + 1);
-                    if (((fbits >> (i & 63)) & 1u) && __builtin_amdgcn_ballot_w64(x > x_lo && !ps.dead) != 0)
+                    if (((fbits >> (i & 63)) & 1u) && (__builtin_amdgcn_ballot_w64(x > x_lo) & open) != 0) {
                         observe(0, zone_spot(x), SampleRow{});
+                        open = ~__builtin_amdgcn_ballot_w64(ps.dead);
+                    }
                 } else if constexpr (BOOK && DUP) {
                     // (a plain barrier sample changes nothing while every state
                     // is under the zones)
@@ -1368,9 +1381,14 @@ __device__ __forceinline__ void path_body(const LaunchParams& P, const int bid, 
                     if (s >= 0) observe(s, DUP ? state_spot(x, s0) : x, row_of(s, 0));
                 }
             };
-            // FP32 Dupire adjoint kernels other than the book: groups of four steps
-            // (the book's sample code, four times over, and FP64 measured slower)
-            constexpr int UF = AD && DUP && !BOOK && sizeof(R) == 4 ? 4 : 1;
+            // FP32 Dupire kernels other than the book: groups of four steps,
+            // their Sobol words in two 16-byte reads and their four normals
+            // drawn side by side (the book's sample code, four times over, and
+            // FP64 measured slower).  A step is 25 vector instructions and five
+            // LDS reads, from 33 and six; pricing 2^19 paths x 156 steps 0.116 ->
+            // 0.101 ms, 2^20 paths' risk 0.379 -> 0.363, recompute 0.557 -> 0.395
+            // (its knot search from LDS, the entry half as wide).
+            constexpr int UF = DUP && !BOOK && sizeof(R) == 4 ? 4 : 1;
             int i = 0;
             if constexpr (UF > 1) {
                 // (UF = 4 kernels with interleaved checkpoints: one 16-byte
@@ -1919,7 +1937,7 @@ __device__ __forceinline__ void path_body(const LaunchParams& P, const int bid, 
                         if constexpr (QUADS) g = inv_normal(sw[k], invn_tab);
                         else if constexpr (MRG || sizeof(R) == 8) g = mz[k];
                         else g = draw(i);
-                        const Bracket<R> b = local_vol<LEAN>(ks, kxi, iv + i * mp, xi);
+                        const Bracket<R> b = local_vol_at(kxi, iv + i * mp, xi, knot_count(xi));
                         const R ws = g - b.vol;    // d x_{i+1} / d vol
                         ca[k] = R(1) + ws * b.slope;
                         cw[k] = ws * b.wa;
@@ -2048,7 +2066,7 @@ __device__ __forceinline__ void path_body(const LaunchParams& P, const int bid, 
                         js[k] = 0;
                         if (PART && i >= n) continue;
                         const R xi = buf[k];
-                        const int lo = ck_lo ? lbuf[k] : count_le<LEAN>(ks, xi);
+                        const int lo = ck_lo ? lbuf[k] : knot_count(xi);
                         const Bracket<R> b = local_vol_at(kxi, iv + i * mp, xi, lo);
                         // d x_{i+1} / d vol = g - vol, recovered from the two states:
                         // x_{i+1} - x_i = vol (g - vol / 2) up to the rounding of
@@ -2127,7 +2145,7 @@ __device__ __forceinline__ void path_body(const LaunchParams& P, const int bid, 
                             const SampleRow row = prow;
                             if constexpr (BOOK) prow = bk_rows(max(i - 1, 0));
                             const bool on = BOOK ? (row.bars | row.grps) != 0 || row.van_hi > row.van_lo : smp >= 0;
-                            if (!ck_lo) lo = count_le<LEAN>(ks, xi);
+                            if (!ck_lo) lo = knot_count(xi);
                             const Bracket<R> b = local_vol_at(kxi, iv + i * mp, xi, lo);
                             R ws = recip_mul(xnext - xi, b.vol) - R(0.5) * b.vol;
                             if constexpr (!REC)
