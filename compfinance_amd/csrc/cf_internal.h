@@ -478,7 +478,9 @@ CF_HD inline SmemLayout smem_layout(int n_steps, int n_spots, int n_samples, int
     L.invn = o;        o = cf_align16(o + (real_bytes == 4 && !lean ? size_t(kInvNormalRows) * 4 * 4 : 0));
     // interval (start, inverse width) pairs, interleaved
     L.knots = o;       o = cf_align16(o + (dupire ? size_t(2 * (n_spots + 1)) * real_bytes : 0));
-    L.bucket = o;      o = cf_align16(o + (dupire && !lean ? size_t(n_buckets) * size_t(2 * real_bytes) : 0));
+    L.bucket = o;      o = cf_align16(o + (dupire && !lean ? size_t(n_buckets) * (real_bytes == 4 ? sizeof(BucketEntry<float>)
+                                                                                            : sizeof(BucketEntry<double>))
+                                                           : 0));
     L.iv = o;          o = cf_align16(o + (dupire && !lean ? size_t(n_steps) * lv_cols(n_spots) * real_bytes : 0));
     L.drift = o;       o = cf_align16(o + (dupire ? 0 : size_t(n_steps) * real_bytes));
     L.stdv = o;        o = cf_align16(o + (dupire ? 0 : size_t(n_steps) * real_bytes));
