@@ -713,6 +713,8 @@ Engine& engine()
         // into the library's module variable: creating the engine allocates no device memory
         const int rc = cfk::upload_sobol_dirs(dirs.data(), &e->d_dirs);
         if (rc != 0) hip_check(hipError_t(rc), "direction numbers");
+        const int rd = cfk::blocks_done_counter(&e->d_blocks_done);
+        if (rd != 0) hip_check(hipError_t(rd), "block counter");
         slot = std::move(e);
     }
     return *slot;
@@ -1196,6 +1198,7 @@ void enqueue_sequence(const Sequence& q, hipStream_t stream, hipEvent_t ev_kerne
     int rc = cfk::launch_path_kernel(q.cfg, q.P, q.grid, q.block, q.smem, stream);
     if (rc != 0) hip_check(hipError_t(rc), "path kernel launch");
     if (ev_kernel1) hip_check(hipEventRecord(ev_kernel1, stream), "hipEventRecord");
+    if (q.P.blocks_done) return;   // summed by the kernel's last block
     rc = cfk::launch_reduce_rows(q.block_out, q.stride, q.reduced, q.ivbar_blocks, int(q.ivn), q.ivbar, q.grid,
                                  stream);
     if (rc != 0) hip_check(hipError_t(rc), "reduce launch");
@@ -1309,9 +1312,16 @@ int run(const cf_model* mdl, const cf_product* prd, Call& c)
             E.weights_on_device = B.weights;
         }
     }
-    const cfk::LaunchParams P = launch_params(E, PR, S, B);
+    cfk::LaunchParams P = launch_params(E, PR, S, B);
+    const bool fused = cfk::fused_reduction(S.npay, c.adjoint, PR.md.kind == CF_MODEL_DUPIRE);
+    if (fused) {
+        P.blocks_done = E.d_blocks_done;
+        P.reduced = B.reduced;
+    }
+    // (a fused pricing call is one kernel: the first and last event bound it)
+    const bool one = fused && !c.adjoint;
     const double setup_ms = ms_since(t_start);
-    enqueue_call(PR, S, B, P, E.stream, E.ev[1], E.ev[2]);
+    enqueue_call(PR, S, B, P, E.stream, one ? nullptr : E.ev[1], one ? nullptr : E.ev[2]);
     hip_check(hipEventRecord(E.ev[3], E.stream), "hipEventRecord");
 
     if (B.per_path)
@@ -1325,9 +1335,13 @@ int run(const cf_model* mdl, const cf_product* prd, Call& c)
     const double waited_ms = ms_since(t_start);
 
     float t_main = 0, t_red = 0, t_all = 0;
-    hip_check(hipEventElapsedTime(&t_main, E.ev[1], E.ev[2]), "event");
-    hip_check(hipEventElapsedTime(&t_red, E.ev[2], E.ev[3]), "event");
     hip_check(hipEventElapsedTime(&t_all, E.ev[0], E.ev[3]), "event");
+    if (one) {
+        t_main = t_all;
+    } else {
+        hip_check(hipEventElapsedTime(&t_main, E.ev[1], E.ev[2]), "event");
+        hip_check(hipEventElapsedTime(&t_red, E.ev[2], E.ev[3]), "event");
+    }
 
     collect_results(PR, S, h_out, h_out + S.stride, c);
 

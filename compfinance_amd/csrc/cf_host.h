@@ -234,6 +234,7 @@ struct Engine {
     hipStream_t stream = nullptr;
     hipEvent_t ev[4] = {};
     uint32_t* d_dirs = nullptr;
+    uint32_t* d_blocks_done = nullptr;
     DevBuf block_out, ivbar_blocks, reduced, per_path, per_path_agg, ckpt, weights;
     PinnedBuf pin_in, pin_out;
     // itemized risk: checkpoints, lists and grids of one call, kept between

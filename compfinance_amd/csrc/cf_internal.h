@@ -200,7 +200,21 @@ struct LaunchParams {
                                  // itemized risk: the one payoff's last observation)
     void* state;                 // [blocks of 64 paths][state_rows(product)][64] reals
     int ck_slots;                // checkpoint slots of a wave, at least 1 (kMaxCkSlots)
+    // cross-block sums by the kernel's last block (fused_reduction): the count
+    // of blocks done, 0 between launches, or null; and the sums
+    uint32_t* blocks_done;
+    double* reduced;
 };
+
+// Calls whose last block sums the other blocks' rows itself: those without a
+// local-vol grid to sum and of few columns.  A second launch and its gap take
+// some 9 us; a wave of the last block sums a column in one.
+constexpr int kMaxFusedCols = 16;
+CF_HD inline int fused_cols(int n_pay, bool adjoint) { return adjoint ? out_stride(n_pay) : 2 * n_pay; }
+CF_HD inline bool fused_reduction(int n_pay, bool adjoint, bool dupire)
+{
+    return !(adjoint && dupire) && fused_cols(n_pay, adjoint) <= kMaxFusedCols;
+}
 
 // Calls packed into one launch of a path kernel: call r runs on blocks
 // [first[r], first[r + 1]).  Passed by value (kernel arguments stay under
@@ -216,7 +230,7 @@ struct PackArgs {
     int first[kMaxPack + 1];
     int n;
 };
-static_assert(sizeof(PackArgs) <= 3584, "packed kernel arguments");
+static_assert(sizeof(PackArgs) <= 3712, "packed kernel arguments");
 
 // The cross-block reductions of the calls of a packed launch, one launch:
 // call r's column sums run on blocks [first[r], first[r + 1]).
@@ -612,6 +626,9 @@ int launch_reduce_rows(const double* in0, int cols0, double* out0, const double*
                        int rows, void* stream);
 // A packed launch (cfg.packed: Sobol, not itemized) of A.n calls over grid =
 // A.first[A.n] blocks, and the calls' reductions in one launch.
+// The engine's count of blocks done (LaunchParams::blocks_done) on the current
+// device, a module variable.
+int blocks_done_counter(uint32_t** device);
 int launch_path_kernel_packed(const KernelConfig& cfg, const PackArgs& A, int block, size_t smem, void* stream);
 int launch_reduce_packed(const ReducePack& R, void* stream);
 int path_kernel_occupancy(const KernelConfig& cfg, int block, size_t smem, int* blocks_per_cu);

@@ -80,6 +80,17 @@ int upload_sobol_dirs(const uint32_t* host, uint32_t** device)
     return 0;
 }
 
+// Blocks done of the synchronous calls' kernel in flight (one at a time)
+__device__ uint32_t g_blocks_done;
+
+int blocks_done_counter(uint32_t** device)
+{
+    void* p = nullptr;
+    const hipError_t e = hipGetSymbolAddress(&p, HIP_SYMBOL(g_blocks_done));
+    *device = static_cast<uint32_t*>(p);
+    return int(e);
+}
+
 // ------------------------------------------------------------------ Sobol points
 
 // Words and normals of paths [first, first + npath) in dim dimensions, formed

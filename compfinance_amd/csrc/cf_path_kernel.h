@@ -2338,7 +2338,41 @@ __device__ __forceinline__ void path_body(const LaunchParams& P, const int bid, 
     for (int c = tid; c < stride; c += nthr) {
         double s = 0.0;
         for (int w = 0; w < waves; ++w) s += acc[w * stride + c];
-        P.block_out[size_t(bid) * stride + c] = s;
+        // (through to the memory that all caches share: see below)
+        __hip_atomic_store(P.block_out + size_t(bid) * stride + c, s, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+    if constexpr (!(AD && DUP)) {
+        // the last block to get here sums the rows, in the order in which the
+        // reduction kernel sums them (phase l of rows l, l + 64, ..., then the
+        // phases), so the result does not depend on which block it is.  The
+        // rows' stores and loads bypass the caches that are not shared and are
+        // waited for, which orders them; a device-wide fence in each wave
+        // instead writes back and drops its L2 (2^19 paths: 100 us more).
+        if (P.blocks_done) {
+            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+            __syncthreads();
+            int* is_last = reinterpret_cast<int*>(smem);   // (the tables are done with)
+            if (tid == 0) *is_last = atomicInc(P.blocks_done, unsigned(nblk - 1)) == unsigned(nblk - 1) ? 1 : 0;
+            __syncthreads();
+            if (*is_last) {
+                const int cols = fused_cols(npay, AD);
+                for (int c = wave; c < cols; c += waves) {
+                    double s = 0.0;
+                    for (int r = lane; r < nblk; r += kWave) 
+                        s += __hip_atomic_load(P.block_out + size_t(r) * stride + c, __ATOMIC_RELAXED,
+                                               __HIP_MEMORY_SCOPE_AGENT);
+                    const uint64_t b = __builtin_bit_cast(uint64_t, s);
+                    double t = 0.0;
+#pragma unroll 16
+                    for (int k = 0; k < kWave; ++k) {
+                        const uint32_t lo = __builtin_amdgcn_readlane(uint32_t(b), k);
+                        const uint32_t hi = __builtin_amdgcn_readlane(uint32_t(b >> 32), k);
+                        t += __builtin_bit_cast(double, uint64_t(hi) << 32 | lo);
+                    }
+                    if (lane == 0) P.reduced[c] = t;
+                }
+            }
+        }
     }
     if constexpr (AD && DUP) {
         double* dst = P.ivbar_blocks + size_t(bid) * n * m;
