@@ -394,16 +394,9 @@ BookTables build_book(const ProductPlan& d, double width0)
     };
     vector<vector<std::pair<double, int>>> van(ns);
     vector<uint32_t> bar_mask(ns, 0u), bar_last(ns, 0u), grp_mask(ns, 0u), grp_last(ns, 0u);
-    // the barriers take their places in order of the lower end B - w of their
-    // zone: the kernels stop at the first zone no path has reached
-    vector<double> bar_lo;
-    for (const ProductPlan* q : parts)
-        if (q->kind == CF_PRODUCT_BARRIER) bar_lo.push_back(q->barrier - width0 * q->smooth);
-    vector<int> bar_place(bar_lo.size());
-    for (size_t i = 0; i < bar_lo.size(); ++i)
-        for (size_t j = 0; j < bar_lo.size(); ++j)
-            if (bar_lo[j] < bar_lo[i] || (bar_lo[j] == bar_lo[i] && j < i)) ++bar_place[i];
-    const size_t n_bars = bar_lo.size();
+    const size_t n_bars = size_t(std::count_if(parts.begin(), parts.end(), [](const ProductPlan* q) {
+        return q->kind == CF_PRODUCT_BARRIER;
+    }));
     if (n_bars > size_t(cfk::kMaxBookBarriers))
         fail(CF_ERR_CAPACITY, "a book holds at most " + std::to_string(cfk::kMaxBookBarriers) + " barriers");
     size_t bars_seen = 0;
@@ -419,7 +412,7 @@ BookTables build_book(const ProductPlan& d, double width0)
             for (size_t i = 0; i < q->mats.size(); ++i)
                 for (double k : q->strikes[i]) van[at(q->mats[i])].push_back({k, col++});
         } else if (q->kind == CF_PRODUCT_BARRIER) {
-            const size_t b = size_t(bar_place[bars_seen++]);
+            const size_t b = bars_seen++;
             for (double t : q->timeline) bar_mask[at(t)] |= 1u << b;
             bar_last[at(q->timeline.back())] |= 1u << b;
             const double w = width0 * q->smooth;
@@ -508,6 +501,7 @@ BookTables build_book(const ProductPlan& d, double width0)
             p[4 + j] = bar_par[4 * (b + j) + 1];
             p[8 + j] = bar_par[4 * (b + j) + 3];
         }
+        p[12] = *std::min_element(p, p + 4);
         pars.insert(pars.end(), p, p + 16);
     }
     L.bar_par = put(pars.data(), pars.size() * 8);

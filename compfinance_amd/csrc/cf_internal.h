@@ -65,9 +65,9 @@ struct BookLayout {
                       // and maturing at s (16-31), schedules fixing at s (bits 0-3) and ending
                       // at s (4-7) with kBookAllBars and kBookPlain, first vanilla of s, first
                       // vanilla of s + 1
-    int bar_par;      // [n_bar][4] double: strike, B + w, B - w, 1 / 2w, in order of B - w; then
+    int bar_par;      // [n_bar][4] double: strike, B + w, B - w, 1 / 2w; then
                       // [kMaxBookBarriers / 4][16]: the same by fours (four B - w, four B + w,
-                      // four 1 / 2w, four unused), +infinity past the last barrier
+                      // four 1 / 2w, the lowest B - w), +infinity past the last barrier
     int bar_par_f;    // the same in float
     int bar_col;      // [n_bar] int: column of the barrier payoff (vanilla next)
     int bar_put;      // [n_bar] int

@@ -980,9 +980,10 @@ __device__ __forceinline__ void path_body(const LaunchParams& P, const int bid, 
         return r;
     };
     // barriers by fours, in the kernel's precision, past the last one at
-    // +infinity: the lower ends of their zones, B + w, 1 / 2w
+    // +infinity: the lower ends of their zones, B + w, 1 / 2w, and the lowest
+    // of the lower ends
     struct alignas(16) BarFour {
-        R lo[4], up[4], i2s[4], pad[4];
+        R lo[4], up[4], i2s[4], lo_min[4];
     };
     CPtr<BarFour> bk_four_c =
         cptr<BarFour>(bkb + (sizeof(R) == 4 ? P.bk.bar_par_f + P.bk.n_bar * 16 : P.bk.bar_par + P.bk.n_bar * 32));
@@ -1187,7 +1188,7 @@ __device__ __forceinline__ void path_body(const LaunchParams& P, const int bid, 
                 if (all_bars) {
 #pragma unroll
                     for (int b = 0; b + 3 < NBAR; b += 4) {
-                        if (__builtin_amdgcn_ballot_w64(F > bk_four_c[b >> 2].lo[0]) == 0) continue;
+                        if (__builtin_amdgcn_ballot_w64(F > bk_four_c[b >> 2].lo_min[0]) == 0) continue;
                         R up[4], i2s[4];
 #pragma unroll
                         for (int j = 0; j < 4; ++j) {
@@ -1816,14 +1817,15 @@ __device__ __forceinline__ void path_body(const LaunchParams& P, const int bid, 
                                 // weight x survival factor (FP64: from the
                                 // weighted vanilla times the state, where the
                                 // vanilla is 0 it does not matter)
-                                R wa;
+                                // (FP32: one expression, one rounding)
+                                R euro_bar;
                                 if constexpr (ZT) {
                                     const R euro = intrinsic / numv;
-                                    wa = euro != R(0) && !(fabs(bst[b]) > R(kZeroMark)) ? bst[b] / euro : R(0);
+                                    const R wa = euro != R(0) && !(fabs(bst[b]) > R(kZeroMark)) ? bst[b] / euro : R(0);
+                                    euro_bar = wa + R(wts[col + 1]);
                                 } else {
-                                    wa = R(wts[col]) * bar_alive(bst[b]);
+                                    euro_bar = R(wts[col]) * bar_alive(bst[b]) + R(wts[col + 1]);
                                 }
-                                const R euro_bar = wa + R(wts[col + 1]);
                                 Fb += euro_bar * dmax / numv;
                                 nb += -euro_bar * (intrinsic / numv) / numv;
                             }
