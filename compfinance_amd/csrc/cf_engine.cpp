@@ -865,7 +865,8 @@ std::shared_ptr<Prepared> prepare(Engine& E, const cf_model* mdl, const cf_produ
     auto lds_bytes = [&](int copies) {
         return cfk::smem_layout(md.n_steps, md.n_spots, int(pd.timeline.size()), pd.n_pay, waves, fp64 ? 8 : 4, dup,
                                 pd.kind == CF_PRODUCT_EUROPEANS, adjoint, P->cfg.lean, dup ? P->bt.nb : 0, copies,
-                                cfk::split_layout(fp64 ? 8 : 4, dup, adjoint, P->cfg.lean))
+                                cfk::split_layout(fp64 ? 8 : 4, dup, adjoint, P->cfg.lean),
+                                cfk::bs_row_layout(dup, P->cfg.product, P->cfg.lean))
             .total;
     };
     P->ivbar_copies = 1;

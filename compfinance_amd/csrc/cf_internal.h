@@ -246,7 +246,7 @@ struct ReducePack {
 
 // Shared-memory carve of one block.  Offsets in bytes, 16-byte aligned.
 struct SmemLayout {
-    size_t lo, mtab, hi, hi_tail, step_sample, invn, knots, bucket, iv, drift, stdv, samples, pay_first, pay_strike, acc,
+    size_t lo, mtab, hi, hi_tail, step_sample, invn, knots, bucket, iv, drift, stdv, bs, samples, pay_first, pay_strike, acc,
         tails, ivbar, total;
 };
 
@@ -472,13 +472,19 @@ CF_HD inline int lv_cols(int n_spots) { return n_spots + 2; }
 constexpr int kIvbarCopyPad = 8;
 CF_HD inline int ivbar_copy_stride(int n_steps, int n_spots) { return n_steps * lv_cols(n_spots) + kIvbarCopyPad; }
 
+// The FULL Black-Scholes barrier kernels hold a step's numbers together, in
+// the kernel's precision: (drift, std, forward factor of its sample or NaN, 0)
+// and, for the tangents, (vol term, sqrt(dt), dt, 0).
+CF_HD constexpr bool bs_row_layout(bool dupire, int product, bool lean) { return !dupire && product == PRD_BARRIER && !lean; }
+CF_HD constexpr int bs_row_reals(bool adjoint) { return adjoint ? 8 : 4; }
+
 CF_HD constexpr bool split_layout(int real_bytes, bool dupire, bool adjoint, bool lean)
 {
     return real_bytes == 8 && dupire && adjoint && !lean;
 }
 CF_HD inline SmemLayout smem_layout(int n_steps, int n_spots, int n_samples, int n_pay, int waves,
                                     int real_bytes, bool dupire, bool europeans, bool adjoint, bool lean,
-                                    int n_buckets, int ivbar_copies, bool split = false)
+                                    int n_buckets, int ivbar_copies, bool split = false, bool bs_rows = false)
 {
     SmemLayout L{};
     size_t o = 0;
@@ -496,8 +502,9 @@ CF_HD inline SmemLayout smem_layout(int n_steps, int n_spots, int n_samples, int
                                                                                             : sizeof(BucketEntry<double>))
                                                            : 0));
     L.iv = o;          o = cf_align16(o + (dupire && !lean ? size_t(n_steps) * lv_cols(n_spots) * real_bytes : 0));
-    L.drift = o;       o = cf_align16(o + (dupire ? 0 : size_t(n_steps) * real_bytes));
-    L.stdv = o;        o = cf_align16(o + (dupire ? 0 : size_t(n_steps) * real_bytes));
+    L.drift = o;       o = cf_align16(o + (dupire || bs_rows ? 0 : size_t(n_steps) * real_bytes));
+    L.stdv = o;        o = cf_align16(o + (dupire || bs_rows ? 0 : size_t(n_steps) * real_bytes));
+    L.bs = o;          o = cf_align16(o + (bs_rows ? size_t(n_steps) * bs_row_reals(adjoint) * real_bytes : 0));
     L.samples = o;     o = cf_align16(o + (dupire ? 0 : size_t(n_samples) * 3 * 8));
     L.pay_first = o;   o = cf_align16(o + (europeans ? size_t(n_samples + 1) * 4 : 0));
     L.pay_strike = o;  o = cf_align16(o + (europeans ? size_t(n_pay) * 8 : 0));

@@ -769,8 +769,9 @@ __device__ __forceinline__ void path_body(const LaunchParams& P, const int bid, 
     const int stride = out_stride(npay);
     constexpr bool BOOK = PRD == PRD_BOOK;
     constexpr bool SPLIT = split_layout(int(sizeof(R)), DUP, AD, LEAN);
+    constexpr bool BSR = bs_row_layout(DUP, PRD, LEAN);
     const SmemLayout L = smem_layout(n, m, ns, npay, waves, int(sizeof(R)), DUP, EUS, AD, LEAN, P.n_buckets,
-                                     P.ivbar_copies, SPLIT);
+                                     P.ivbar_copies, SPLIT, BSR);
 
     uint32_t* lo_tab = reinterpret_cast<uint32_t*>(smem + L.lo);
     uint32_t* hi_all = reinterpret_cast<uint32_t*>(smem + L.hi);
@@ -780,6 +781,8 @@ __device__ __forceinline__ void path_body(const LaunchParams& P, const int bid, 
     R* iv_lds = reinterpret_cast<R*>(smem + L.iv);
     R* drift = reinterpret_cast<R*>(smem + L.drift);
     R* stdv = reinterpret_cast<R*>(smem + L.stdv);
+    constexpr int kBsReals = bs_row_reals(AD);
+    R* bsr = reinterpret_cast<R*>(smem + L.bs);      // BSR: [n][kBsReals]
     double* s_ff = reinterpret_cast<double*>(smem + L.samples);
     double* s_disc = s_ff + ns;
     double* s_num = s_disc + ns;
@@ -801,10 +804,10 @@ __device__ __forceinline__ void path_body(const LaunchParams& P, const int bid, 
     // the knot search table as well the vector memory path saturates instead.)
     constexpr bool GINV = LEAN || (sizeof(R) == 4 && (RECOMP || (DUP && !BOOK)));
 
-    // Sobol LO layout: the FP32 Dupire kernels other than the book read four
-    // dimensions at once (quads), FP64 ones too (split); the others one at a
+    // Sobol LO layout: the FP32 Dupire kernels other than the book and the FP32
+    // Black-Scholes barrier read four dimensions at once (quads), FP64 ones too (split); the others one at a
     // time (rows)
-    constexpr bool QUADS = sizeof(R) == 4 && DUP && !BOOK && !LEAN && !MRG;
+    constexpr bool QUADS = sizeof(R) == 4 && ((DUP && !BOOK && !LEAN) || BSR) && !MRG;
     constexpr int LOL = LEAN ? kLoLean : SPLIT ? kLoSplit : (QUADS ? kLoQuads : kLoRows);
     // ---- stage the block's tables in LDS
     if constexpr (!MRG) sobol_stage_lo<LOL>(lo_tab, P.dirs, n, tid, nthr);
@@ -830,7 +833,23 @@ __device__ __forceinline__ void path_body(const LaunchParams& P, const int bid, 
     } else {
         const R* gd = static_cast<const R*>(P.drift);
         const R* gs = static_cast<const R*>(P.stdv);
-        for (int e = tid; e < n; e += nthr) { drift[e] = gd[e]; stdv[e] = gs[e]; }
+        if constexpr (BSR) {
+            const double* dt = P.bs_aux + 3 * ns;
+            for (int e = tid; e < n; e += nthr) {
+                const int s = P.step_sample[e + 1];
+                bsr[e * kBsReals] = gd[e];
+                bsr[e * kBsReals + 1] = gs[e];
+                bsr[e * kBsReals + 2] = s >= 0 ? R(P.ff[s]) : R(NAN);
+                if constexpr (AD) {
+                    const R dti = R(dt[e]), vol = R(P.bs_vol);
+                    bsr[e * kBsReals + 4] = P.spot_measure ? vol * dti : -vol * dti;
+                    bsr[e * kBsReals + 5] = R(sqrt(dt[e]));
+                    bsr[e * kBsReals + 6] = dti;
+                }
+            }
+        } else {
+            for (int e = tid; e < n; e += nthr) { drift[e] = gd[e]; stdv[e] = gs[e]; }
+        }
         for (int e = tid; e < ns; e += nthr) { s_ff[e] = P.ff[e]; s_disc[e] = P.disc[e]; s_num[e] = P.num[e]; }
     }
     if constexpr (EUS) {
@@ -1360,7 +1379,7 @@ __device__ __forceinline__ void path_body(const LaunchParams& P, const int bid, 
             uint32_t glo = 0;
             R gz[4];          // QW: the group's four normals, drawn before its steps
             uint64_t fbits = 0;   // UNDER: bit b, point 64 (i >> 6) + 1 + b is a sample
-            uint64_t open = UNDER ? ~__builtin_amdgcn_ballot_w64(ps.dead) : 0;   // the lanes not breached
+            uint64_t open = UNDER || BSR ? ~__builtin_amdgcn_ballot_w64(ps.dead) : 0;   // the lanes not breached
             auto fwd_step = [&](int i0, int k, auto grp, auto qw) {
                 constexpr bool GRP = decltype(grp)::value, QW = decltype(qw)::value;
                 const int i = i0 + k;
@@ -1384,7 +1403,20 @@ __device__ __forceinline__ void path_body(const LaunchParams& P, const int bid, 
                     x = euler_step(x, b.vol, g);
                 } else {
                     if constexpr (ADJ == ADJ_CHECKPOINT) ck[i * kWave + lane] = g;
-                    x = x * rexp(drift[i] + stdv[i] * g);      // mcMdlBS.h:344-345
+                    if constexpr (BSR) {
+                        const R* r = bsr + i0 * kBsReals + k * kBsReals;
+                        x = x * rexp(r[0] + r[1] * g);         // mcMdlBS.h:344-345
+                        // (as for Dupire: a sample other than the last one
+                        // changes nothing on a path under the zone or breached)
+                        const R F = x * r[2];
+                        if ((__builtin_amdgcn_ballot_w64(F > R(P.minus_smooth)) & open) != 0) {
+                            observe(__builtin_amdgcn_readfirstlane((step_sample + i0 + 1)[k]), x, row);
+                            open = ~__builtin_amdgcn_ballot_w64(ps.dead);
+                        }
+                        return;
+                    } else {
+                        x = x * rexp(drift[i] + stdv[i] * g);
+                    }
                 }
                 // a wave-uniform test: the sample's code runs with all lanes (a lane
                 // under the zone changes nothing there)
@@ -1413,7 +1445,7 @@ __device__ __forceinline__ void path_body(const LaunchParams& P, const int bid, 
             // LDS reads, from 33 and six; pricing 2^19 paths x 156 steps 0.116 ->
             // 0.101 ms, 2^20 paths' risk 0.379 -> 0.363, recompute 0.557 -> 0.395
             // (its knot search from LDS, the entry half as wide).
-            constexpr int UF = DUP && !BOOK && sizeof(R) == 4 ? 4 : 1;
+            constexpr int UF = ((DUP && !BOOK) || BSR) && sizeof(R) == 4 ? 4 : 1;
             int i = 0;
             if constexpr (UF > 1) {
                 // (UF = 4 kernels with interleaved checkpoints: one 16-byte
@@ -1616,8 +1648,8 @@ __device__ __forceinline__ void path_body(const LaunchParams& P, const int bid, 
             // 0.53 -> 0.38 ms, FP64 0.92 -> 0.80, FP32 recompute 0.63 -> 0.56).
             // (A state or weight out of range is not left out.)
             bool live = active;
-            if constexpr (DUP && (PRD == PRD_BARRIER || PRD == PRD_EUROPEAN)) {
-                const R F = state_spot(x, s0), k = R(P.strike);
+            if constexpr ((DUP && (PRD == PRD_BARRIER || PRD == PRD_EUROPEAN)) || BSR) {
+                const R F = DUP ? state_spot(x, s0) : ps.fin_f, k = R(P.strike);
                 const bool in = PRD == PRD_BARRIER && P.put ? k > F : F > k;
                 const bool zero = PRD == PRD_EUROPEAN ? ns == 1 && !in : !in || (ps.dead && w1 == R(0));
                 live = active && !(zero && x - x == R(0) && F - F == R(0) && w0 - w0 == R(0));
@@ -2303,7 +2335,7 @@ __device__ __forceinline__ void path_body(const LaunchParams& P, const int bid, 
                     } else {
                         dN[0] = R(0); dN[1] = R(0); dN[2] = numv * ts; dN[3] = R(0);
                     }
-                    if (active)
+                    if (live)
                         for (int c = 0; c < 4; ++c) padj[c] += double(Fb * dF[c] + db * dD[c] + nb * dN[c]);
                 };
                 {
@@ -2311,6 +2343,50 @@ __device__ __forceinline__ void path_body(const LaunchParams& P, const int bid, 
                     if (s >= 0) accumulate(s, spot);
                 }
                 const int nrev = min(n, P.rev_point);   // samples after it carry no weight
+                // barrier: only the last sample and those where a path that
+                // has a survival adjoint is above the zone's lower end.  (A
+                // step's numbers in the kernel's precision from one row in LDS;
+                // every sample worked, sqrt(dt) and the conversions formed at
+                // each step: the three risk calls of a serving burst 180 us on
+                // average, now 106; the two pricing calls 173, now 122.)
+                const uint64_t some = BSR ? __builtin_amdgcn_ballot_w64(live) : 0;
+                const uint64_t zoned = BSR ? __builtin_amdgcn_ballot_w64(live && !ps.dead && ps.euro != R(0)) : 0;
+                if constexpr (BSR) {
+                    auto step = [&](int i, R g) {
+                        const R* r = bsr + i * kBsReals;
+                        spot = spot * rexp(r[0] + r[1] * g);
+                        tau[1] = tau[1] + r[4] + r[5] * g;
+                        tau[2] = tau[2] + r[6];
+                        tau[3] = tau[3] - r[6];
+                        const R F = spot * r[2];
+                        if (i == n - 1 || (__builtin_amdgcn_ballot_w64(F > R(P.minus_smooth)) & zoned) != 0) {
+                            const int s = __builtin_amdgcn_readfirstlane(step_sample[i + 1]);
+                            if (s >= 0) accumulate(s, spot);
+                        }
+                    };
+                    int i = 0;
+                    if (some != 0) {
+                        // (four normals at a time)
+                        R g4[4] = {R(0), R(0), R(0), R(0)};
+                        auto normals4 = [&](int at) {
+                            if constexpr (QUADS && RECOMP) {
+                                uint32_t gw[4];
+                                sobol_words4(lo_tab, hl, lane, at, gw);
+#pragma unroll
+                                for (int k = 0; k < 4; ++k) g4[k] = inv_normal(gw[k], invn_tab);
+                            } else {
+#pragma unroll
+                                for (int k = 0; k < 4; ++k) g4[k] = RECOMP ? draw(at + k) : ck[(at + k) * kWave + lane];
+                            }
+                        };
+                        for (; i + 4 <= nrev; i += 4) {
+                            normals4(i);
+#pragma unroll
+                            for (int k = 0; k < 4; ++k) step(i + k, g4[k]);
+                        }
+                        for (; i < nrev; ++i) step(i, RECOMP ? draw(i) : ck[i * kWave + lane]);
+                    }
+                } else
                 for (int i = 0; i < nrev; ++i) {
                     R g;
                     if constexpr (RECOMP) g = draw(i);   // regenerated
