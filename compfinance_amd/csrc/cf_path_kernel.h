@@ -681,19 +681,47 @@ __device__ __forceinline__ void sobol_words4(const uint32_t* lo_tab, const uint3
     w[3] = lw.w ^ hw.w;
 }
 
-// HI_qb of the n dimensions into a wave's LDS row, formed by the wave's lanes
+// HI_qb of the n dimensions into a wave's LDS row, formed by the wave's lanes.
+// AHEAD: sixteen direction numbers loaded together and masked, for the Dupire
+// adjoint kernels, whose few waves wait for them (2^20 paths x 156 steps, risk:
+// FP32 0.354 -> 0.346 ms, FP64 0.654 -> 0.650); the others, with up to twice
+// the waves, take only the ones they need (FP64 pricing 0.239 against 0.251 ms).
+template <bool AHEAD>
 __device__ __forceinline__ void sobol_fill_hi(uint32_t* row, const uint32_t* dirs, int n, int64_t qb, int lane)
 {
     const uint32_t gq = uint32_t(qb ^ (qb >> 1));
-    for (int d = lane; d < n; d += kWave) {
-        uint32_t x = (qb & 1) ? dirs[5 * kSobolDims + d] : 0u;
-        uint32_t b = gq;
-        while (b) {
-            const int j = __builtin_ctz(b);
-            x ^= dirs[(j + 6) * kSobolDims + d];
-            b &= b - 1u;
+    if constexpr (AHEAD) {
+        // the direction numbers of the row, by the bits of g
+        uint32_t g = gq << 6 | uint32_t(qb & 1) << 5;
+        for (int d = lane; d < n; d += kWave) {
+            // (opaque: the bits' masks and the addresses are formed here, not
+            // kept in registers over the whole kernel)
+            uint32_t at = uint32_t(d);
+            asm volatile("" : "+s"(g), "+v"(at));
+            uint32_t x = 0;
+            auto rows = [&](auto first, auto count) {
+                constexpr int B = decltype(first)::value, N = decltype(count)::value;
+                uint32_t v[N];
+#pragma unroll
+                for (int k = 0; k < N; ++k) v[k] = (dirs + (B + k) * kSobolDims)[at];
+#pragma unroll
+                for (int k = 0; k < N; ++k) x ^= v[k] & uint32_t(-int((g >> (B + k)) & 1u));
+            };
+            rows(std::integral_constant<int, 5>{}, std::integral_constant<int, 16>{});
+            if (g >> 21) rows(std::integral_constant<int, 21>{}, std::integral_constant<int, 11>{});
+            row[d] = x;
         }
-        row[d] = x;
+    } else {
+        for (int d = lane; d < n; d += kWave) {
+            uint32_t x = (qb & 1) ? dirs[5 * kSobolDims + d] : 0u;
+            uint32_t b = gq;
+            while (b) {
+                const int j = __builtin_ctz(b);
+                x ^= dirs[(j + 6) * kSobolDims + d];
+                b &= b - 1u;
+            }
+            row[d] = x;
+        }
     }
 }
 
@@ -713,14 +741,15 @@ struct SobolLane {
 // tail row is free, so that lane reads words of 2^31 from it instead (its low
 // words are 0) and its draws stay inside the table.  fill: the rows are
 // formed (false when the words are not used).
+template <bool AHEAD = false>
 __device__ __forceinline__ SobolLane sobol_block(uint32_t* hi, uint32_t* hi_tail, const uint32_t* dirs, int n,
                                                  int64_t q, int64_t q0, int64_t q1, int64_t nlo, int64_t nhi,
                                                  bool merge, int lane, bool fill)
 {
     const bool tail_wave = merge && q == q0;
     if (fill) {
-        sobol_fill_hi(hi, dirs, n, q, lane);
-        if (tail_wave) sobol_fill_hi(hi_tail, dirs, n, q1, lane);
+        sobol_fill_hi<AHEAD>(hi, dirs, n, q, lane);
+        if (tail_wave) sobol_fill_hi<AHEAD>(hi_tail, dirs, n, q1, lane);
         if (!merge && q == 0)
             for (int d = lane; d < n; d += kWave) hi_tail[d] = 0x80000000u;
         wave_sync_lds();
@@ -1072,7 +1101,7 @@ __device__ __forceinline__ void path_body(const LaunchParams& P, const int bid, 
     for (int64_t q = q0 + int64_t(bid) * waves + wave; q <= qe; q += int64_t(nblk) * waves) {
         // ---- high Sobol words of this block of 64 indices (and of the
         // merged last block); this lane's row, index and path
-        const SobolLane sl = sobol_block(hi, hi_tail, P.dirs, n, q, q0, q1, nlo, nhi, merge, lane, !MRG);
+        const SobolLane sl = sobol_block<AD && DUP && !BOOK>(hi, hi_tail, P.dirs, n, q, q0, q1, nlo, nhi, merge, lane, !MRG);
         const uint32_t* hl = sl.hl;
         const bool active = sl.active;
         const int64_t pidx = sl.pidx;
