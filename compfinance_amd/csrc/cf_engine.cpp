@@ -1294,12 +1294,14 @@ int run(const cf_model* mdl, const cf_product* prd, Call& c)
     if (c.per_path_agg) B.per_path_agg = static_cast<double*>(E.per_path_agg.ensure(size_t(S.n_path) * 8));
 
     hip_check(hipEventRecord(E.ev[0], E.stream), "hipEventRecord");
+    bool uploads = false;
     if (c.adjoint) {
         // the device copy of the weights is reused while the call's weights are
         // the last ones uploaded to the same buffer (only this path writes it)
         const size_t wb = size_t(S.npay) * 8;
         const bool same = E.weights_on_device == B.weights && E.weights_last.size() == size_t(S.npay) &&
                           std::memcmp(E.weights_last.data(), c.weights, wb) == 0;
+        uploads = !same;
         if (!same) {
             std::memcpy(h_in, c.weights, wb);
             hip_check(hipMemcpyAsync(B.weights, h_in, wb, hipMemcpyHostToDevice, E.stream), "upload");
@@ -1313,8 +1315,9 @@ int run(const cf_model* mdl, const cf_product* prd, Call& c)
         P.blocks_done = E.d_blocks_done;
         P.reduced = B.reduced;
     }
-    // (a fused pricing call is one kernel: the first and last event bound it)
-    const bool one = fused && !c.adjoint;
+    // (a fused call without an upload is one kernel: the first and last event
+    // bound it)
+    const bool one = fused && !uploads;
     const double setup_ms = ms_since(t_start);
     enqueue_call(PR, S, B, P, E.stream, one ? nullptr : E.ev[1], one ? nullptr : E.ev[2]);
     hip_check(hipEventRecord(E.ev[3], E.stream), "hipEventRecord");

@@ -2462,22 +2462,36 @@ __device__ __forceinline__ void path_body(const LaunchParams& P, const int bid, 
             if (tid == 0) *is_last = atomicInc(P.blocks_done, unsigned(nblk - 1)) == unsigned(nblk - 1) ? 1 : 0;
             __syncthreads();
             if (*is_last) {
+                // (the columns of a wave, up to four at a time: their loads
+                // and their chains of additions overlap)
                 const int cols = fused_cols(npay, AD);
-                for (int c = wave; c < cols; c += waves) {
-                    double s = 0.0;
-                    for (int r = lane; r < nblk; r += kWave) 
-                        s += __hip_atomic_load(P.block_out + size_t(r) * stride + c, __ATOMIC_RELAXED,
-                                               __HIP_MEMORY_SCOPE_AGENT);
-                    const uint64_t b = __builtin_bit_cast(uint64_t, s);
-                    double t = 0.0;
+                auto sum = [&](auto at) {
+                    constexpr int N = decltype(at)::value;
+                    for (int c0 = wave; c0 < cols; c0 += N * waves) {
+                        double s[N] = {}, t[N] = {};
+                        for (int r = lane; r < nblk; r += kWave)
+#pragma unroll
+                            for (int j = 0; j < N; ++j)
+                                if (c0 + j * waves < cols)
+                                    s[j] += __hip_atomic_load(P.block_out + size_t(r) * stride + c0 + j * waves,
+                                                              __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 #pragma unroll 16
-                    for (int k = 0; k < kWave; ++k) {
-                        const uint32_t lo = __builtin_amdgcn_readlane(uint32_t(b), k);
-                        const uint32_t hi = __builtin_amdgcn_readlane(uint32_t(b >> 32), k);
-                        t += __builtin_bit_cast(double, uint64_t(hi) << 32 | lo);
+                        for (int k = 0; k < kWave; ++k)
+#pragma unroll
+                            for (int j = 0; j < N; ++j) {
+                                const uint64_t b = __builtin_bit_cast(uint64_t, s[j]);
+                                const uint32_t lo = __builtin_amdgcn_readlane(uint32_t(b), k);
+                                const uint32_t hi = __builtin_amdgcn_readlane(uint32_t(b >> 32), k);
+                                t[j] += __builtin_bit_cast(double, uint64_t(hi) << 32 | lo);
+                            }
+#pragma unroll
+                        for (int j = 0; j < N; ++j)
+                            if (lane == 0 && c0 + j * waves < cols) P.reduced[c0 + j * waves] = t[j];
                     }
-                    if (lane == 0) P.reduced[c] = t;
-                }
+                };
+                if (cols <= waves) sum(std::integral_constant<int, 1>{});
+                else if (cols <= 2 * waves) sum(std::integral_constant<int, 2>{});
+                else sum(std::integral_constant<int, 4>{});
             }
         }
     }
