@@ -2517,9 +2517,18 @@ __device__ __forceinline__ void path_body(const LaunchParams& P, const int bid, 
 #define CF_PATH_KERNEL_ATTR
 #endif
 
+// Waves a SIMD has to hold at least (beside those that a block implies): the
+// FP32 recompute book on Black-Scholes, bound by its waves, takes 133 registers
+// without the limit, three waves instead of four (2^19 mrg32k3a paths of 5
+// steps: 147 against 112 us).
+constexpr int min_waves(int model, int prd, int real_bytes, int adj)
+{
+    return model == MODEL_BS && prd == PRD_BOOK && real_bytes == 4 && adj == ADJ_RECOMPUTE ? 4 : 1;
+}
+
 template <typename R, int MODEL, int PRD, int ADJ, bool LEAN, bool MRG, bool ITEM>
-__global__ void __launch_bounds__(book_block_limit(PRD, int(sizeof(R)), ADJ)) CF_PATH_KERNEL_ATTR
-path_kernel(const LaunchParams P)
+__global__ void __launch_bounds__(book_block_limit(PRD, int(sizeof(R)), ADJ), min_waves(MODEL, PRD, int(sizeof(R)), ADJ))
+CF_PATH_KERNEL_ATTR path_kernel(const LaunchParams P)
 {
     path_body<R, MODEL, PRD, ADJ, LEAN, MRG, ITEM>(P, int(blockIdx.x), int(gridDim.x));
 }
