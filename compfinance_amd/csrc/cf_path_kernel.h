@@ -934,9 +934,12 @@ __device__ __forceinline__ void path_body(const LaunchParams& P, const int bid, 
     const bool ck_lo = CKB && (!LEAN || m <= kMaxStoredKnots);
     // States and bracket bytes interleaved by groups of four steps (a lane's
     // four in one 16-byte, in FP64 32-byte, word and one 4-byte word), except
+    // those of the FP64 book, whose steps run one by one: gathering four costs
+    // it more than the wider access saves (55 payoffs, 250,007 paths 0.84
+    // against 0.79 ms; an Asian alone, 2^19 paths of 52 steps 0.33 against 0.28).
     // FP32 pads the steps to whole groups; FP64 keeps the steps from n4 on,
     // up to three, in rows.
-    constexpr bool IL = CKB;
+    constexpr bool IL = CKB && !(BOOK && sizeof(R) == 8);
     const int nck = ckpt_steps(n, int(sizeof(R)));
     const int n4 = n & ~3;
     uint8_t* const ckl0 = CKB ? reinterpret_cast<uint8_t*>(ck + size_t(nck) * kWave) : nullptr;
@@ -1537,8 +1540,6 @@ __device__ __forceinline__ void path_body(const LaunchParams& P, const int bid, 
                 // select, so the book's step is compiled once)
                 double* trow = tails + wave * TR;
                 double gb[4] = {0.0, 0.0, 0.0, 0.0};
-                double gs0 = 0.0, gs1 = 0.0, gs2 = 0.0;
-                uint32_t gl4 = 0;
                 for (; i < n; ++i) {
                     const int k = i & 3;
                     if (k == 0 && i < n4) {
@@ -1559,27 +1560,7 @@ __device__ __forceinline__ void path_body(const LaunchParams& P, const int bid, 
                     }
                     if (i < n4) gz[0] = k == 0 ? gb[0] : k == 1 ? gb[1] : k == 2 ? gb[2] : gb[3];
                     else gz[0] = draw(i);
-                    // (checkpoints: the four steps' states and brackets
-                    // gathered, stored with the last)
-                    glo = 0;
-                    fwd_step(i, 0, std::integral_constant<bool, IL>{}, std::true_type{});
-                    if constexpr (IL) {
-                        if (i < n4) {
-                            if (k == 0) gs0 = gx[0];
-                            if (k == 1) gs1 = gx[0];
-                            if (k == 2) gs2 = gx[0];
-                            gl4 = (gl4 >> 8) | (glo << 24);
-                            if (k == 3) {
-                                double2* c = reinterpret_cast<double2*>(ck + ck_el(i - 3));
-                                c[0] = make_double2(gs0, gs1);
-                                c[1] = make_double2(gs2, gx[0]);
-                                if (ck_lo) *reinterpret_cast<uint32_t*>(ckl + ck_el(i - 3)) = gl4;
-                            }
-                        } else {
-                            ck[i * kWave + lane] = gx[0];
-                            if (ck_lo) ckl[i * kWave + lane] = uint8_t(glo);
-                        }
-                    }
+                    fwd_step(i, 0, std::false_type{}, std::true_type{});
                 }
             } else {
                 for (; i < n; ++i) fwd_step(i, 0, std::false_type{}, std::false_type{});
@@ -2226,12 +2207,8 @@ __device__ __forceinline__ void path_body(const LaunchParams& P, const int bid, 
                                 }
                                 smp = int(((rbits >> (i & 63)) & 1u)) - 1;
                             } else {
-                                smp = BOOK ? 0 : __builtin_amdgcn_readfirstlane(step_sample[i]);
+                                smp = __builtin_amdgcn_readfirstlane(step_sample[i]);
                             }
-                            // (book: the row read a step ahead)
-                            const SampleRow row = prow;
-                            if constexpr (BOOK) prow = bk_rows(max(i - 1, 0));
-                            const bool on = BOOK ? (row.bars | row.grps) != 0 || row.van_hi > row.van_lo : smp >= 0;
                             if (!ck_lo) lo = knot_count(xi);
                             const Bracket<R> b = local_vol_at(kxi, iv + i * mp, xi, lo);
                             R ws = recip_mul(xnext - xi, b.vol) - R(0.5) * b.vol;
@@ -2242,10 +2219,10 @@ __device__ __forceinline__ void path_body(const LaunchParams& P, const int bid, 
                             if constexpr (UNDER) {
                                 if (smp >= 0 && __builtin_amdgcn_ballot_w64(xi > x_adj) != 0)
                                     sf = barrier_sf(zone_spot(xi));
-                            } else if (on && (!(row.grps & kBookPlain) || __builtin_amdgcn_ballot_w64(xi > rv_x) != 0)) {
+                            } else if (smp >= 0) {
                                 const R S = state_spot(xi, s0);
                                 R Fb, nb, db;
-                                sample_adj(smp, row, S, S, R(1), R(1), Fb, nb, db, false);
+                                sample_adj(smp, SampleRow{}, S, S, R(1), R(1), Fb, nb, db, false);
                                 sf = S * Fb;
                             }
                             const R vb = abar * ws;
@@ -2286,34 +2263,6 @@ __device__ __forceinline__ void path_body(const LaunchParams& P, const int bid, 
                                 step(i, a0.x, int(w & 0xffu), recover);
                             }
                         };
-                        if constexpr (BOOK) {
-                            // the book's step is compiled once: steps from
-                            // n4 on read their row, the others a group of
-                            // four loaded a group ahead
-                            prow = bk_rows(last);
-                            load4(min(last, n4 - 1) >> 2);
-                            double2 a0 = c0, a1 = c1;
-                            uint32_t w = cw;
-                            for (int i = last; i >= 0; --i) {
-                                const int k = i & 3;
-                                R xi;
-                                int lo;
-                                if (i >= n4) {
-                                    xi = ck[i * kWave + lane];
-                                    lo = ck_lo ? int(ckl[i * kWave + lane]) : 0;
-                                } else {
-                                    if (k == 3 || i == last) {
-                                        a0 = c0;
-                                        a1 = c1;
-                                        w = cw;
-                                        load4((i >> 2) - 1);
-                                    }
-                                    xi = k == 3 ? a1.y : k == 2 ? a1.x : k == 1 ? a0.y : a0.x;
-                                    lo = int((w >> (8 * k)) & 0xffu);
-                                }
-                                step(i, xi, lo, std::false_type{});
-                            }
-                        } else
                         if (iv_recover) sweep(std::true_type{}); else sweep(std::false_type{});
                     }
                 } else if (n > 0) {
