@@ -14,18 +14,18 @@
 //     so the point of lane r in dimension d is  LO[d][r] ^ HI_q[d]:  LO is a
 //     per-block LDS table built once, HI_q a per-wave LDS row built per block
 //     of paths;
-//   * local-vol table, interval table, knot search table, inverse-normal
-//     table and timeline sample map in LDS (the LEAN layout of long timelines
-//     and large grids reads the local-vol, knot search and inverse-normal
-//     tables from global memory through L1 instead);
+//   * local-vol table, interval table, knot search table and timeline sample
+//     map in LDS (the LEAN layout of long timelines and large grids reads the
+//     local-vol and knot search tables from global memory through L1 instead);
+//     the FP32 inverse-normal table through L1 or in LDS (GINV);
 //   * FP64 draws four steps at a time, the inverse normal's tail form
 //     evaluated once per wave for the lanes that need it (a per-wave LDS row
 //     of 64 doubles, 32 in the LEAN layout);
 //   * mrg32k3a instead of Sobol: one generator per lane in registers, jumped
 //     to its path's block of numbers and stepped back in the reverse sweeps;
 //   * payoffs reduced per wave with DPP cross-lane moves into per-wave LDS
-//     accumulators, then per block, then across blocks by a separate kernel
-//     in fixed order;
+//     accumulators, then per block, then across blocks in fixed order by the
+//     last block or a separate kernel (fused_reduction);
 //   * adjoint: path states checkpointed in a per-wave HBM slot (reused by the
 //     wave for each block of paths) with the knot bracket of each state in a
 //     byte, reverse sweep over the Euler steps,
