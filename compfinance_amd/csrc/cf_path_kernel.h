@@ -1070,15 +1070,15 @@ __device__ __forceinline__ void path_body(const LaunchParams& P, const int bid, 
     constexpr int NBAR = BOOK ? kMaxBookBarriers : 1, NGRP = BOOK ? kMaxBookGroups : 1;
     // Book barrier state in one real per barrier:
     //   sign bit set  breached (survival 0, no derivative)
-    //   v in [0, 1]   no exactly-zero smoothing factor yet, v = product of the
-    //                 factors (the survival factor)
-    //   v > 1         one zero factor, v = 2^1000 x the product of the others
-    //                 (FP64; a second one makes it 0, as two have no derivative)
+    //   v in [0, 1]   the product of the smoothing factors (the survival factor)
     // A smoothing factor is (B + w - F) / 2w clamped to [0, 1], so an update is
-    // a product for every lane, in the zone, under it or breached.  FP32 keeps
-    // every factor at least 1e-30 (as the single barrier keeps B + w - F above
-    // a floor), so its states are only [0, 1] or breached.
-    constexpr double kZeroScale = 0x1p1000, kZeroMark = 0x1p600;   // (weighted: above the mark)
+    // a product for every lane, in the zone, under it or breached.  An
+    // exactly-zero factor (FP64) is left out of the product and marked in the
+    // path's bit mask zmask, beside the state, whose range stays free for any
+    // weight: the survival factor is 0, and v is the product of the others,
+    // which the derivative takes at that factor; a second one makes v 0 too, as
+    // two have no derivative.  FP32 keeps every factor at least 1e-30 (as the
+    // single barrier keeps B + w - F above a floor) and marks none.
     // v after an observation at distance t = B + w - F, 1 / 2w = i2s
     auto bar_update = [&](R v, R t, R i2s) -> R {
         if constexpr (sizeof(R) == 4) {
@@ -1091,8 +1091,6 @@ __device__ __forceinline__ void path_body(const LaunchParams& P, const int bid, 
             return __builtin_bit_cast(double, __builtin_bit_cast(uint64_t, v * f) | sign);
         }
     };
-    // the survival factor of a state
-    auto bar_alive = [&](R v) -> R { return v > R(0) && (!ZT || v <= R(1)) ? v : R(0); };
     const R bk_xlo = BOOK && DUP ? R(P.bar_xlo) : R(0);   // every zone is above this state
 
     // PK: swept paths waiting for a full wave, in lanes 0 .. pk_n - 1 of pk_src
@@ -1152,12 +1150,26 @@ __device__ __forceinline__ void path_body(const LaunchParams& P, const int bid, 
         // vanilla, the adjoint of its survival factor; per fixing schedule
         // the running sum, replaced at its last fixing by the adjoint of each
         // fixing, and the weighted intrinsic value (numeraire adjoint)
-        // (FP64 keeps one value per barrier: at its maturity the state is
-        // replaced by its product with weight x vanilla, 0 after a breach,
-        // which is all that the reverse needs; its registers bound the waves
-        // on a compute unit)
-        constexpr int NBB = ZT ? 1 : NBAR;
+        // (LAZY keeps one value per barrier, its registers bound the waves on a
+        // compute unit: a sweep that meets the maturity before the samples
+        // before it replaces the state there by its product with weight x
+        // vanilla; up to then a path without a vanilla counts as breached,
+        // which has no adjoint either)
+        constexpr bool LAZY = ZT && CKB;
+        constexpr int NBB = LAZY ? 1 : NBAR;
         R bst[NBAR], babar[NBB], gsum[NGRP], gq[NGRP];
+        uint32_t zmask = 0;
+        // the survival factor of barrier b
+        auto bar_alive = [&](int b) -> R {
+            return bst[b] > R(0) && !(ZT && ((zmask >> b) & 1u)) ? bst[b] : R(0);
+        };
+        // an exactly-zero factor of barrier b: the distance t = 0 that the
+        // update takes it from, a first one as far below the zone (factor 1)
+        auto mark_zero = [&](int b, R& t) {
+            if (t != R(0)) return;
+            if (!((zmask >> b) & 1u)) t = R(INFINITY);
+            zmask |= 1u << b;
+        };
 #pragma unroll
         for (int b = 0; b < NBAR; ++b) bst[b] = R(1);
 #pragma unroll
@@ -1246,21 +1258,20 @@ __device__ __forceinline__ void path_body(const LaunchParams& P, const int bid, 
                             up[j] = bk_four_c[b >> 2].up[j];
                             i2s[j] = bk_four_c[b >> 2].i2s[j];
                         }
-                        R t[4], v[4];
+                        R t[4];
                         uint64_t zero = 0;
 #pragma unroll
                         for (int j = 0; j < 4; ++j) {
                             t[j] = up[j] - F;
-                            v[j] = bst[b + j];
                             if constexpr (ZT) zero |= __builtin_amdgcn_ballot_w64(t[j] == R(0));
-                            bst[b + j] = bar_update(v[j], t[j], i2s[j]);
                         }
                         if (ZT && zero != 0) {
-                            asm volatile("");   // an exactly-zero factor: rare, a branch of its own
+                            asm volatile("");   // (rare: a branch of its own)
 #pragma unroll
-                            for (int j = 0; j < 4; ++j)
-                                if (t[j] == R(0) && !(v[j] > R(1))) bst[b + j] = v[j] * R(kZeroScale);
+                            for (int j = 0; j < 4; ++j) mark_zero(b + j, t[j]);
                         }
+#pragma unroll
+                        for (int j = 0; j < 4; ++j) bst[b + j] = bar_update(bst[b + j], t[j], i2s[j]);
                     }
                 }
                 if (!all_bars && sm.bars) {
@@ -1269,16 +1280,16 @@ __device__ __forceinline__ void path_body(const LaunchParams& P, const int bid, 
                         if (!(((sm.bars | bl) >> b) & 1u)) continue;
                         const BarPar bp = bar_par(b);
                         if ((sm.bars >> b) & 1u) {
-                            const R t = bp.up - F, v = bst[b];
-                            bst[b] = bar_update(v, t, bp.i2s);
-                            if (ZT && t == R(0) && !(v > R(1))) bst[b] = v * R(kZeroScale);
+                            R t = bp.up - F;
+                            if constexpr (ZT) mark_zero(b, t);
+                            bst[b] = bar_update(bst[b], t, bp.i2s);
                         }
                         if ((bl >> b) & 1u) {
                             const R k = bp.k;
                             const R intrinsic = bk_bar_put[b] ? (k - F > R(0) ? k - F : R(0))
                                                                          : (F - k > R(0) ? F - k : R(0));
                             const R euro = intrinsic / numv;
-                            const R alive = bar_alive(bst[b]);
+                            const R alive = bar_alive(b);
                             const int col = bk_bar_col[b];
                             emit(col, alive * euro);
                             emit(col + 1, euro);
@@ -1286,9 +1297,9 @@ __device__ __forceinline__ void path_body(const LaunchParams& P, const int bid, 
                             // factor (the ITEM kernels keep the vanilla and
                             // weigh it before the reverse sweep)
                             if constexpr (AD) {
-                                const R we = ITEM ? euro : R(wts[col]) * euro;
-                                if constexpr (ZT) bst[b] = bst[b] > R(0) ? we * bst[b] : R(0);
-                                else babar[b] = we;
+                                const R w = ITEM ? R(1) : R(wts[col]);
+                                if constexpr (LAZY) bst[b] = euro != R(0) && w != R(0) ? bst[b] : R(-1);
+                                else babar[b] = w * euro;
                             }
                         }
                     }
@@ -1378,6 +1389,7 @@ __device__ __forceinline__ void path_body(const LaunchParams& P, const int bid, 
             ps.alive = stq[1 * kWave];
             ps.pnz = stq[2 * kWave];
             ps.nzero = int(stq[3 * kWave]);
+            if constexpr (BOOK && ZT) zmask = uint32_t(ps.nzero);
             ps.dead = stq[4 * kWave] != R(0);
             ps.euro = stq[5 * kWave];
             ps.fin_f = stq[6 * kWave];
@@ -1385,7 +1397,7 @@ __device__ __forceinline__ void path_body(const LaunchParams& P, const int bid, 
 #pragma unroll
             for (int b = 0; b < NBAR; ++b) {
                 bst[b] = stq[(8 + b) * kWave];
-                if constexpr (!ZT) babar[b] = stq[(8 + NBAR + b) * kWave];
+                if constexpr (!LAZY) babar[b] = stq[(8 + NBAR + b) * kWave];
             }
 #pragma unroll
             for (int g = 0; g < NGRP; ++g) {
@@ -1600,7 +1612,7 @@ __device__ __forceinline__ void path_body(const LaunchParams& P, const int bid, 
                 stq[0] = x;
                 stq[1 * kWave] = ps.alive;
                 stq[2 * kWave] = ps.pnz;
-                stq[3 * kWave] = R(ps.nzero);
+                stq[3 * kWave] = R(BOOK ? int(zmask) : ps.nzero);
                 stq[4 * kWave] = ps.dead ? R(1) : R(0);
                 stq[5 * kWave] = ps.euro;
                 stq[6 * kWave] = ps.fin_f;
@@ -1608,7 +1620,7 @@ __device__ __forceinline__ void path_body(const LaunchParams& P, const int bid, 
 #pragma unroll
                 for (int b = 0; b < NBAR; ++b) {
                     stq[(8 + b) * kWave] = bst[b];
-                    if constexpr (!ZT) stq[(8 + NBAR + b) * kWave] = babar[b];
+                    if constexpr (!LAZY) stq[(8 + NBAR + b) * kWave] = babar[b];
                 }
 #pragma unroll
                 for (int g = 0; g < NGRP; ++g) {
@@ -1626,8 +1638,9 @@ __device__ __forceinline__ void path_body(const LaunchParams& P, const int bid, 
 #pragma unroll
                 for (int b = 0; b < NBAR; ++b)
                     if (b < P.bk.n_bar) {
-                        if constexpr (ZT) bst[b] = R(wts[bk_bar_col[b]]) * bst[b];
-                        else babar[b] = R(wts[bk_bar_col[b]]) * babar[b];
+                        const R w = R(wts[bk_bar_col[b]]);
+                        if constexpr (LAZY) bst[b] = w != R(0) ? bst[b] : R(-1);
+                        else babar[b] = w * babar[b];
                     }
 #pragma unroll
                 for (int g = 0; g < NGRP; ++g) {
@@ -1763,7 +1776,7 @@ __device__ __forceinline__ void path_body(const LaunchParams& P, const int bid, 
                 for (int b = 0; b < NBAR; ++b) {
                     const float lo = float(bk_four_c[b >> 2].lo[b & 3]);
                     const float th = sizeof(R) == 4 ? lo : lo - 1e-6f * fabsf(lo);
-                    if constexpr (ZT) rth[b] = bst[b] != R(0) ? th : INFINITY;
+                    if constexpr (LAZY) rth[b] = bst[b] > R(0) ? th : INFINITY;
                     else rth[b] = bst[b] > R(0) && babar[b] != R(0) ? th : INFINITY;
                     lo_min = fminf(lo_min, rth[b]);
                 }
@@ -1774,6 +1787,8 @@ __device__ __forceinline__ void path_body(const LaunchParams& P, const int bid, 
                     if (!(lo_min < INFINITY)) rv_x = R(INFINITY);
                 }
             }
+
+            const bool zany = BOOK && ZT && __builtin_amdgcn_ballot_w64(zmask != 0) != 0;
 
             // adjoints of the forward, numeraire and discount at sample s
             const R alive_eff = ps.dead ? R(0) : ps.alive;
@@ -1821,21 +1836,19 @@ __device__ __forceinline__ void path_body(const LaunchParams& P, const int bid, 
                     // state over the factor without a zero factor; with one,
                     // its product for the zero factor and 0 for the others
                     auto zone_adj = [&](int b, R up, R i2s) {
-                        const R v = bst[b];
                         if constexpr (ZT) {
                             // v: the weighted vanilla times the state
-                            const R d = up - F;
+                            const R v = LAZY ? bst[b] : babar[LAZY ? 0 : b] * bst[b], d = up - F;
                             R a = recip_mul(v, d);
-                            const bool one = fabs(v) > R(kZeroMark);
-                            if (__builtin_amdgcn_ballot_w64(one) != 0) {
+                            if (zany) {
                                 asm volatile("");   // (rare: a branch of its own)
-                                if (one) a = d == R(0) ? v * R(1.0 / kZeroScale) * i2s : R(0);
+                                if ((zmask >> b) & 1u) a = d == R(0) ? v * i2s : R(0);
                             }
                             Fb -= a;
                         } else {
                             // FP32 (factors at least 1e-30)
                             const R f = max((up - F) * i2s, R(1e-30));
-                            Fb -= babar[b] * i2s * recip_mul(v, f);
+                            Fb -= babar[b] * i2s * recip_mul(bst[b], f);
                         }
                     };
                     const uint32_t bm = sm.bars & 0xffffu;
@@ -1856,20 +1869,11 @@ __device__ __forceinline__ void path_body(const LaunchParams& P, const int bid, 
                                 const R intrinsic = put ? (k - F > R(0) ? k - F : R(0))
                                                         : (F - k > R(0) ? F - k : R(0));
                                 const R dmax = put ? (k > F ? R(-1) : R(0)) : (F > k ? R(1) : R(0));
-                                // weight x survival factor (FP64: from the
-                                // weighted vanilla times the state, where the
-                                // vanilla is 0 it does not matter)
-                                // (FP32: one expression, one rounding)
-                                R euro_bar;
-                                if constexpr (ZT) {
-                                    const R euro = intrinsic / numv;
-                                    const R wa = euro != R(0) && !(fabs(bst[b]) > R(kZeroMark)) ? bst[b] / euro : R(0);
-                                    euro_bar = wa + R(wts[col + 1]);
-                                } else {
-                                    euro_bar = R(wts[col]) * bar_alive(bst[b]) + R(wts[col + 1]);
-                                }
+                                // (one expression, one rounding)
+                                const R euro_bar = R(wts[col]) * bar_alive(b) + R(wts[col + 1]);
                                 Fb += euro_bar * dmax / numv;
                                 nb += -euro_bar * (intrinsic / numv) / numv;
+                                if constexpr (LAZY) bst[b] = R(wts[col]) * intrinsic * bst[b];
                             }
                             if (Ff > rth[b] && F > bp.lo && ((bm >> b) & 1u)) zone_adj(b, bp.up, bp.i2s);
                         }
