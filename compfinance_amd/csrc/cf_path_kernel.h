@@ -449,14 +449,18 @@ __device__ __forceinline__ double exp_series(double d)
     for (int k = N - 2; k >= 3; --k) q = fma_s(q, d, c[k]);
     return fma(q, d, 0.5);
 }
-// exp in FP64: x = n ln(2) + d, 2^n (1 + (d + d^2 series)), within 0.8 ulp; x
-// beyond +-800 saturates to 0 or infinity.  22 instructions, no table (a load
-// would wait for the checkpoint stores issued before it), against the library
-// function's 35.
+// exp in FP64 by Cody and Waite's reduction: x = n ln(2) + d,
+// 2^n (1 + (d + d^2 series)), within 0.8 ulp; x beyond +-800 saturates to 0 or
+// infinity, and a NaN stays one (v_max_f64 would drop it: under -800 the high
+// word is replaced instead, by that of -800; above 800 only n is bounded, d
+// overflows).  23 instructions, no table (a load would wait for the checkpoint
+// stores issued before it), against the library function's 35.
 __device__ __forceinline__ double exp_f64(double x)
 {
-    x = min_f64(max_f64(x, -800.0), 800.0);
-    const double n = __builtin_rint(x * 1.4426950408889634);
+    const uint64_t bits = __builtin_bit_cast(uint64_t, x);
+    const uint32_t hi = x < -800.0 ? 0xc0890000u : uint32_t(bits >> 32);
+    x = __builtin_bit_cast(double, uint64_t(hi) << 32 | uint32_t(bits));
+    const double n = __builtin_rint(min_f64(x, 800.0) * 1.4426950408889634);
     // ln(2) in two parts, the first of 33 bits: n times it is exact
     double d = fma(n, -6.93147180369123816490e-01, x);
     d = fma(n, -1.90821492927058770002e-10, d);
