@@ -377,7 +377,7 @@ int kernel_product(const ProductPlan& d)
 }
 
 
-BookTables build_book(const ProductPlan& d, double width0)
+BookTables build_book(const ProductPlan& d, double width0, bool fp64)
 {
     vector<const ProductPlan*> parts;
     if (d.kind == CF_PRODUCT_BOOK) {
@@ -480,10 +480,22 @@ BookTables build_book(const ProductPlan& d, double width0)
     // vanillas [van_first[s], van_first[s + 1])
     vector<uint32_t> masks(size_t(ns) * 4);
     const uint32_t all_bars = (1u << n_bars) - 1u;
+    // The update by fours takes the factor of a state at or under the zone for
+    // 1, which it is where the zone has a width in the kernel's precision.
+    // Without one (no smoothing in FP32: B + w = B - w) a state on the barrier
+    // would get the factor 0 of its upper end: such books observe barrier by
+    // barrier, which asks for the zone first.
+    auto has_width = [&](auto real, size_t b) {
+        using T = decltype(real);
+        const T up = T(bar_par[4 * b + 1]), lo = T(bar_par[4 * b + 2]);
+        return lo < up && std::isfinite(up) && std::isfinite(lo) && std::isfinite(T(bar_par[4 * b + 3]));
+    };
+    bool by_fours = n_bars > 0;
+    for (size_t b = 0; b < n_bars; ++b) by_fours = by_fours && (fp64 ? has_width(double(), b) : has_width(float(), b));
     for (int k = 0; k < ns; ++k) {
         masks[4 * k] = bar_mask[k] | (bar_last[k] << 16);
         masks[4 * k + 1] = grp_mask[k] | (grp_last[k] << 4);
-        if (n_bars > 0 && bar_mask[k] == all_bars && bar_last[k] == 0) {
+        if (by_fours && bar_mask[k] == all_bars && bar_last[k] == 0) {
             masks[4 * k + 1] |= cfk::kBookAllBars;
             if (grp_mask[k] == 0 && van[k].empty()) masks[4 * k + 1] |= cfk::kBookPlain;
         }
@@ -857,7 +869,7 @@ std::shared_ptr<Prepared> prepare(Engine& E, const cf_model* mdl, const cf_produ
         }
     }
     const bool book = kernel_product(pd) == cfk::PRD_BOOK;
-    if (book) P->book = build_book(pd, md.s_t0);
+    if (book) P->book = build_book(pd, md.s_t0, fp64);
     P->cfg = cfk::KernelConfig{fp64 ? 0 : 1, md.kind, kernel_product(pd), adjoint, false, adj == cfk::ADJ_RECOMPUTE};
     P->block = std::min(block, cfk::book_block_limit(P->cfg.product, fp64 ? 8 : 4, adj));
     const int waves = P->block / cfk::kWave;

@@ -42,8 +42,9 @@ constexpr double kRecoverVolF64 = 0x1p-10, kRecoverVolF32 = 0x1p-8;
 // barrier and each distinct fixing schedule keeps per-lane state in registers,
 // hence the bounds on them and on the book kernels' blocks.
 constexpr int kMaxBookBarriers = 16, kMaxBookGroups = 4;
-// Bits of a sample's schedule word: every barrier of the book observes at it
-// and none matures; and nothing else happens at it either.
+// Bits of a sample's schedule word: every barrier of the book observes at it,
+// none matures and all have a zone of some width in the kernel's precision;
+// and nothing else happens at it either.
 constexpr uint32_t kBookAllBars = 0x100u, kBookPlain = 0x200u;
 
 // Threads per block of a path kernel: 1024, except the book kernels whose

@@ -1283,7 +1283,7 @@ __device__ __forceinline__ void path_body(const LaunchParams& P, const int bid, 
                     for (int b = 0; b < NBAR; ++b) {
                         if (!(((sm.bars | bl) >> b) & 1u)) continue;
                         const BarPar bp = bar_par(b);
-                        if ((sm.bars >> b) & 1u) {
+                        if (((sm.bars >> b) & 1u) && F > bp.lo) {
                             R t = bp.up - F;
                             if constexpr (ZT) mark_zero(b, t);
                             bst[b] = bar_update(bst[b], t, bp.i2s);
