@@ -1679,7 +1679,7 @@ __device__ __forceinline__ void path_body(const LaunchParams& P, const int bid, 
                 const R F = DUP ? state_spot(x, s0) : ps.fin_f, k = R(P.strike);
                 const bool in = PRD == PRD_BARRIER && P.put ? k > F : F > k;
                 const bool zero = PRD == PRD_EUROPEAN ? ns == 1 && !in : !in || (ps.dead && w1 == R(0));
-                live = active && !(zero && x - x == R(0) && F - F == R(0) && w0 - w0 == R(0));
+                live = active && !(zero && x - x == R(0) && F - F == R(0) && (w0 + w1) - (w0 + w1) == R(0));
             }
             // PK: the swept paths of up to ck_slots blocks are gathered, each
             // lane of a sweep reading the checkpoints and the end state of its

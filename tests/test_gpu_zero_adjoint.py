@@ -58,3 +58,18 @@ def test_paths_of_several_blocks_are_swept_together(engine, n, first, strike, we
         total = total + m * cf.mcParallelSimulAAD(
             prd, mdl, num=cf.NumericalParam(numPath=m, firstPath=first + lo), weights=weights).risks
     assert np.abs(res.risks - total / n).max() <= 1e-11 * np.abs(total / n).max()
+
+
+@pytest.mark.parametrize("mode", [cf.AAD_CHECKPOINT, cf.AAD_RECOMPUTE])
+@pytest.mark.parametrize("precision", [cf.FP64, cf.FP32])
+@pytest.mark.parametrize("bad", [np.inf, np.nan])
+@pytest.mark.parametrize("model", ["dupire", "bs"])
+def test_weights_out_of_range_show(engine, model, bad, precision, mode):
+    """A weight that is not finite makes the risks NaN on a path out of the money
+    too (0 times it), so no path is left out: risks of a strike no path reaches."""
+    mdl = cf.Dupire(**W.dupire_args(30)) if model == "dupire" else cf.BlackScholes(100.0, 0.2, False, 0.01, 0.0)
+    prd = cf.UOC(**W.barrier_args(strike=1.0e4, maturity=0.2))
+    num = cf.NumericalParam(numPath=200, precision=precision, aadMode=mode)
+    for weights in ([1.0, bad], [bad, 0.5]):
+        assert np.isnan(cf.mcParallelSimulAAD(prd, mdl, weights=weights, num=num).risks[0])
+    assert np.all(cf.mcParallelSimulAAD(prd, mdl, weights=[1.0, 0.5], num=num).risks == 0.0)
