@@ -1145,7 +1145,9 @@ cfk::LaunchParams launch_params(const Engine& E, const Prepared& PR, const CallS
     P.pay_strike = reinterpret_cast<const double*>(dt + PR.o_pk);
     P.book = dt + PR.o_book;
     P.bk = PR.book.L;
-    if (PR.cfg.product == cfk::PRD_BOOK) {
+    if (PR.cfg.product == cfk::PRD_BOOK && md.kind != CF_MODEL_DUPIRE) {
+        P.bar_xlo = PR.book.lo_min;
+    } else if (PR.cfg.product == cfk::PRD_BOOK) {
         P.bar_xlo = PR.book.lo_min > 0 ? std::log(S.fp64 ? PR.book.lo_min : PR.book.lo_min / md.spot) : -HUGE_VAL;
         if (std::isfinite(P.bar_xlo)) P.bar_xlo -= (S.fp64 ? 1e-10 : 1e-4) * (1 + std::fabs(P.bar_xlo));
     }

@@ -167,7 +167,8 @@ struct LaunchParams {
     double strike;
     double bar_smooth, minus_smooth, two_smooth, inv_two_smooth;
     double bar_xlo;              // Dupire barrier and book: at or below this state the spot is under
-                                 // every smoothing zone (with a margin over exp's rounding)
+                                 // every smoothing zone (with a margin over exp's rounding); a book on
+                                 // Black-Scholes: the lowest B - w, as a forward
     const int* pay_first;        // Europeans [n_samples + 1]: payoffs of sample s; a book on Dupire:
                                  // [n_steps + 1][4], its rows (BookLayout::masks) by timeline point
     const double* pay_strike;    // Europeans [n_pay]

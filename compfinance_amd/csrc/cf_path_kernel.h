@@ -587,30 +587,36 @@ __device__ __forceinline__ void sobol_stage_lo(uint32_t* lo_tab, const uint32_t*
         // word e: rows dimension e >> 6, lane e & 63; quads dimension
         // 4 (e >> 8) + (e & 3), lane (e >> 2) & 63; split dimension
         // 4 (e >> 6) + (e & 3), entry (e >> 2) & 15 (lane % 8, then 8 + lane / 8)
-        constexpr int kBatch = 4;
         const int total = sobol_dims4(n) * (LO == kLoSplit ? 16 : kWave);
-        for (int e0 = tid; e0 < total; e0 += kBatch * nthr) {
-            uint32_t v[kBatch][6], g[kBatch];
-            int dim[kBatch];
+        auto stage = [&](auto batch) {
+            constexpr int kBatch = decltype(batch)::value;
+            for (int e0 = tid; e0 < total; e0 += kBatch * nthr) {
+                uint32_t v[kBatch][6], g[kBatch];
+                int dim[kBatch];
 #pragma unroll
-            for (int b = 0; b < kBatch; ++b) {
-                const int e = e0 + b * nthr;
-                const int o = (e >> 2) & 15;
-                const int r = LO == kLoSplit ? (o < 8 ? o : (o - 8) << 3) : LO == kLoQuads ? (e >> 2) & 63 : e & 63;
-                dim[b] = LO == kLoSplit ? ((e >> 6) << 2) + (e & 3) : LO == kLoQuads ? ((e >> 8) << 2) + (e & 3) : e >> 6;
-                g[b] = uint32_t(r ^ (r >> 1));
-                const uint32_t d = uint32_t(min(dim[b], n - 1));
+                for (int b = 0; b < kBatch; ++b) {
+                    const int e = e0 + b * nthr;
+                    const int o = (e >> 2) & 15;
+                    const int r = LO == kLoSplit ? (o < 8 ? o : (o - 8) << 3) : LO == kLoQuads ? (e >> 2) & 63 : e & 63;
+                    dim[b] = LO == kLoSplit ? ((e >> 6) << 2) + (e & 3) : LO == kLoQuads ? ((e >> 8) << 2) + (e & 3) : e >> 6;
+                    g[b] = uint32_t(r ^ (r >> 1));
+                    const uint32_t d = uint32_t(min(dim[b], n - 1));
 #pragma unroll
-                for (int k = 0; k < 6; ++k) v[b][k] = (dirs + k * kSobolDims)[d];
+                    for (int k = 0; k < 6; ++k) v[b][k] = (dirs + k * kSobolDims)[d];
+                }
+#pragma unroll
+                for (int b = 0; b < kBatch; ++b) {
+                    uint32_t x = 0;
+#pragma unroll
+                    for (int k = 0; k < 6; ++k) x ^= v[b][k] & uint32_t(-int((g[b] >> k) & 1u));
+                    if (dim[b] < n) lo_tab[e0 + b * nthr] = x;
+                }
             }
-#pragma unroll
-            for (int b = 0; b < kBatch; ++b) {
-                uint32_t x = 0;
-#pragma unroll
-                for (int k = 0; k < 6; ++k) x ^= v[b][k] & uint32_t(-int((g[b] >> k) & 1u));
-                if (dim[b] < n) lo_tab[e0 + b * nthr] = x;
-            }
-        }
+        };
+        // (a few steps, at most one word a thread: 18 loads less each; 5 steps
+        // on 2^10 paths, FP32 risk 20.6 -> 19.9 us)
+        if (total <= nthr) stage(std::integral_constant<int, 1>{});
+        else stage(std::integral_constant<int, 4>{});
     }
 }
 
@@ -1096,6 +1102,10 @@ __device__ __forceinline__ void path_body(const LaunchParams& P, const int bid, 
         }
     };
     const R bk_xlo = BOOK && DUP ? R(P.bar_xlo) : R(0);   // every zone is above this state
+    // Black-Scholes: and above this forward, one test a sample where the fours
+    // load and test four (5 steps, a book of 2 barriers, 2^22 FP32 paths: risk
+    // 208 -> 198 us)
+    const R bk_lo = BOOK && !DUP ? R(P.bar_xlo) : R(0);
 
     // PK: swept paths waiting for a full wave, in lanes 0 .. pk_n - 1 of pk_src
     // (lane of the block, slot << 6, count of zero factors << 28, breached
@@ -1252,7 +1262,7 @@ __device__ __forceinline__ void path_body(const LaunchParams& P, const int bid, 
                 // but costs more scalar work and branches than it saves.
                 const uint32_t bl = sm.bars >> 16;
                 const bool all_bars = (sm.grps & kBookAllBars) != 0;
-                if (all_bars) {
+                if (all_bars && (DUP || __builtin_amdgcn_ballot_w64(F > bk_lo) != 0)) {
 #pragma unroll
                     for (int b = 0; b + 3 < NBAR; b += 4) {
                         if (__builtin_amdgcn_ballot_w64(F > bk_four_c[b >> 2].lo_min[0]) == 0) continue;
@@ -1777,12 +1787,18 @@ __device__ __forceinline__ void path_body(const LaunchParams& P, const int bid, 
             if constexpr (BOOK) {
                 float lo_min = INFINITY;
 #pragma unroll
-                for (int b = 0; b < NBAR; ++b) {
-                    const float lo = float(bk_four_c[b >> 2].lo[b & 3]);
-                    const float th = sizeof(R) == 4 ? lo : lo - 1e-6f * fabsf(lo);
-                    if constexpr (LAZY) rth[b] = bst[b] > R(0) ? th : INFINITY;
-                    else rth[b] = bst[b] > R(0) && babar[b] != R(0) ? th : INFINITY;
-                    lo_min = fminf(lo_min, rth[b]);
+                for (int b0 = 0; b0 + 3 < NBAR; b0 += 4) {
+#pragma unroll
+                    for (int b = b0; b < b0 + 4; ++b) rth[b] = INFINITY;
+                    if (b0 >= P.bk.n_bar) continue;
+#pragma unroll
+                    for (int b = b0; b < b0 + 4; ++b) {
+                        const float lo = float(bk_four_c[b >> 2].lo[b & 3]);
+                        const float th = sizeof(R) == 4 ? lo : lo - 1e-6f * fabsf(lo);
+                        if constexpr (LAZY) rth[b] = bst[b] > R(0) ? th : INFINITY;
+                        else rth[b] = bst[b] > R(0) && babar[b] != R(0) ? th : INFINITY;
+                        lo_min = fminf(lo_min, rth[b]);
+                    }
                 }
                 rv_lo = R(lo_min);
                 if constexpr (DUP) {
@@ -1858,7 +1874,8 @@ __device__ __forceinline__ void path_body(const LaunchParams& P, const int bid, 
                     const uint32_t bm = sm.bars & 0xffffu;
                     uint32_t bl = sm.bars >> 16;
                     const float Ff = float(F);
-                    if (bl) {
+                    const bool above = bm && __builtin_amdgcn_ballot_w64(F > rv_lo) != 0;
+                    if (bl || (!DUP && above)) {
                         // (opaque: the tests of the mask's bits stay here,
                         // where some barrier matures)
                         asm volatile("" : "+s"(bl));
@@ -1881,10 +1898,14 @@ __device__ __forceinline__ void path_body(const LaunchParams& P, const int bid, 
                             }
                             if (Ff > rth[b] && F > bp.lo && ((bm >> b) & 1u)) zone_adj(b, bp.up, bp.i2s);
                         }
-                    } else if (bm && __builtin_amdgcn_ballot_w64(F > rv_lo) != 0) {
+                    } else if (DUP && above) {
                         // some lane is above the lowest zone that its path
                         // has an adjoint in (one sample in three of the
-                        // 55-payoff book); then few barriers have one
+                        // 55-payoff book); then few barriers have one.
+                        // (Black-Scholes takes the loop above for both, a copy
+                        // of the zones' code less in kernels of some 90 KB
+                        // beside an instruction cache of 64: FP64 risk of 5
+                        // steps 98 -> 95 us.)
 #pragma unroll
                         for (int b = 0; b < NBAR; ++b) {
                             if (Ff > rth[b]) {
@@ -2475,16 +2496,18 @@ __device__ __forceinline__ void path_body(const LaunchParams& P, const int bid, 
 #endif
 
 // Waves a SIMD has to hold at least (beside those that a block implies): the
-// FP32 recompute book on Black-Scholes, bound by its waves, takes 133 registers
-// without the limit, three waves instead of four (2^19 mrg32k3a paths of 5
-// steps: 147 against 112 us).
-constexpr int min_waves(int model, int prd, int real_bytes, int adj)
+// FP32 recompute book on Black-Scholes with mrg32k3a normals, bound by its
+// waves, takes more than 128 registers without the limit, three waves instead
+// of four (2^19 paths, 5 steps 124 against 92 us, 52 steps 409 against 264).
+// The Sobol kernel needs 120 by itself, and the limit only costs it (5 steps
+// 53.7 against 51.5 us, 52 steps 211 against 190).
+constexpr int min_waves(int model, int prd, int real_bytes, int adj, bool mrg)
 {
-    return model == MODEL_BS && prd == PRD_BOOK && real_bytes == 4 && adj == ADJ_RECOMPUTE ? 4 : 1;
+    return model == MODEL_BS && prd == PRD_BOOK && real_bytes == 4 && adj == ADJ_RECOMPUTE && mrg ? 4 : 1;
 }
 
 template <typename R, int MODEL, int PRD, int ADJ, bool LEAN, bool MRG, bool ITEM>
-__global__ void __launch_bounds__(book_block_limit(PRD, int(sizeof(R)), ADJ), min_waves(MODEL, PRD, int(sizeof(R)), ADJ))
+__global__ void __launch_bounds__(book_block_limit(PRD, int(sizeof(R)), ADJ), min_waves(MODEL, PRD, int(sizeof(R)), ADJ, MRG))
 CF_PATH_KERNEL_ATTR path_kernel(const LaunchParams P)
 {
     path_body<R, MODEL, PRD, ADJ, LEAN, MRG, ITEM>(P, int(blockIdx.x), int(gridDim.x));
