@@ -88,6 +88,18 @@ void hip_check(hipError_t e, const char* what)
     if (e != hipSuccess) fail(CF_ERR_DEVICE, string(what) + ": " + hipGetErrorString(e));
 }
 
+void* dev_malloc(size_t bytes, const char* what)
+{
+    void* p = nullptr;
+    const hipError_t e = hipMalloc(&p, bytes);
+    if (e == hipErrorOutOfMemory) {
+        (void)hipGetLastError();   // (not the next launch's)
+        throw OutOfMemory(CF_ERR_DEVICE, string(what) + ": " + hipGetErrorString(e));
+    }
+    hip_check(e, what);
+    return p;
+}
+
 string fmt2(double x)
 {
     std::ostringstream o;
@@ -1055,19 +1067,21 @@ CallShape shape_call(const Engine& E, const Prepared& PR, const cf_num* num, boo
     return S;
 }
 
-void add_ck_slots(const Prepared& PR, size_t limit, CallShape* S)
+CallShape shape_sync(const Engine& E, const Prepared& PR, const cf_num* num, bool adjoint)
 {
+    CallShape S = shape_call(E, PR, num, adjoint);
     // (a redrawn normal would need the words of each path's own block)
     const bool product = PR.cfg.product == cfk::PRD_BARRIER ||
                          (PR.cfg.product == cfk::PRD_EUROPEAN && PR.pd.timeline.size() == 1);
-    if (!S->adjoint || !S->fp64 || PR.md.kind != CF_MODEL_DUPIRE || PR.cfg.recompute || !product || !PR.iv_recover ||
-        S->slots == 0)
-        return;
-    const int64_t q0 = (S->first + 1) >> 6, q1 = (S->first + S->n_path) >> 6;
-    const int64_t blocks = q1 - q0 + 1 - (S->merge ? 1 : 0);
-    const size_t one = call_bytes(*S).ckpt / size_t(S->ck_slots);
-    S->ck_slots = int(std::max<int64_t>(1, std::min({int64_t(cfk::kMaxCkSlots), (blocks + S->slots - 1) / S->slots,
-                                                     one ? int64_t(limit / one) : int64_t(1)})));
+    if (!S.adjoint || !S.fp64 || PR.md.kind != CF_MODEL_DUPIRE || PR.cfg.recompute || !product || !PR.iv_recover ||
+        S.slots == 0)
+        return S;
+    const int64_t q0 = (S.first + 1) >> 6, q1 = (S.first + S.n_path) >> 6;
+    const int64_t blocks = q1 - q0 + 1 - (S.merge ? 1 : 0);
+    const size_t one = call_bytes(S).ckpt;
+    S.ck_slots = int(std::max<int64_t>(1, std::min({int64_t(cfk::kMaxCkSlots), (blocks + S.slots - 1) / S.slots,
+                                                    one ? int64_t(kCkSlotsBytes / one) : int64_t(1)})));
+    return S;
 }
 
 static size_t al256(size_t x) { return (x + 255) & ~size_t(255); }
@@ -1265,6 +1279,54 @@ int adjoint_kind(const Call& c)
     return c.num->aad_mode == CF_AAD_RECOMPUTE ? cfk::ADJ_RECOMPUTE : cfk::ADJ_CHECKPOINT;
 }
 
+// The buffers of a synchronous call, the engine's own.  Slots beyond one a wave
+// are taken where the memory that the call adds leaves seven times as much
+// free; if memory does not last all the same, the call runs with one, after
+// the engine has given back its spare buffers.
+static CallBuffers sync_buffers(Engine& E, const Prepared& PR, CallShape* S, bool per_path, bool per_path_agg)
+{
+    const size_t pp = per_path ? size_t(S->n_path) * S->npay * 8 : 0, pa = per_path_agg ? size_t(S->n_path) * 8 : 0;
+    if (S->ck_slots > 1) {
+        const CallBytes nb = call_bytes(*S);
+        if (E.ckpt.growth(nb.ckpt) > 0) {
+            const size_t grows = E.ckpt.growth(nb.ckpt) + E.block_out.growth(nb.block_out) +
+                                 E.ivbar_blocks.growth(nb.ivbar_blocks) + E.weights.growth(nb.weights) +
+                                 E.per_path.growth(pp) + E.per_path_agg.growth(pa);
+            size_t free_b = 0, total_b = 0;
+            hip_check(hipMemGetInfo(&free_b, &total_b), "hipMemGetInfo");
+            if (grows > free_b / 8) S->ck_slots = 1;
+        }
+    }
+    auto take = [&] {
+        const CallBytes nb = call_bytes(*S);
+        CallBuffers B;
+        B.tables = static_cast<const unsigned char*>(PR.tables.p);
+        B.block_out = static_cast<double*>(E.block_out.ensure(nb.block_out));
+        // the reduced sums and the local-vol adjoints side by side, written by the
+        // reduction straight into mapped host memory
+        E.pin_out.ensure((size_t(S->stride) + S->ivn) * 8);
+        B.reduced = static_cast<double*>(E.pin_out.dev);
+        if (S->ivn) {
+            B.ivbar_blocks = static_cast<double*>(E.ivbar_blocks.ensure(nb.ivbar_blocks));
+            B.ivbar = B.reduced + S->stride;
+        }
+        if (S->adjoint) {
+            B.weights = static_cast<double*>(E.weights.ensure(nb.weights));
+            B.ckpt = E.ckpt.ensure(nb.ckpt);
+        }
+        if (per_path) B.per_path = static_cast<double*>(E.per_path.ensure(pp));
+        if (per_path_agg) B.per_path_agg = static_cast<double*>(E.per_path_agg.ensure(pa));
+        return B;
+    };
+    try {
+        return take();
+    } catch (const OutOfMemory&) {
+        E.give_back_spare();
+        S->ck_slots = 1;
+        return take();
+    }
+}
+
 // Synchronous call on the engine's own stream and buffers.
 int run(const cf_model* mdl, const cf_product* prd, Call& c)
 {
@@ -1276,36 +1338,13 @@ int run(const cf_model* mdl, const cf_product* prd, Call& c)
     Engine& E = engine();
     std::lock_guard<std::mutex> lk(E.sync_mu);
     hip_check(hipSetDevice(E.device), "hipSetDevice");
-    const std::shared_ptr<Prepared> PP = lookup(E, mdl, prd, fp64, adjoint_kind(c), true, call_block(E, c.num, fp64));
+    const std::shared_ptr<Prepared> PP = E.with_spare(
+        [&] { return lookup(E, mdl, prd, fp64, adjoint_kind(c), true, call_block(E, c.num, fp64)); });
     const Prepared& PR = *PP;
-    CallShape S = shape_call(E, PR, c.num, c.adjoint);
-    add_ck_slots(PR, kCkSlotsBytes, &S);
-    if (S.ck_slots > 1 && call_bytes(S).ckpt > E.ckpt.cap) {
-        // (as many as the device's memory holds)
-        size_t free_b = 0, total_b = 0;
-        hip_check(hipMemGetInfo(&free_b, &total_b), "hipMemGetInfo");
-        if (call_bytes(S).ckpt + (size_t(256) << 20) > free_b + E.ckpt.cap) S.ck_slots = 1;
-    }
-    const CallBytes nb = call_bytes(S);
-
+    CallShape S = shape_sync(E, PR, c.num, c.adjoint);
     double* h_in = static_cast<double*>(E.pin_in.ensure(size_t(S.npay) * 8));
-    double* h_out = static_cast<double*>(E.pin_out.ensure((size_t(S.stride) + S.ivn) * 8));
-    CallBuffers B;
-    B.tables = static_cast<const unsigned char*>(PR.tables.p);
-    B.block_out = static_cast<double*>(E.block_out.ensure(nb.block_out));
-    // the reduced sums and the local-vol adjoints side by side, written by the
-    // reduction straight into mapped host memory
-    B.reduced = static_cast<double*>(E.pin_out.dev);
-    if (S.ivn) {
-        B.ivbar_blocks = static_cast<double*>(E.ivbar_blocks.ensure(nb.ivbar_blocks));
-        B.ivbar = B.reduced + S.stride;
-    }
-    if (c.adjoint) {
-        B.weights = static_cast<double*>(E.weights.ensure(nb.weights));
-        B.ckpt = E.ckpt.ensure(nb.ckpt);
-    }
-    if (c.per_path) B.per_path = static_cast<double*>(E.per_path.ensure(size_t(S.n_path) * S.npay * 8));
-    if (c.per_path_agg) B.per_path_agg = static_cast<double*>(E.per_path_agg.ensure(size_t(S.n_path) * 8));
+    const CallBuffers B = sync_buffers(E, PR, &S, c.per_path != nullptr, c.per_path_agg != nullptr);
+    double* h_out = static_cast<double*>(E.pin_out.p);
 
     hip_check(hipEventRecord(E.ev[0], E.stream), "hipEventRecord");
     bool uploads = false;
@@ -1406,8 +1445,10 @@ int cf_sobol_points(int64_t first_path, int64_t n_paths, int dim, int precision,
         struct Owned : DevBuf {
             ~Owned() { if (p) (void)hipFree(p); }
         } dw, dn;
-        if (words) dw.ensure(n * 4);
-        if (normals) dn.ensure(n * size_t(rb));
+        E.with_spare([&] {
+            if (words) dw.ensure(n * 4);
+            if (normals) dn.ensure(n * size_t(rb));
+        });
         const int rc = cfk::launch_sobol_points(rb, layout, E.d_dirs, dim, first_path, n_paths,
                                                 static_cast<uint32_t*>(dw.p), dn.p, E.stream);
         if (rc != 0) hip_check(hipError_t(rc), "Sobol points launch");
@@ -1626,6 +1667,19 @@ struct ItemTables {
     }
 };
 
+// Whether `bytes` fit the free device memory with 256 MiB to spare, without the
+// checkpoints of earlier calls if need be.
+static bool fits_free(Engine& E, size_t bytes)
+{
+    for (;;) {
+        size_t free_b = 0, total_b = 0;
+        hip_check(hipMemGetInfo(&free_b, &total_b), "hipMemGetInfo");
+        if (bytes + (size_t(256) << 20) <= free_b) return true;
+        if (!E.ckpt.p) return false;
+        E.ckpt.give_back();
+    }
+}
+
 // Itemized risk of a Europeans product on Dupire: the calls of a maturity
 // share their sweeps (cf_itemized.hip).  The caller holds the engine's lock.
 // Returns false, doing nothing, where its kernels do not apply: grids of more
@@ -1680,11 +1734,19 @@ static bool run_multi_europeans(Engine& E, const Prepared& PR, const CallShape& 
     DevBuf& buf = total <= Engine::kItemKeep ? E.item : static_cast<DevBuf&>(once);
     if (total > buf.cap) {
         E.item.give_back();
-        size_t free_b = 0, total_b = 0;
-        hip_check(hipMemGetInfo(&free_b, &total_b), "hipMemGetInfo");
-        if (total + (size_t(256) << 20) > free_b) return false;
+        if (!fits_free(E, total)) return false;
     }
-    unsigned char* d = static_cast<unsigned char*>(buf.ensure(total));
+    const CallBytes nb = call_bytes(S);
+    try {
+        E.block_out.ensure(nb.block_out);
+        E.ivbar_blocks.ensure(nb.ivbar_blocks);
+        E.weights.ensure(nb.weights);
+        buf.ensure(total);
+    } catch (const OutOfMemory&) {
+        E.give_back_spare();
+        return false;
+    }
+    unsigned char* d = static_cast<unsigned char*>(buf.p);
     DevBuf& tab = const_cast<Prepared&>(PR).item;   // (under the engine's lock)
     if (!tab.p) {
         tab.ensure(T.st.bytes.size());
@@ -1693,14 +1755,13 @@ static bool run_multi_europeans(Engine& E, const Prepared& PR, const CallShape& 
     const unsigned char* dt = static_cast<const unsigned char*>(tab.p);
 
     // the forward: payoff means, checkpoints and end states
-    const CallBytes nb = call_bytes(S);
     double* h_out = static_cast<double*>(E.pin_out.ensure((size_t(S.stride) + S.ivn) * 8));
     double* h_in = static_cast<double*>(E.pin_in.ensure(size_t(S.npay) * 8));
     CallBuffers B;
     B.tables = static_cast<const unsigned char*>(PR.tables.p);
-    B.block_out = static_cast<double*>(E.block_out.ensure(nb.block_out));
+    B.block_out = static_cast<double*>(E.block_out.p);
     B.reduced = static_cast<double*>(E.pin_out.dev);
-    B.weights = static_cast<double*>(E.weights.ensure(nb.weights));
+    B.weights = static_cast<double*>(E.weights.p);
     B.ckpt = d + o_ck;
     E.weights_on_device = nullptr;   // this call rewrites the weights buffer
     std::fill(h_in, h_in + S.npay, 0.0);
@@ -1711,7 +1772,6 @@ static bool run_multi_europeans(Engine& E, const Prepared& PR, const CallShape& 
     Sequence q;
     CallShape S_fwd = S;
     S_fwd.ivn = 0;   // (no adjoint grids to sum)
-    E.ivbar_blocks.ensure(nb.ivbar_blocks);
     P.ivbar_blocks = static_cast<double*>(E.ivbar_blocks.p);
     make_sequence(PR, S_fwd, B, P, &q);
     q.cfg.item = true;
@@ -1781,8 +1841,8 @@ bool run_multi(const cf_model* mdl, const cf_product* prd, const cf_num* num, do
     Engine& E = engine();
     std::lock_guard<std::mutex> lk(E.sync_mu);
     hip_check(hipSetDevice(E.device), "hipSetDevice");
-    const std::shared_ptr<Prepared> PP =
-        lookup(E, mdl, prd, fp64, cfk::ADJ_CHECKPOINT, true, call_block(E, num, fp64));
+    const std::shared_ptr<Prepared> PP = E.with_spare(
+        [&] { return lookup(E, mdl, prd, fp64, cfk::ADJ_CHECKPOINT, true, call_block(E, num, fp64)); });
     const Prepared& PR = *PP;
     const CallShape S = shape_call(E, PR, num, true);
     if (run_multi_europeans(E, PR, S, num, payoff_means, risks)) return true;
@@ -1793,26 +1853,28 @@ bool run_multi(const cf_model* mdl, const cf_product* prd, const cf_num* num, do
     const size_t rb = fp64 ? 8 : 4;
     const size_t ck_bytes = blocks64 * size_t(S.ck_rows) * cfk::kWave * rb;
     const size_t st_bytes = blocks64 * size_t(cfk::state_rows(PR.cfg.product == cfk::PRD_BOOK)) * cfk::kWave * rb;
-    size_t free_b = 0, total_b = 0;
-    hip_check(hipMemGetInfo(&free_b, &total_b), "hipMemGetInfo");
-    if (ck_bytes + st_bytes + (size_t(256) << 20) > free_b) return false;
+    if (!fits_free(E, ck_bytes + st_bytes)) return false;
 
     struct Owned : DevBuf {
         ~Owned() { if (p) (void)hipFree(p); }
     } ckb, stb;
-    ckb.ensure(ck_bytes);
-    stb.ensure(st_bytes);
     CallBuffers B;
     B.tables = static_cast<const unsigned char*>(PR.tables.p);
-    B.block_out = static_cast<double*>(E.block_out.ensure(nb.block_out));
-    B.reduced = static_cast<double*>(E.reduced.ensure((size_t(S.stride) + S.ivn) * 8));
-    if (S.ivn) {
-        B.ivbar_blocks = static_cast<double*>(E.ivbar_blocks.ensure(nb.ivbar_blocks));
-        B.ivbar = B.reduced + S.stride;
+    try {
+        B.ckpt = ckb.ensure(ck_bytes);
+        stb.ensure(st_bytes);
+        B.block_out = static_cast<double*>(E.block_out.ensure(nb.block_out));
+        B.reduced = static_cast<double*>(E.reduced.ensure((size_t(S.stride) + S.ivn) * 8));
+        if (S.ivn) {
+            B.ivbar_blocks = static_cast<double*>(E.ivbar_blocks.ensure(nb.ivbar_blocks));
+            B.ivbar = B.reduced + S.stride;
+        }
+        B.weights = static_cast<double*>(E.weights.ensure(nb.weights));
+    } catch (const OutOfMemory&) {
+        E.give_back_spare();
+        return false;
     }
-    B.weights = static_cast<double*>(E.weights.ensure(nb.weights));
     E.weights_on_device = nullptr;   // this call rewrites the weights buffer
-    B.ckpt = ckb.p;
     cfk::LaunchParams P = launch_params(E, PR, S, B);
     P.state = stb.p;
 
@@ -1902,7 +1964,7 @@ int64_t cf_aad_footprint(const cf_model* mdl, const cf_product* prd, const cf_nu
         const bool fp64 = num->precision == CF_FP64;
         const int adj = num->aad_mode == CF_AAD_RECOMPUTE ? cfk::ADJ_RECOMPUTE : cfk::ADJ_CHECKPOINT;
         const std::shared_ptr<Prepared> P = lookup(E, mdl, prd, fp64, adj, false, call_block(E, num, fp64));
-        bytes = int64_t(call_bytes(shape_call(E, *P, num, true)).total() + P->staged.size());
+        bytes = int64_t(call_bytes(shape_sync(E, *P, num, true)).total() + P->staged.size());
         return CF_OK;
     });
     return rc == CF_OK ? bytes : int64_t(rc);

@@ -40,6 +40,12 @@ struct CfError : std::runtime_error {
     CfError(int c, const string& m) : std::runtime_error(m), code(c) {}
 };
 
+// A device allocation that failed: the caller may give back what it can spare
+// and try again.
+struct OutOfMemory : CfError {
+    using CfError::CfError;
+};
+
 [[noreturn]] void fail(int code, const string& msg);
 void hip_check(hipError_t e, const char* what);
 
@@ -133,6 +139,9 @@ struct BucketTable {
 
 // ------------------------------------------------------------------ device
 
+// Device memory; OutOfMemory when there is not enough.
+void* dev_malloc(size_t bytes, const char* what);
+
 // Grow-only device buffer.
 struct DevBuf {
     void* p = nullptr;
@@ -144,10 +153,12 @@ struct DevBuf {
         p = nullptr;
         cap = 0;
         size_t want = std::max<size_t>(bytes, 256);
-        hip_check(hipMalloc(&p, want), "hipMalloc");
+        p = dev_malloc(want, "hipMalloc");
         cap = want;
         return p;
     }
+    // what ensure(bytes) adds to the device memory taken
+    size_t growth(size_t bytes) const { return bytes > cap ? bytes - cap : 0; }
     void give_back()
     {
         if (p) (void)hipFree(p);
@@ -249,6 +260,24 @@ struct Engine {
     std::list<std::pair<string, std::shared_ptr<Prepared>>> plans;   // most recent first
     std::mutex plan_mu;   // the plan cache
     std::mutex sync_mu;   // the synchronous entry points' stream and buffers
+    // Gives back the largest buffers kept between calls, the checkpoints and
+    // the itemized ones (the caller holds sync_mu; no call is in flight).
+    void give_back_spare()
+    {
+        ckpt.give_back();
+        item.give_back();
+    }
+    // f(); if device memory does not last, once more without the spare buffers.
+    template <class F>
+    auto with_spare(F&& f)
+    {
+        try {
+            return f();
+        } catch (const OutOfMemory&) {
+            give_back_spare();
+            return f();
+        }
+    }
 };
 
 Engine& engine();
@@ -313,9 +342,9 @@ struct CallShape {
 CallShape shape_call(const Engine& E, const Prepared& PR, const cf_num* num, bool adjoint);
 // Checkpoints of the synchronous calls with more than one slot per wave.
 constexpr size_t kCkSlotsBytes = size_t(2) << 30;
-// More checkpoint slots per wave for the kernels that sweep the paths of
-// several blocks together, within `limit` bytes of checkpoints.
-void add_ck_slots(const Prepared& PR, size_t limit, CallShape* S);
+// shape_call of a synchronous call: with more checkpoint slots per wave, within
+// kCkSlotsBytes, for the kernels that sweep the paths of several blocks together.
+CallShape shape_sync(const Engine& E, const Prepared& PR, const cf_num* num, bool adjoint);
 
 // Device buffers of one call.
 struct CallBuffers {

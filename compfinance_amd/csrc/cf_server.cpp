@@ -46,7 +46,7 @@ class Arena {
     void init(size_t bytes)
     {
         cap_ = (bytes + 255) & ~size_t(255);
-        hip_check(hipMalloc(&base_, cap_), "hipMalloc (server arena)");
+        base_ = dev_malloc(cap_, "hipMalloc (server arena)");
         free_[0] = cap_;
     }
     ~Arena()
@@ -722,7 +722,14 @@ int cf_server_create(const cf_server_opts* opts, cf_server** out)
         if (mp < 0 || mp > cfk::kMaxPack) fail(CF_ERR_ARG, "max_pack must be in 0..8");
         S->max_pack = mp == 0 ? cfk::kMaxPack : mp;
         hip_check(hipSetDevice(S->device), "hipSetDevice");
-        S->arena.init(size_t(budget));
+        try {
+            S->arena.init(size_t(budget));
+        } catch (const OutOfMemory&) {
+            // without what the synchronous calls keep between calls
+            std::lock_guard<std::mutex> lk(S->E->sync_mu);
+            S->E->give_back_spare();
+            S->arena.init(size_t(budget));
+        }
         for (int i = 0; i < n_slots; ++i) {
             auto s = std::make_unique<Slot>();
             hip_check(hipStreamCreateWithFlags(&s->stream, hipStreamNonBlocking), "hipStreamCreate");

@@ -179,8 +179,12 @@ int cf_mc_simul_aad_noalloc(const cf_model* mdl, const cf_product* prd, const cf
 int cf_mc_simul_aad_multi(const cf_model* mdl, const cf_product* prd, const cf_num* num,
                           double* payoff_means, double* risks);
 
-/* Device memory one AAD call on this product would take (checkpoint buffers
- * dominate); used for admission.  Bytes, or negative on error. */
+/* Device memory cf_mc_simul_aad takes at most for one call on this product,
+ * per-path outputs aside (checkpoint buffers dominate); used for admission.
+ * FP64 risk of a barrier or a single-date European on Dupire takes up to four
+ * checkpoint slots a wave, at most 2 GiB, where eight times as much memory is
+ * free, else one, and gives them back when memory runs short; served calls and
+ * cf_mc_simul_aad_noalloc always take one.  Bytes, or negative on error. */
 int64_t cf_aad_footprint(const cf_model* mdl, const cf_product* prd, const cf_num* num);
 
 /* ------------------------------------------------------------ store level */
