@@ -1027,10 +1027,7 @@ std::shared_ptr<Prepared> lookup(Engine& E, const cf_model* mdl, const cf_produc
         E.plans.emplace_front(key, P);
         if (E.plans.size() > kMaxPlans) E.plans.pop_back();
     }
-    if (with_tables && !P->tables.p) {
-        P->tables.ensure(P->staged.size());
-        hip_check(hipMemcpy(P->tables.p, P->staged.data(), P->staged.size(), hipMemcpyHostToDevice), "table upload");
-    }
+    if (with_tables && !P->tables.p) P->tables.upload(P->staged);
     return P;
 }
 
@@ -1737,7 +1734,9 @@ static bool run_multi_europeans(Engine& E, const Prepared& PR, const CallShape& 
         if (!fits_free(E, total)) return false;
     }
     const CallBytes nb = call_bytes(S);
+    DevBuf& tab = const_cast<Prepared&>(PR).item;   // (under the engine's lock)
     try {
+        if (!tab.p) tab.upload(T.st.bytes);
         E.block_out.ensure(nb.block_out);
         E.ivbar_blocks.ensure(nb.ivbar_blocks);
         E.weights.ensure(nb.weights);
@@ -1747,11 +1746,6 @@ static bool run_multi_europeans(Engine& E, const Prepared& PR, const CallShape& 
         return false;
     }
     unsigned char* d = static_cast<unsigned char*>(buf.p);
-    DevBuf& tab = const_cast<Prepared&>(PR).item;   // (under the engine's lock)
-    if (!tab.p) {
-        tab.ensure(T.st.bytes.size());
-        hip_check(hipMemcpy(tab.p, T.st.bytes.data(), T.st.bytes.size(), hipMemcpyHostToDevice), "table upload");
-    }
     const unsigned char* dt = static_cast<const unsigned char*>(tab.p);
 
     // the forward: payoff means, checkpoints and end states

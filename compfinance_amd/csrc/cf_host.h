@@ -157,6 +157,14 @@ struct DevBuf {
         cap = want;
         return p;
     }
+    // holds these bytes, or nothing when the copy fails
+    void upload(const vector<unsigned char>& bytes)
+    {
+        ensure(bytes.size());
+        const hipError_t e = hipMemcpy(p, bytes.data(), bytes.size(), hipMemcpyHostToDevice);
+        if (e != hipSuccess) give_back();
+        hip_check(e, "table upload");
+    }
     // what ensure(bytes) adds to the device memory taken
     size_t growth(size_t bytes) const { return bytes > cap ? bytes - cap : 0; }
     void give_back()

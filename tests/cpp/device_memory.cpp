@@ -191,7 +191,7 @@ int main(int argc, char** argv)
         g_hide = true;
         rc = itemized(num);
     } else if (scenario == "upload") {
-        // every upload of the two calls fails once
+        // one upload of the first call fails
         (void)risk(num);
         g_uploads = 0;
         eus.n_options = 2;

@@ -1,8 +1,9 @@
 """The engine's device memory, on the CPU: the library's objects linked with
 stand-ins for the HIP calls that count allocations on a device of a chosen size
 and run no kernel (tests/cpp/device_memory.cpp).  cf_aad_footprint bounds what a
-call takes; a call that needs what earlier ones keep gets it; and a call whose
-larger choice does not fit takes the smaller one."""
+call takes; a call that needs what earlier ones keep gets it; a call whose
+larger choice does not fit takes the smaller one; and tables whose upload failed
+are uploaded again."""
 import json
 import os
 import shutil
@@ -67,3 +68,12 @@ def test_kept_buffers_are_given_back(device, scenario):
 def test_itemized_falls_back(device):
     r = device("itemized_short")
     assert r["rc"] == 1 + 30 * 36 and r["launches"] > 0, r
+
+
+@pytest.mark.parametrize("failing", [1, 2])
+def test_a_failed_upload_is_done_again(device, failing):
+    """An itemized call uploads two tables, those of the plan and its own."""
+    r = device("upload", FP64, CHECKPOINT, 4096, failing)
+    assert r["rc0"] < 0 and r["rc"] > 0, r
+    assert r["before"] == failing                      # (the first call ended at the failing upload)
+    assert r["uploads"] - r["before"] == 3 - failing   # the second did it again, and those after it
