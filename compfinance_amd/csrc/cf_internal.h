@@ -381,8 +381,8 @@ struct KnotSearch {
 
 // #{knots <= x}, exactly as upper_bound (interp.h:40): states below the first
 // knot map to bucket 0, whose count is 0 and whose comparisons all fail.
-// WIDE: tables with more than two knots in a bucket (fix > 2); the FULL layout
-// is only chosen for tables with fix <= 2 and compiles without the loop.
+// WIDE: tables with more than two knots in a bucket (fix > 2) too, as the LEAN
+// kernels take them; without it, tables of at most two.
 template <bool WIDE = true, typename R>
 CF_HD inline int count_le(const KnotSearch<R>& s, R x)
 {
@@ -400,6 +400,15 @@ CF_HD inline int count_le(const KnotSearch<R>& s, R x)
     return c;
 }
 
+// FP32, FULL: the byte offset of the entry of x in a table at `table`, straight
+// from the bucket's bits; at = bucket_base(table), modulo 2^32.
+CF_HD inline uint32_t bucket_base(size_t table) { return uint32_t(table) - (kBucketMagicBits << 3); }
+CF_HD inline uint32_t bucket_offset(float x, float invh, float c0, float top, uint32_t at)
+{
+    static_assert(sizeof(BucketOne<float>) == 8, "eight bytes an entry");
+    return (bucket_bits(x, invh, c0, top) << 3) + at;
+}
+
 // The FULL layout's search (at most one knot a bucket).
 template <typename R>
 CF_HD inline int count_le_one(const BucketOne<R>& e, R x)
@@ -409,7 +418,7 @@ CF_HD inline int count_le_one(const BucketOne<R>& e, R x)
 
 // Host: the knot search table of increasing knots (at least one), in the
 // kernel's real type.  Buckets of width at most half the smallest knot gap
-// (at most 16384 of them), so that normally no more than two knots share one.
+// (at most 16384 of them), so that normally no two knots share one.
 template <typename R>
 struct KnotTable {
     std::vector<BucketEntry<R>> entries;
@@ -633,11 +642,11 @@ int launch_path_kernel(const KernelConfig& cfg, const LaunchParams& p, int grid,
 // (cols1 may be 0), one launch.
 int launch_reduce_rows(const double* in0, int cols0, double* out0, const double* in1, int cols1, double* out1,
                        int rows, void* stream);
-// A packed launch (cfg.packed: Sobol, not itemized) of A.n calls over grid =
-// A.first[A.n] blocks, and the calls' reductions in one launch.
 // The engine's count of blocks done (LaunchParams::blocks_done) on the current
 // device, a module variable.
 int blocks_done_counter(uint32_t** device);
+// A packed launch (cfg.packed: Sobol, not itemized) of A.n calls over grid =
+// A.first[A.n] blocks, and the calls' reductions in one launch.
 int launch_path_kernel_packed(const KernelConfig& cfg, const PackArgs& A, int block, size_t smem, void* stream);
 int launch_reduce_packed(const ReducePack& R, void* stream);
 int path_kernel_occupancy(const KernelConfig& cfg, int block, size_t smem, int* blocks_per_cu);

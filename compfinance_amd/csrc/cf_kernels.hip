@@ -96,10 +96,12 @@ int blocks_done_counter(uint32_t** device)
 // Words and normals of paths [first, first + npath) in dim dimensions, formed
 // exactly as the path kernels form them (sobol_stage_lo, sobol_block,
 // sobol_low_word / sobol_words4, inv_normal); written [path][dim].
-// 256-thread blocks; LDS: LO (rows, split, quads or LEAN), one high row per wave,
-// the tail row, and (FP32 FULL) the inverse-normal table.  The quads and
-// split layouts read dimensions four at a time up to the last whole group, then one at a
-// time, as the FP32 adjoint kernels' forward sweep does.
+// 256-thread blocks; LDS: LO (rows, quads, split or LEAN), one high row per wave,
+// the tail row, and (FP32 FULL) the inverse-normal table.  Quads (FP32) and
+// split (FP64) are the Dupire adjoint kernels' layouts: dimensions read four at a
+// time up to the last whole group, then one at a time, the high words from
+// sixteen direction numbers at once; rows those of the FP64 pricing and the
+// Black-Scholes kernels.
 template <typename R, int LO>
 __global__ void __launch_bounds__(256) sobol_points_kernel(const uint32_t* dirs, int dim, int64_t first, int64_t npath,
                                                            int merge_tail, uint32_t* words, R* normals)
@@ -129,14 +131,15 @@ __global__ void __launch_bounds__(256) sobol_points_kernel(const uint32_t* dirs,
     const bool merge = merge_tail != 0;
     const int64_t qe = merge ? q1 - 1 : q1;
     for (int64_t q = q0 + int64_t(blockIdx.x) * waves + wave; q <= qe; q += int64_t(gridDim.x) * waves) {
-        const SobolLane sl = sobol_block(hi, hi_tail, dirs, dim, q, q0, q1, nlo, nhi, merge, lane, true);
+        constexpr bool FOURS = LO == kLoQuads || LO == kLoSplit;
+        const SobolLane sl = sobol_block<FOURS>(hi, hi_tail, dirs, dim, q, q0, q1, nlo, nhi, merge, lane, true);
         if (sl.active) {
             auto put = [&](int i, uint32_t w) {
                 if (words) words[size_t(sl.pidx) * dim + i] = w;
                 if (normals) normals[size_t(sl.pidx) * dim + i] = inv_normal(w, tab);
             };
             int i = 0;
-            if constexpr (LO == kLoQuads || LO == kLoSplit) {
+            if constexpr (FOURS) {
                 for (; i + 4 <= dim; i += 4) {
                     uint32_t w4[4];
                     sobol_words4<LO>(lo_tab, sl.hl, lane, i, w4);
@@ -171,9 +174,8 @@ int launch_sobol_points(int real_bytes, int layout, const uint32_t* dirs, int di
     auto pick = [&](auto real) -> const void* {
         using T = decltype(real);
         if (layout == kLoLean) return reinterpret_cast<const void*>(&sobol_points_kernel<T, kLoLean>);
-        if (layout == kLoQuads) return reinterpret_cast<const void*>(&sobol_points_kernel<T, kLoQuads>);
-        // (FULL as the Dupire kernels of the precision hold it)
-        return reinterpret_cast<const void*>(&sobol_points_kernel<T, sizeof(T) == 8 ? kLoSplit : kLoRows>);
+        if (layout == kLoRows) return reinterpret_cast<const void*>(&sobol_points_kernel<T, kLoRows>);
+        return reinterpret_cast<const void*>(&sobol_points_kernel<T, sizeof(T) == 8 ? kLoSplit : kLoQuads>);
     };
     f = real_bytes == 4 ? pick(0.0f) : pick(0.0);
     if (smem > 65536) {

@@ -973,12 +973,12 @@ __device__ __forceinline__ void path_body(const LaunchParams& P, const int bid, 
     ks.itop = P.n_buckets - 1;
     // number of knots <= x.  FP32: the entry's address straight from the
     // bucket's bits
-    const uint32_t bucket_at = uint32_t(L.bucket) - (kBucketMagicBits << 3);
+    const uint32_t bucket_at = bucket_base(L.bucket);
     auto knot_count = [&](R x) -> int {
         if constexpr (LEAN) {
             return count_le<true>(ks, x);
         } else if constexpr (sizeof(R) == 4) {
-            const uint32_t off = (bucket_bits(x, ks.invh, ks.c0, ks.top) << 3) + bucket_at;
+            const uint32_t off = bucket_offset(x, ks.invh, ks.c0, ks.top, bucket_at);
             return count_le_one(*reinterpret_cast<const BucketOne<R>*>(smem + off), x);
         } else {
             return count_le_one(bucket[bucket_index(x, ks.invh, ks.c0, ks.top, ks.itop)], x);

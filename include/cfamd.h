@@ -428,8 +428,9 @@ int cf_device_synchronize(void);
  * FP64, the kernels' table form in FP32 (nullable).  layout: 0 the kernels'
  * FULL form (low words staged per lane, [dimension][lane]), 1 LEAN (formed
  * from six direction numbers), 2 FULL interleaved by groups of four
- * dimensions and read four at a time (the FP32 adjoint kernels' form), -1
- * FULL when its tables fit the block's shared memory. */
+ * dimensions and read four at a time (the Dupire adjoint kernels' forms: FP32
+ * a word per lane, FP64 two words of sixteen), -1 FULL when its tables fit the
+ * block's shared memory. */
 int cf_sobol_points(int64_t first_path, int64_t n_paths, int dim, int precision, int layout, uint32_t* words,
                     void* normals);
 
