@@ -450,11 +450,13 @@ __device__ __forceinline__ double exp_series(double d)
     return fma(q, d, 0.5);
 }
 // exp in FP64 by Cody and Waite's reduction: x = n ln(2) + d,
-// 2^n (1 + (d + d^2 series)), within 0.8 ulp; x beyond +-800 saturates to 0 or
-// infinity, and a NaN stays one (v_max_f64 would drop it: under -800 the high
-// word is replaced instead, by that of -800; above 800 only n is bounded, d
-// overflows).  23 instructions, no table (a load would wait for the checkpoint
-// stores issued before it), against the library function's 35.
+// 2^n (1 + d (1 + d series)), the last step rounded once: within 0.85 ulp, 0.257
+// on average, over 2^21 arguments of -30 to 14, as the library function (0.85,
+// 0.258); 1 + (d + d^2 series) is within 0.96 (0.267).  x beyond +-800 saturates
+// to 0 or infinity, and a NaN stays one (v_max_f64 would drop it: under -800 the
+// high word is replaced instead, by that of -800; above 800 only n is bounded, d
+// overflows).  22 instructions, no table (a load would wait for the checkpoint
+// stores issued before it), against the library's 35.
 __device__ __forceinline__ double exp_f64(double x)
 {
     const uint64_t bits = __builtin_bit_cast(uint64_t, x);
@@ -464,8 +466,8 @@ __device__ __forceinline__ double exp_f64(double x)
     // ln(2) in two parts, the first of 33 bits: n times it is exact
     double d = fma(n, -6.93147180369123816490e-01, x);
     d = fma(n, -1.90821492927058770002e-10, d);
-    const double r = fma(d * d, exp_series<13>(d), d);
-    return __builtin_amdgcn_ldexp(1.0 + r, int(n));
+    const double s = fma(d, exp_series<13>(d), 1.0);
+    return __builtin_amdgcn_ldexp(fma(d, s, 1.0), int(n));
 }
 
 // e^x as a sum hi + lo good to some 2^-60, for constants formed once per block:
