@@ -127,7 +127,7 @@ int main(int argc, char** argv)
     uoc.maturity = 3.0;
     uoc.monitor_freq = 1.0 / 52;
     uoc.smooth = 0.05;
-    double mats[3] = {1.0, 2.0, 2.0}, ks[3] = {90.0, 100.0, 110.0};
+    double mats[4] = {1.0, 2.0, 2.0, 1.0}, ks[4] = {90.0, 100.0, 110.0, 95.0};
     cf_product eus{};
     eus.kind = CF_PRODUCT_EUROPEANS;
     eus.n_options = 3;
@@ -138,9 +138,9 @@ int main(int argc, char** argv)
     num.num_path = paths;
     num.precision = precision;
     num.aad_mode = mode;
-    const double w[3] = {1.0, 0.0, 0.0};
-    double means[3], agg = 0.0;
-    std::vector<double> risks(3 * (1 + 30 * 36)), per_path;
+    const double w[4] = {1.0, 0.0, 0.0, 0.0};
+    double means[4], agg = 0.0;
+    std::vector<double> risks(4 * (1 + 30 * 36)), per_path;
     auto risk = [&](const cf_num& n) {
         return cf_mc_simul_aad(&lv, &uoc, &n, w, means, &agg, risks.data(), nullptr, nullptr);
     };
@@ -186,6 +186,9 @@ int main(int argc, char** argv)
             std::vector<double> z(size_t(1) << 25);
             rc = cf_sobol_points(0, 1 << 18, 128, CF_FP64, 0, nullptr, z.data());
         }
+    } else if (scenario == "itemized_calls") {
+        eus.n_options = argc > 5 ? std::atoi(argv[5]) : 3;
+        rc = itemized(num);
     } else if (scenario == "itemized_short") {
         g_size = size_t(500) << 20;
         g_hide = true;

@@ -2,8 +2,8 @@
 stand-ins for the HIP calls that count allocations on a device of a chosen size
 and run no kernel (tests/cpp/device_memory.cpp).  cf_aad_footprint bounds what a
 call takes; a call that needs what earlier ones keep gets it; a call whose
-larger choice does not fit takes the smaller one; and tables whose upload failed
-are uploaded again."""
+larger choice does not fit takes the smaller one; tables whose upload failed are
+uploaded again; and itemized risk shares its sweeps by what they cost."""
 import json
 import os
 import shutil
@@ -68,6 +68,15 @@ def test_kept_buffers_are_given_back(device, scenario):
 def test_itemized_falls_back(device):
     r = device("itemized_short")
     assert r["rc"] == 1 + 30 * 36 and r["launches"] > 0, r
+
+
+@pytest.mark.parametrize("calls,paths,shared", [(2, 1 << 14, True), (3, 1 << 14, True), (3, 1 << 20, False),
+                                                (4, 1 << 20, True)])
+def test_few_calls_on_many_paths_are_swept_by_the_payoff(device, calls, paths, shared):
+    """A forward and its sums, then a sweep and its sums by the payoff, or the
+    four kernels of the shared sweeps."""
+    r = device("itemized_calls", FP64, CHECKPOINT, paths, calls)
+    assert r["rc"] > 0 and r["launches"] == (6 if shared else 2 + 2 * calls), r
 
 
 @pytest.mark.parametrize("failing", [1, 2])

@@ -69,3 +69,12 @@ def test_columns_match_the_oracle_tape(engine):
     for k in range(risks.shape[1]):
         _, _, ref = po.aad(om, op, n, k)
         assert np.abs(risks[:, k] - ref).max() <= 1e-10 * max(np.abs(ref).max(), 1e-300)
+
+
+@pytest.mark.parametrize("prec,paths", [(cf.FP64, 260001), (cf.FP32, 450001)])
+@pytest.mark.parametrize("calls", [3, 4])
+def test_both_sides_of_the_rule_for_few_calls(engine, calls, prec, paths):
+    """More buffers than the shared sweeps keep: three calls are swept by the
+    payoff, four share."""
+    prd = cf.Europeans(maturities=[3.0, 3.0, 1.5, 3.0][:calls], strikes=[90.0, 110.0, 100.0, 95.0][:calls])
+    _one_hot(prd, cf.Dupire(**W.dupire_args(30)), cf.NumericalParam(numPath=paths, precision=prec))
