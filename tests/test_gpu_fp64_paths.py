@@ -42,3 +42,24 @@ def test_mrg_barrier_paths_and_risks(engine, mode, weeks):
     pay, _, risks = po.aad(om, op, 500, 0, mrg=(num.seed1, num.seed2))
     np.testing.assert_allclose(res.payoffs, pay, rtol=1e-11, atol=1e-11)
     assert np.abs(res.risks - risks).max() <= 1e-10 * np.abs(risks).max()
+
+
+@pytest.mark.parametrize("mode", [cf.AAD_CHECKPOINT, cf.AAD_RECOMPUTE])
+@pytest.mark.parametrize("smooth,barrier", [(0.03125, 0.96875), (0.125, 0.875)])
+@pytest.mark.parametrize("again", [False, True])
+def test_exactly_zero_factor(engine, again, smooth, barrier, mode):
+    """Spot 1, whose logarithm and exponential are exact, on barrier + width at
+    the first date, in the narrow and the wide form of the zone; without vol on
+    every date (more than one zero factor)."""
+    assert barrier + smooth == 1.0
+    vol = 0.0 if again else 0.2
+    mk = dict(spot=1.0, spots=[0.5, 1.0, 2.0], times=[0.5, 1.0], vols=[[vol, vol]] * 3, maxDt=1.0 / 52.0)
+    pk = W.barrier_args(strike=0.75, barrier=barrier, maturity=0.25, freq=1.0 / 12.0, smooth=smooth)
+    w = [1e9, 0.4]
+    res = cf.mcParallelSimulAAD(cf.UOC(**pk), cf.Dupire(**mk), weights=w, per_path=True,
+                                num=cf.NumericalParam(numPath=500, aadMode=mode))
+    pay, _, risks = po.aad(po.Model(**mk), po.Product(**pk), 500, weights=w)
+    np.testing.assert_allclose(res.payoffs, pay, rtol=1e-11, atol=1e-11)
+    assert np.all(res.payoffs[:, 0] == 0.0)
+    assert again or np.abs(risks[0]) > 1e6         # (the oracle: the zero factor carries the delta)
+    assert np.abs(res.risks - risks).max() <= 1e-10 * np.abs(risks).max()

@@ -73,3 +73,20 @@ def test_weights_out_of_range_show(engine, model, bad, precision, mode):
     for weights in ([1.0, bad], [bad, 0.5]):
         assert np.isnan(cf.mcParallelSimulAAD(prd, mdl, weights=weights, num=num).risks[0])
     assert np.all(cf.mcParallelSimulAAD(prd, mdl, weights=[1.0, 0.5], num=num).risks == 0.0)
+
+
+@pytest.mark.parametrize("weeks,barrier", [(0, False)] + [(n, b) for n in (1, 3, 4, 5) for b in (False, True)])
+def test_short_timelines_of_several_blocks(engine, weeks, barrier):
+    """Gathered sweeps of no step, of steps in rows alone, and of one group of
+    four: as the calls of one block a wave, to 1e-11 of their scale."""
+    mdl = cf.Dupire(**W.dupire_args(30))
+    prd = cf.UOC(**W.barrier_args(strike=98.0, barrier=107.0, maturity=weeks / 52.0)) if barrier else \
+        cf.European(98.0, weeks / 52.0)
+    n, part, total = (1 << 19) + 77, 1 << 17, 0.0
+    res = cf.mcParallelSimulAAD(prd, mdl, num=cf.NumericalParam(numPath=n))
+    for lo in range(0, n, part):
+        m = min(part, n - lo)
+        total = total + m * cf.mcParallelSimulAAD(prd, mdl, num=cf.NumericalParam(numPath=m, firstPath=lo)).risks
+    assert np.abs(res.risks - total / n).max() <= 1e-11 * np.abs(total / n).max()
+    if weeks == 0:
+        assert abs(res.risks[0] - 1.0) < 1e-12 and np.all(res.risks[1:] == 0.0)
