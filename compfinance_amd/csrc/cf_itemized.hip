@@ -20,7 +20,8 @@
 // What bounds it: the sweeps' vector instructions and LDS atomics.  The lanes
 // of a wave gather their checkpoints from different blocks of 64 paths, a
 // 32-byte (FP64) or 16-byte (FP32) word and a bracket word per four steps,
-// which the caches hold up to some 2^17 paths.  30 calls over six maturities
+// which the caches hold up to some 2^17 paths (the engine leaves few calls on
+// many paths to the sweep per payoff).  30 calls over six maturities
 // on 2^16 paths, 156 steps, 30 x 36 grid, FP64: one launch per call took 3.2 ms
 // (17.5 sweeps of all paths over the 156 steps, a synchronisation each); the
 // lists are 2.6 sweeps, 0.14 ms of reverse.  (A grid per chunk, summed by the

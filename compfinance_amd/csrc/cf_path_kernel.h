@@ -1257,9 +1257,9 @@ __device__ __forceinline__ void path_body(const LaunchParams& P, const int bid, 
                     emit(bk_van_col[k], (F - kk > R(0) ? F - kk : R(0)) / numv);
                 }
                 // up-and-out barriers (mcPrd.h:256-287, one state per barrier,
-                // ordered by the lower end of their zone): a product per
-                // barrier for all lanes (bar_update), no state changes while no
-                // lane is above the zone.  A wave vote per barrier instead, to
+                // in the book's order): by fours a product per barrier for all
+                // lanes (bar_update), while some lane is above the lowest of
+                // their zones; no state changes otherwise.  A wave vote per barrier instead, to
                 // skip those with no live lane in the zone, visits half as many
                 // but costs more scalar work and branches than it saves.
                 const uint32_t bl = sm.bars >> 16;
@@ -1745,6 +1745,8 @@ __device__ __forceinline__ void path_body(const LaunchParams& P, const int bid, 
                 if (__builtin_amdgcn_ballot_w64(live) == 0) pk_cnt = 0;
             }
 
+            // (one sweep, two where the wave's last block leaves a rest; the
+            // body, to the end of the block's work, is not indented further)
             for (bool more = pk_cnt > 0; more;) {
             more = false;
             // the lane's path of the sweep: its lane in the block and its slot
@@ -2395,22 +2397,23 @@ __device__ __forceinline__ void path_body(const LaunchParams& P, const int bid, 
                         }
                         for (; i < nrev; ++i) step(i, RECOMP ? draw(i) : ck[i * kWave + lane]);
                     }
-                } else
-                for (int i = 0; i < nrev; ++i) {
-                    R g;
-                    if constexpr (RECOMP) g = draw(i);   // regenerated
-                    else g = ck[i * kWave + lane];
-                    spot = spot * rexp(drift[i] + stdv[i] * g);
-                    const R dti = R(dt[i]);
-                    const R sq = R(sqrt(dt[i]));
-                    tau[1] = tau[1] + (P.spot_measure ? R(vol) * dti : -R(vol) * dti) + sq * g;
-                    tau[2] = tau[2] + dti;
-                    tau[3] = tau[3] - dti;
-                    const int s = step_sample[i + 1];
-                    if (s >= 0) accumulate(s, spot);
+                } else {
+                    for (int i = 0; i < nrev; ++i) {
+                        R g;
+                        if constexpr (RECOMP) g = draw(i);   // regenerated
+                        else g = ck[i * kWave + lane];
+                        spot = spot * rexp(drift[i] + stdv[i] * g);
+                        const R dti = R(dt[i]);
+                        const R sq = R(sqrt(dt[i]));
+                        tau[1] = tau[1] + (P.spot_measure ? R(vol) * dti : -R(vol) * dti) + sq * g;
+                        tau[2] = tau[2] + dti;
+                        tau[3] = tau[3] - dti;
+                        const int s = step_sample[i + 1];
+                        if (s >= 0) accumulate(s, spot);
+                    }
                 }
             }
-            }
+            }   // (the sweeps of this block)
         }
     }
 

@@ -1,9 +1,9 @@
 """The barriers of a book where their shared update and the reverse's zone
 tests can go wrong, against the CPU oracle: one, four, five and sixteen
-barriers (the kernels update them by fours), given out of order (they are
-placed by the lower end of their zone), with one schedule and with several
-schedules and maturities (some samples observe a part of them), and smoothing
-factors that are exactly zero (the spot on barrier + width today).  FP64 payoffs
+barriers (the kernels update them by fours), their zones in no order, with one
+schedule and with several schedules and maturities (some samples observe a part
+of them), and smoothing factors that are exactly zero (the spot on barrier +
+width today).  FP64 payoffs
 to 1e-11 and risks to 1e-10 of their scale, the bounds of the parity tests;
 FP32 prices to 0.1 standard errors of FP64."""
 import numpy as np
